@@ -57,8 +57,7 @@ __global__ __launch_bounds__(256) void embed_q6k_kernel(const int32_t* ids, int6
 // x <- f16(v) (the residual stream is updated in place, ops.ts:41), and the sum of squares takes
 // the unrounded v (ops.ts:42); without: v = f32(x).  normalized = f16(f32(x) * inv * w) with the
 // stored (rounded) x and inv = 1 / sqrt(sum / width + eps) (ops.ts:52-55).  residual_at(c) gives
-// the residual's 8 values at columns c..c+7 (from memory, or from a projection's split-K sums),
-// so both kernels below run the same arithmetic in the same order.
+// the residual's 8 values at columns c..c+7.
 template <bool RESIDUAL, typename ResidualAt>
 __device__ inline void rmsnorm_row(half_t* xr, ResidualAt residual_at, const float* weight, half_t* out_row,
                                    int width, float eps, int lane) {
@@ -120,31 +119,6 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(half_t* x, const half_t* r
   }
 }
 
-// A projection's split-K sums as the residual: r = f16(part[0] + part[1] + ...) in chunk order
-// (part: chunks x rows x width fp32, the layout and sums of q4_reduce_kernel), then
-// rmsnorm_row as above: bit for bit the projection's output followed by rmsnorm_kernel.
-__global__ __launch_bounds__(256) void reduce_rmsnorm_kernel(const float* part, int chunks, half_t* x,
-                                                             const float* weight, half_t* out, int64_t rows,
-                                                             int width, int64_t x_stride, int64_t out_stride,
-                                                             float eps) {
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const int lane = threadIdx.x & 63;
-  const size_t plane = (size_t)rows * (size_t)width;
-  const float* pr = part + (size_t)row * width;
-  auto sums = [&](int c) {
-    f4 s0 = *reinterpret_cast<const f4*>(pr + c), s1 = *reinterpret_cast<const f4*>(pr + c + 4);
-    for (int ch = 1; ch < chunks; ++ch) {
-      s0 = s0 + *reinterpret_cast<const f4*>(pr + (size_t)ch * plane + c);
-      s1 = s1 + *reinterpret_cast<const f4*>(pr + (size_t)ch * plane + c + 4);
-    }
-    return h8{(_Float16)s0[0], (_Float16)s0[1], (_Float16)s0[2], (_Float16)s0[3],
-              (_Float16)s1[0], (_Float16)s1[1], (_Float16)s1[2], (_Float16)s1[3]};
-  };
-  rmsnorm_row<true>(x + row * x_stride, sums, weight, out + row * out_stride, width, eps, lane);
-}
-
 // ---- SwiGLU (SwiGLUKernel, ops.ts:74-102) ------------------------------------------------------
 // out[r][c] = f16(silu(g) * u), g = f32(gate_up[r][c]), u = f32(gate_up[r][width + c]),
 // silu(g) = g / (1 + exp(-g)) in f32.  One thread per 8 columns.
@@ -171,14 +145,6 @@ hipError_t launch_embed_q6k(const int32_t* ids, int64_t tokens, const uint8_t* t
   if (threads <= 0) return hipSuccess;
   hipLaunchKernelGGL(embed_q6k_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, ids, tokens,
                      table, vocab, width, out, out_stride);
-  return hipGetLastError();
-}
-
-hipError_t launch_reduce_rmsnorm(const float* part, int chunks, int rows, int width, const RowNorm& norm,
-                                 hipStream_t stream) {
-  if (rows <= 0) return hipSuccess;
-  hipLaunchKernelGGL(reduce_rmsnorm_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, part, chunks,
-                     norm.x, norm.weight, norm.out, (int64_t)rows, width, norm.x_stride, norm.out_stride, norm.eps);
   return hipGetLastError();
 }
 

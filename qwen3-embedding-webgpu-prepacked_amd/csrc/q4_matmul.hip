@@ -8,32 +8,23 @@
 // The weight is f16(scale * (q - 8)), as the reference dequantises it; the products and sums run
 // in fp32 on the matrix cores (the reference accumulates in f16).
 //
-// The CDNA4 shape:
-//   * workgroup tile 128 (M) x 128 (N), four wavefronts of 64 x 64, each 2 x 2 blocks of
-//     v_mfma_f32_32x32x16_f16 with fp32 accumulators (64 VGPRs); 128 VGPRs in all, so up to four
-//     workgroups share a CU.  Small launches use 64 x 128 tiles (wavefronts of 32 x 64);
-//   * per 32-column K block: the X tile (128 rows x 64 B) goes HBM -> LDS by LDS-DMA
-//     (buffer_load ... lds, 16 B per lane); each weight record of the tile's 128 rows is read
-//     once (scale word + 8 quant bytes per thread) and dequantised into a B tile in LDS: the
-//     nibbles become f16 by bit-OR into 1024.0 (f16(1024 + q)), an exact subtract of 1032 and one
-//     f16 multiply by the scale (the same single rounding as the reference's f16 product);
-//   * both tiles are double-buffered with one barrier per K block, laid out with a 16-byte XOR
-//     swizzle so the fragment reads (ds_read_b128) are conflict free; the next block's
-//     fragments are read into a second register set right after the barrier, and the weight
-//     records are loaded three blocks ahead (clamped past the end, so every path issues the same
-//     loads and the wait counts are exact);
-//   * tiles are numbered so that consecutive workgroups on one XCD (workgroup b runs on XCD
-//     b % 8) walk the N tiles of one M tile: its X rows stay in that XCD's L2;
-//   * the SWIGLU variant (the FFN's gate/up projection, model.ts:126-127) maps each workgroup's B
-//     rows onto a feature's gate and up rows and writes silu(gate) * up instead of the projection.
-//   * launches of at most kQ4DirectBlocks 32 x 32 output blocks (small M) run q4_direct_kernel
-//     instead: one workgroup per block, no tile staging, the same MFMA chains per output element,
-//     so its rows equal the tiled kernel's bit for bit; up to one block per CU each K chunk runs
-//     in a wavefront of its own and the chains meet in LDS.
+// Three kernels, one result: every output element is the same MFMA chain (its K blocks in turn from
+// a zero accumulator, the two halves of a K above 1024 columns added at the end), so a row does not
+// depend on the launch it is in.  v_mfma_f32_16x16x32_f16 on a K block equals two chained
+// v_mfma_f32_32x32x16_f16 on its halves bit for bit, which lets each kernel take the shape it needs.
+//   * q4_tile_kernel, large launches: 256 x 256 / 256 x 128 / 128 x 128 workgroup tiles, X by
+//     LDS-DMA, every weight record dequantised once per workgroup into an LDS tile;
+//   * q4_mid_kernel, medium launches: 64 x 128 tiles, X by LDS-DMA, the weights dequantised
+//     straight into each wavefront's MFMA fragments;
+//   * q4_direct_kernel, at most kQ4DirectBlocks 32 x 32 output blocks: one workgroup per block, no
+//     tile staging.
+// Tiles are numbered so that consecutive workgroups on one XCD (workgroup b runs on XCD b % 8)
+// walk the N tiles of one M tile: its X rows stay in that XCD's L2.  The SWIGLU variants (the FFN's
+// gate/up projection, model.ts:126-127) map B rows onto a feature's gate and up rows and write
+// silu(gate) * up instead of the projection.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <type_traits>
 
 #include "model_ops.h"
 
@@ -45,341 +36,606 @@ typedef float f16x __attribute__((ext_vector_type(16)));
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
-constexpr int kQ4TileN = 128;   // workgroup tile columns; rows 64 BM (BM = 2, or 1 for small launches)
-constexpr int kQ4Record = 20;   // bytes per (row, 32-column block)
-// Below this many 128 x 128 tiles a launch uses 64-row workgroup tiles (twice as many
-// workgroups on the 256 CUs; measured 10-11% faster for the model's output and down projections
-// at M = 500-1,419, slower above about 160 tiles).  Each output element is computed the same way
-// in both.
-constexpr int kQ4SmallLaunch = 160;
-// Fixed K split: every output element is the fp32 sum, in chunk order, of MFMA chains over
-// chunks of kQ4ChunkBlocks 32-column K blocks, each chain from a zero accumulator:
-// y = f16((c0 + c1) + c2) for K = 3072.  The split depends on K alone, so a row's result does
-// not depend on the batch whichever way a launch computes it: in registers (every chunk in one
-// workgroup, a second accumulator set) or, for launches with few tiles, one workgroup per
-// (tile, chunk) writing fp32 partials that q4_reduce_kernel sums in the same order.
-constexpr int kQ4ChunkBlocks = 32;
-// Launches with fewer than this many 64 x 128 tiles (two per CU) and more than one chunk split
-// the chunks over workgroups when the caller provides a workspace (chunks x M x N fp32).  The
-// model's output and down projections split up to M = 4,095: 16 x 150 tokens forward 2.5% faster
-// than with the limit at 256 tiles, the other batch sizes unchanged.
-constexpr int kQ4SplitTiles = 512;
-
+constexpr int kQ4Record = 20;  // bytes per (row, 32-column block)
+// Every output element is the fp32 sum of at most two MFMA chains, each from a zero accumulator:
+// one over all of K up to 1024 columns, else one per half, y = f16(c0 + c1).  The split depends on
+// K alone, so a row's result does not depend on the batch, and the halves of a launch with few
+// tiles run side by side.
+// K blocks per chain (a multiple of 8 where there are two).
+__host__ __device__ constexpr int q4_chunk_blocks(int K) {
+  return K <= 1024 ? K / 32 : ((K / 32 + 1) / 2 + 7) / 8 * 8;
+}
 __device__ inline __amdgpu_buffer_rsrc_t q4_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
 }
 
-// Two f16 weights from the low (HIGH = false) or high nibbles of bytes 0 and 1 of `pair`
-// (laid out as byte 0 in bits 0..7 and byte 1 in bits 16..23): f16(scale * (q - 8)).
+// Four weights of four quant bytes: f16(scale * (q - 8)) of their low (HIGH = false) or high
+// nibbles.  A byte under 0x64 is the f16 1024 + byte; q - 8 follows exactly (for high nibbles
+// 1024 + 16 q -> 64 + q - 72 in one fma), and one f16 multiply rounds as the reference's does.
 template <bool HIGH>
-__device__ inline h2 dequant2(uint32_t pair, h2 scale) {
-  const uint32_t q = (HIGH ? pair >> 4 : pair) & 0x000F000Fu;
-  const h2 biased = __builtin_bit_cast(h2, q | 0x64006400u);  // 1024 + q, exact
-  const h2 centred = biased - h2{(_Float16)1032.0f, (_Float16)1032.0f};  // q - 8, exact
-  return centred * scale;  // one rounding, as the reference's f16 multiply
+__device__ inline u2 dequant4(uint32_t q, h2 scale) {
+  const uint32_t v = q & (HIGH ? 0xF0F0F0F0u : 0x0F0F0F0Fu);
+  const h2 p0 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, v, 0x04010400u));
+  const h2 p1 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, v, 0x04030402u));
+  h2 c0, c1;
+  if constexpr (HIGH) {
+    const h2 m = {(_Float16)0.0625f, (_Float16)0.0625f}, k = {(_Float16)-72.0f, (_Float16)-72.0f};
+    c0 = __builtin_elementwise_fma(p0, m, k);
+    c1 = __builtin_elementwise_fma(p1, m, k);
+  } else {
+    const h2 k = {(_Float16)-1032.0f, (_Float16)-1032.0f};
+    c0 = p0 + k;
+    c1 = p1 + k;
+  }
+  return u2{__builtin_bit_cast(uint32_t, c0 * scale), __builtin_bit_cast(uint32_t, c1 * scale)};
 }
 
 // The 8 weights of a B fragment: quant bytes b0..b7 (two dwords) -> low or high nibbles.
 template <bool HIGH>
 __device__ inline h8 dequant8(u2 q, h2 scale) {
-  // byte pairs (b0,b1), (b2,b3) of each dword into the two 16-bit halves
-  const uint32_t p0 = __builtin_amdgcn_perm(0u, q[0], 0x0C010C00u);
-  const uint32_t p1 = __builtin_amdgcn_perm(0u, q[0], 0x0C030C02u);
-  const uint32_t p2 = __builtin_amdgcn_perm(0u, q[1], 0x0C010C00u);
-  const uint32_t p3 = __builtin_amdgcn_perm(0u, q[1], 0x0C030C02u);
-  const h2 a = dequant2<HIGH>(p0, scale), b = dequant2<HIGH>(p1, scale);
-  const h2 c = dequant2<HIGH>(p2, scale), d = dequant2<HIGH>(p3, scale);
-  return h8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+  const u2 a = dequant4<HIGH>(q[0], scale), b = dequant4<HIGH>(q[1], scale);
+  return __builtin_bit_cast(h8, u4{a[0], a[1], b[0], b[1]});
 }
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 
-// LDS tiles: 128 rows x 32 columns of fp16 (64 B per row) for X (A) and for the dequantised
-// weights (B, row = output column n).  The four 16-byte chunks of row r sit at physical chunk
+// LDS tiles: rows of 32 columns of fp16 (64 B per row) for X (A) and for the dequantised weights (B,
+// row = output column n).  The four 16-byte chunks of row r sit at physical chunk
 // c ^ ((r >> 2) & 3): 16 consecutive rows reading one logical chunk then cover all 64 banks, so
 // the fragment reads (lanes 0-15 / 16-31 / ... take 16 consecutive rows) are conflict free.
 __device__ inline uint32_t q4_lds_off(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4); }
 
-// The memory and matrix builtins behind plain (non-template) device functions: the kernel uses
-// them in BM-dependent loops, and hipcc's host pass drops a kernel template's host stub when
-// such a builtin sits in a dependent context.
-__device__ inline void q4_dma16(__amdgpu_buffer_rsrc_t rs, char* dst, uint32_t off) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_t*)dst, 16, off, 0, 0, 0);
-}
+// The memory and matrix builtins behind plain (non-template) device functions: hipcc's host pass
+// drops a kernel template's host stub when such a builtin sits in a dependent context.
 __device__ inline void q4_store_b16(_Float16 v, __amdgpu_buffer_rsrc_t rs, uint32_t off) {
   __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), rs, off, 0, 0);
 }
 __device__ inline f16x q4_mfma(h8 a, h8 b, f16x c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+typedef float f4 __attribute__((ext_vector_type(4)));
+__device__ inline f4 q4_mfma16(h8 a, h8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+__device__ inline void q4_dma16(__amdgpu_buffer_rsrc_t rs, char* dst, uint32_t off, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_t*)dst, 16, off, soff, 0, 0);
+}
+__device__ inline void q4_store16(u4 v, __amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  __builtin_amdgcn_raw_buffer_store_b128(v, rs, off, 0, 0);
+}
+__device__ inline uint32_t q4_pack(_Float16 a, _Float16 b) {
+  return (uint32_t)__builtin_bit_cast(unsigned short, a) | (uint32_t)__builtin_bit_cast(unsigned short, b) << 16;
+}
 
-// SWIGLU: the weight is [gate (N/2 rows) | up (N/2 rows)] and the output is silu(gate) * up, N/2
-// columns: the workgroup of tile column tn takes gate rows 64 tn .. +63 and the matching up rows
-// (B rows 0-31 gate, 32-63 up, 64-95 gate, 96-127 up), so every wave holds the gate and up
-// accumulators of the same 32 features in the same lanes and applies swiglu_value to them.
-// CH = 0: K within one chunk (one chain); 1: every chunk in this workgroup (a second set of
-// accumulators holds the finished chunks' sum); 2: one chunk per workgroup (work unit t =
-// tile * chunks + chunk), its chain stored as fp32 to part[chunk][m][n].
-template <bool SWIGLU, int BM, int CH>
-__global__ __launch_bounds__(256, 2) void q4_matmul_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, int K,
-                                                           const uint8_t* __restrict__ w, uint32_t w_bytes, int N,
-                                                           _Float16* __restrict__ y, int64_t ldy, int tiles_n,
-                                                           int tiles_total, int per_xcd, float* __restrict__ part,
-                                                           int chunks) {
-  // Double-buffered A and B tiles: four distinct objects, each buffer choice fixed at compile
-  // time, so the compiler sees that LDS-DMA writes in flight never alias the tile being read.
-  constexpr int kTileM = 64 * BM;
-  __shared__ __attribute__((aligned(1024))) char sA0[kTileM * 64];
-  __shared__ __attribute__((aligned(1024))) char sA1[kTileM * 64];
-  __shared__ __attribute__((aligned(1024))) char sB0[kQ4TileN * 64];
-  __shared__ __attribute__((aligned(1024))) char sB1[kQ4TileN * 64];
+// Waits for all but the newest V vector-memory operations and for all LDS operations of this
+// wavefront, then meets the workgroup.  One block of its own: the compiler's barrier would wait
+// for every LDS-DMA load in flight.
+template <int V>
+__device__ inline void q4_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(V) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
 
-  // Tile of this workgroup: XCD b % 8 owns tiles [xcd * per_xcd, (xcd + 1) * per_xcd).
-  const int b = blockIdx.x;
-  const int u = (b & 7) * per_xcd + (b >> 3);
+#define Q4_INLINE __attribute__((always_inline))
+
+// ---- large launches.
+// Workgroup tile 32 MF x 64 NWN, 2 x NWN wavefronts of 16 MF x 64 per group; G = 2 (K above 1024): two
+// such groups, one per half of K, whose chains meet through LDS at the end.
+//
+// What bounds it: LDS bandwidth (128 B per clock and CU, measured) and power.  A 128 x 64 wavefront
+// (MF = 8) reads 12 KiB of fragments per K block for 512 clocks of MFMA, so two per SIMD keep LDS
+// busy about 1,020 of 1,024 clocks at 256 x 256 (1,150 at 256 x 128); the 64 x 64 wavefronts this
+// replaces needed 1.4x the MFMA time in LDS.  16x16x32 MFMAs sustain 1.9 PFLOP/s under this card's
+// power limit, 32x32x16 ones 1.65 (pure MFMA loops).  Hence the large wavefront tiles, the 16 x 16
+// instruction, and the vector-memory instructions spread one per several MFMAs: issued in a burst
+// after the barrier they filled the texture unit's queue and stalled the MFMAs behind them (70.5 ->
+// 68.1 us).  Not kept: weights dequantised into registers at this size (VALU power: 73 us), four
+// wavefronts of 128 x 128 (one per SIMD cannot issue the dequantisation beside its MFMAs: 65 us).
+// Measured (us, before -> after): 8000 x 1024 -> 4096 80.4 -> 65.5; 20000 x 1024 -> 6144 with SwiGLU
+// 292 -> 254; 8000 x 2048 -> 1024 44.8 -> 38.8; 8000 x 3072 -> 1024 64.9 -> 53.2.
+//
+// Step kb (X tile and weight tile kb in LDS; the first half's fragments in registers): half 1 reads
+// the other row fragments, dequantises weight tile kb + 1 into the free B buffer and runs the first
+// half's MFMAs; the barrier publishes that tile and X tile kb + 1 (loaded two steps ago); half 2
+// reads the next step's fragments under the other half's MFMAs.  X tile kb + 3 goes into the buffer
+// that tile kb - 1 left at the previous barrier.
+template <bool SWIGLU, int MF, int NWN, int G>
+__global__ __launch_bounds__(128 * NWN * G, 2) void q4_tile_kernel(
+    const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N, _Float16* y, int64_t ldy,
+    int chunk_blocks, int tiles_n, int tiles_total, int per_xcd) {
+  constexpr int kWaves = 2 * NWN;                            // per group
+  constexpr int kTileM = 32 * MF, kTileN = 64 * NWN;
+  constexpr int kBytesA = kTileM * 64, kBytesB = kTileN * 64;  // one K block's tiles
+  constexpr int AJ = MF / NWN;                               // X loads per wavefront and K block
+  constexpr int A1 = AJ / 2, A2 = AJ - A1;                   // ... in the first / second half step
+  constexpr int H = MF / 2;                                  // row fragments per half step
+  __shared__ __attribute__((aligned(1024))) char sA0[G * kBytesA];
+  __shared__ __attribute__((aligned(1024))) char sA1[G * kBytesA];
+  __shared__ __attribute__((aligned(1024))) char sA2[G * kBytesA];
+  __shared__ __attribute__((aligned(1024))) char sA3[G * kBytesA];
+  __shared__ __attribute__((aligned(1024))) char sB0[G * kBytesB];
+  __shared__ __attribute__((aligned(1024))) char sB1[G * kBytesB];
+
+  const int u = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (u >= tiles_total) return;
-  const int t = CH == 2 ? u / chunks : u;
-  const int m0 = (t / tiles_n) * kTileM, n0 = (t % tiles_n) * kQ4TileN;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, hl = lane >> 5;
-  const int wr = 32 * BM * (wave & 1), wc = 64 * (wave >> 1);  // this wave's 32 BM x 64 inside the tile
+  const int m0 = (u / tiles_n) * kTileM, n0 = (u % tiles_n) * kTileN;
+  const int gwave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = G == 1 ? 0 : gwave / kWaves, wave = G == 1 ? gwave : gwave % kWaves;
+  const int lane = threadIdx.x & 63, tid = 64 * wave + lane;
+  const int l16 = lane & 15, kq = lane >> 4;
+  const int wr = 16 * MF * (wave & 1), wc = 64 * (wave >> 1);
   const int kblocks = K >> 5;
-  // K blocks of this workgroup: all of them, or (CH == 2) one chunk.
-  const int kb_first = CH == 2 ? (u % chunks) * kQ4ChunkBlocks : 0;
-  const int kb_end = CH == 2 ? min(kb_first + kQ4ChunkBlocks, kblocks) : kblocks;
+  const int kb0 = G == 1 ? 0 : grp * chunk_blocks, kn = G == 1 ? kblocks : chunk_blocks;
+  const int k_here = min(kn, kblocks - kb0);  // blocks from k_here on are read as zeros
 
-  const auto xrs = q4_rsrc(x, (uint32_t)M * (uint32_t)ldx * 2u);  // rows >= M read as zeros
-  const auto wrs = q4_rsrc(w, w_bytes);
-  const auto yrs = q4_rsrc(y, (uint32_t)M * (uint32_t)ldy * 2u);
-
-  // ---- A: LDS-DMA, 16 B per lane per instruction, 1 KiB (16 rows) per wave instruction.
-  // Instruction j of wave `wave` fills rows 16 (BM wave + j) .. +15; lane's LDS slot p = lane * 16
-  // within that KiB is row 16 (BM wave + j) + lane / 4, physical chunk lane & 3, which holds
-  // logical chunk (lane & 3) ^ ((row >> 2) & 3): columns 8 * that .. +7 of the K block.
-  uint32_t a_src[BM];
+  const uint32_t x_bytes = (uint32_t)M * (uint32_t)ldx * 2u;
+  uint32_t a_src[AJ];
 #pragma unroll
-  for (int j = 0; j < BM; ++j) {
-    const int row = 16 * (BM * wave + j) + (lane >> 2);
-    const int chunk = (lane & 3) ^ ((row >> 2) & 3);
-    a_src[j] = (uint32_t)(m0 + row) * (uint32_t)ldx * 2u + 16u * chunk;
+  for (int j = 0; j < AJ; ++j) {
+    const int row = 16 * (AJ * wave + j) + (lane >> 2);
+    a_src[j] = (uint32_t)(m0 + row) * (uint32_t)ldx * 2u + 16u * ((lane & 3) ^ ((row >> 2) & 3));
   }
-  auto load_a = [&](char* dst, int kb) {
-    kb = kb < kb_end ? kb : kb_end - 1;  // past the end: re-read the last block (never used)
+  const uint32_t a_dst = grp * kBytesA + 1024 * AJ * wave;
+  // X loads j0 .. j0 + n - 1 of K block kb: 16 rows (1 KiB) per wavefront instruction; lane's LDS slot
+  // is row lane / 4, physical chunk lane & 3.
+  auto load_a = [&](char* dst, int kb, int j0, int n) Q4_INLINE {
+    const auto rs = q4_rsrc(x, kb < k_here ? x_bytes : 0u);
 #pragma unroll
-    for (int j = 0; j < BM; ++j) q4_dma16(xrs, dst + 1024 * (BM * wave + j), a_src[j] + (uint32_t)kb * 64u);
+    for (int j = j0; j < j0 + n; ++j) q4_dma16(rs, dst + a_dst + 1024 * j, a_src[j], (uint32_t)(kb0 + kb) * 64u);
   };
-
-  // ---- B: thread (row n = tid / 2, half h = tid & 1) owns quant bytes 8h .. 8h+7 of the record
-  // of (n0 + n, kb): their low nibbles are columns 8h .. +7 (chunk h), their high nibbles columns
-  // 16 + 8h .. +7 (chunk 2 + h).  Records of rows past the tensor read as zeros.
+  // Thread (row n = tid / 2, half h = tid & 1) dequantises quant bytes 8h .. 8h + 7 of the record of
+  // (n0 + n, kb): columns 8h .. + 7 (chunk h) and 16 + 8h .. + 7 (chunk 2 + h).  SWIGLU: B rows 0-31
+  // of each 64 are gate rows of 32 features, rows 32-63 their up rows.
   const int brow = tid >> 1, bhalf = tid & 1;
   const int wtile = SWIGLU ? ((brow >> 5) & 1 ? N >> 6 : 0) + (n0 >> 6) + (brow >> 6) : (n0 + brow) >> 5;
   const uint32_t w_rec = ((uint32_t)wtile * (uint32_t)kblocks * 32u + (uint32_t)(brow & 31)) * kQ4Record;
-  const uint32_t w_step = 32u * kQ4Record;
-  const uint32_t b_lo = q4_lds_off(brow, bhalf), b_hi = q4_lds_off(brow, 2 + bhalf);
+  const uint32_t w_q = w_rec + 4u + 8u * bhalf;
+  const uint32_t b_lo = grp * kBytesB + q4_lds_off(brow, bhalf), b_hi = grp * kBytesB + q4_lds_off(brow, 2 + bhalf);
   struct WRegs {
     uint32_t scale;
     u2 q;
   };
-  auto load_w = [&](WRegs& r, int kb) {
-    kb = kb < kb_end ? kb : kb_end - 1;
-    const uint32_t off = w_rec + (uint32_t)kb * w_step;
-    r.scale = __builtin_amdgcn_raw_buffer_load_b32(wrs, off, 0, 0);
-    r.q = __builtin_amdgcn_raw_buffer_load_b64(wrs, off + 4u + 8u * bhalf, 0, 0);
+  auto w_rs = [&](int kb) Q4_INLINE { return q4_rsrc(w, kb < k_here ? w_bytes : 0u); };
+  auto load_ws = [&](WRegs& r, int kb) Q4_INLINE {
+    r.scale = __builtin_amdgcn_raw_buffer_load_b32(w_rs(kb), w_rec, (uint32_t)(kb0 + kb) * (32u * kQ4Record), 0);
   };
-  auto store_b = [&](char* dst, const WRegs& r) {
+  auto load_wq = [&](WRegs& r, int kb) Q4_INLINE {
+    r.q = __builtin_amdgcn_raw_buffer_load_b64(w_rs(kb), w_q, (uint32_t)(kb0 + kb) * (32u * kQ4Record), 0);
+  };
+  auto store_b = [&](char* dst, const WRegs& r) Q4_INLINE {
     const _Float16 s = __builtin_bit_cast(h2, r.scale)[0];
     const h2 scale = {s, s};
     *reinterpret_cast<h8*>(dst + b_lo) = dequant8<false>(r.q, scale);
     *reinterpret_cast<h8*>(dst + b_hi) = dequant8<true>(r.q, scale);
   };
+  f4 acc[MF][4];
+#pragma unroll
+  for (int mb = 0; mb < MF; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) acc[mb][nb] = f4{};
+  const uint32_t a_rd = grp * kBytesA + q4_lds_off(wr + l16, kq), b_rd = grp * kBytesB + q4_lds_off(wc + l16, kq);
 
-  // ---- fragments: lane reads row (wr or wc) + 32 blk + l32, logical chunk 2 s + hl.
-  f16x acc[BM][2];
-#pragma unroll
-  for (int mb = 0; mb < BM; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = f16x{};
-  // Fragments of one K block: two sets, alternating by block parity, so the next block's reads
-  // are in flight while this block's MFMAs run.
-  struct Frags {
-    h8 a[BM][2], b[2][2];
-  };
-  Frags frag[2];
-  auto read_frags = [&](const char* a_t, const char* b_t, Frags& f) {
-#pragma unroll
-    for (int blk = 0; blk < 2; ++blk)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        if (blk < BM) f.a[blk][s] = *reinterpret_cast<const h8*>(a_t + q4_lds_off(wr + 32 * blk + l32, 2 * s + hl));
-        f.b[blk][s] = *reinterpret_cast<const h8*>(b_t + q4_lds_off(wc + 32 * blk + l32, 2 * s + hl));
-      }
-  };
-  // The MFMA order of an output block -- s, then its K blocks in turn -- is the same for BM = 1
-  // and 2, so rows do not depend on the tile height a launch picks.
-  // fresh: the first K block of a chain (CH == 1 chunks after the first): step 0 accumulates onto
-  // the inline constant 0, which is what the zeroed accumulators would add.
-  auto mma = [&](const Frags& f, auto fresh) {
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int mb = 0; mb < BM; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-          acc[mb][nb] = q4_mfma(f.a[mb][s], f.b[nb][s], decltype(fresh)::value && s == 0 ? f16x{} : acc[mb][nb]);
-  };
-
-  // ---- pipeline.  Step kb (P = kb & 1, compile time): issue A(kb+1) into sA<1-P> and W(kb+3)
-  // into register stage (kb+3) % 4; dequantise W(kb+1) (loaded two steps ago) into sB<1-P>; run
-  // block kb's MFMAs on the fragments read at the end of the previous step; wait for A(kb+1)
-  // (only W(kb+3), issued after it, may still be in flight: vmcnt(2)); barrier; read block
-  // kb+1's fragments.  sB<1-P> is free at its write: its last reads (block kb-1's fragments)
-  // were consumed by MFMAs before the previous barrier.  Every load is issued (clamped past the
-  // end), so the counts are the same on every path.
   WRegs wreg[4];
-  load_a(sA0, kb_first);
-  load_w(wreg[0], kb_first);
-  load_w(wreg[1], kb_first + 1);
-  load_w(wreg[2], kb_first + 2);
-  __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8) | 4);  // vmcnt(4): A(0), W(0) landed
+  h8 a_lo[H], a_hi[H], b0[4], b1[4];
+  auto read_a = [&](h8 (&f)[H], const char* p) Q4_INLINE {
+#pragma unroll
+    for (int i = 0; i < H; ++i) f[i] = *reinterpret_cast<const h8*>(p + 1024 * i);
+  };
+  auto read_b = [&](h8 (&f)[4], const char* p) Q4_INLINE {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = *reinterpret_cast<const h8*>(p + 1024 * i);
+  };
+  auto mma = [&](const h8 (&b)[4], const h8 (&a)[H], int m8) Q4_INLINE {
+#pragma unroll
+    for (int mb = 0; mb < H; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) acc[m8 + mb][nb] = q4_mfma16(b[nb], a[mb], acc[m8 + mb][nb]);
+  };
+  load_ws(wreg[0], 0);
+  load_wq(wreg[0], 0);
+  load_a(sA0, 0, 0, AJ);
+  __builtin_amdgcn_sched_barrier(0);
+  load_ws(wreg[1], 1);
+  load_a(sA1, 1, 0, AJ);
+  __builtin_amdgcn_sched_barrier(0);
+  load_wq(wreg[1], 1);
+  load_ws(wreg[2], 2);
+  load_a(sA2, 2, 0, AJ);
+  __builtin_amdgcn_sched_barrier(0);
+  load_wq(wreg[2], 2);
   store_b(sB0, wreg[0]);
-  __syncthreads();
-  read_frags(sA0, sB0, frag[0]);
-  auto step = [&](auto pconst, auto wcur, auto wnext, int kb, auto fresh) {
-    constexpr int P = decltype(pconst)::value;
-    constexpr int WN = decltype(wnext)::value;   // stage of W(kb+1)
-    constexpr int WA = decltype(wcur)::value;    // stage receiving W(kb+3)
-    char* const a_nxt = P == 0 ? sA1 : sA0;
-    char* const b_nxt = P == 0 ? sB1 : sB0;
-    load_a(a_nxt, kb + 1);
-    load_w(wreg[WA], kb + 3);
-    store_b(b_nxt, wreg[WN]);
-    if (kb < kb_end) mma(frag[P], fresh);
-    __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8) | 2);  // vmcnt(2)
-    __syncthreads();
-    read_frags(a_nxt, b_nxt, frag[1 - P]);
-  };
-  using I0 = std::integral_constant<int, 0>;
-  using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  using I3 = std::integral_constant<int, 3>;
-  // Chunks of kQ4ChunkBlocks (a multiple of the 4-step group, so the steps' compile-time
-  // buffer and register-stage choices follow from kb as before); CH == 1 folds each finished
-  // chunk into tot and starts the next chain from zero.
-  using Fresh = std::integral_constant<bool, true>;
-  using Cont = std::integral_constant<bool, false>;
-  auto four_steps = [&](int kb, auto fresh) {
-    step(I0{}, I3{}, I1{}, kb, fresh);
-    step(I1{}, I0{}, I2{}, kb + 1, Cont{});
-    step(I0{}, I1{}, I3{}, kb + 2, Cont{});
-    step(I1{}, I2{}, I0{}, kb + 3, Cont{});
-  };
-  f16x tot[CH == 1 ? BM : 1][2];
-  if constexpr (CH == 1) {
-    // Chunk 0 into acc, copied to tot; every later chunk a fresh chain in acc, added to tot.
-    for (int kb = 0; kb < kQ4ChunkBlocks; kb += 4) four_steps(kb, Cont{});
+  q4_barrier<4 + 2 * AJ>();  // X tile 0: newer are W(1), X(1), W(2), X(2)
+  read_b(b0, sB0 + b_rd);
+  read_a(a_lo, sA0 + a_rd);
+  auto step = [&](const char* a_cur, const char* a_nxt, char* a_new, char* b_nxt, h8 (&b_cur)[4], h8 (&b_new)[4],
+                  const WRegs& w_use, WRegs& w_new, int kb) Q4_INLINE {
+    read_a(a_hi, a_cur + a_rd + 1024 * H);
+    load_ws(w_new, kb + 3);
+    load_a(a_new, kb + 3, 0, A1);
+    store_b(b_nxt, w_use);
+    mma(b_cur, a_lo, 0);
+    if constexpr (MF == 8) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
-    for (int mb = 0; mb < BM; ++mb)
+      for (int i = 0; i < 3; ++i) {
+        if (i <= A1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) tot[mb][nb] = acc[mb][nb];
-    for (int c0 = kQ4ChunkBlocks; c0 < kblocks; c0 += kQ4ChunkBlocks) {
-      const int c1 = min(c0 + kQ4ChunkBlocks, kblocks);
-      four_steps(c0, Fresh{});
-      for (int kb = c0 + 4; kb < c1; kb += 4) four_steps(kb, Cont{});
-#pragma unroll
-      for (int mb = 0; mb < BM; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) tot[mb][nb] = tot[mb][nb] + acc[mb][nb];
+        for (int j = 0; j < 4; ++j) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        }
+      }
+      __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
     }
-  } else {
-    for (int kb = kb_first; kb < kb_end; kb += 4) four_steps(kb, Cont{});
+    // X tile kb + 1: newer are at least step kb - 1's AJ + 2 loads and this half's 1 + A1.
+    q4_barrier<3 + AJ + A1>();
+    read_b(b_new, b_nxt + b_rd);
+    read_a(a_lo, a_nxt + a_rd);
+    load_a(a_new, kb + 3, A1, A2);
+    load_wq(w_new, kb + 3);
+    mma(b_cur, a_hi, H);
+    if constexpr (MF == 8) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        if (i <= A2) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (4 * i + j < 8) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (int kb = 0; kb < kn; kb += 4) {  // blocks past the end add zero products
+    step(sA0, sA1, sA3, sB1, b0, b1, wreg[1], wreg[3], kb);
+    step(sA1, sA2, sA0, sB0, b1, b0, wreg[2], wreg[0], kb + 1);
+    step(sA2, sA3, sA1, sB1, b0, b1, wreg[3], wreg[1], kb + 2);
+    step(sA3, sA0, sA2, sB0, b1, b0, wreg[0], wreg[2], kb + 3);
   }
-  __builtin_amdgcn_s_waitcnt(0);  // the clamped loads past the end land before the LDS is released
-  if constexpr (CH == 1) {
+  q4_barrier<0>();
+
+  // G = 2: the groups' chains meet.  Group g finishes the rows of half g of every wavefront's tile.
+  if constexpr (G == 2) {
+    char* const ex = (wave == 0 ? sA0 : wave == 1 ? sA1 : wave == 2 ? sA2 : sA3) + 16 * lane;
+    auto send = [&](int m8, char* p) Q4_INLINE {
 #pragma unroll
-    for (int mb = 0; mb < BM; ++mb)
+      for (int mb = 0; mb < H; ++mb)
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = tot[mb][nb];
+        for (int nb = 0; nb < 4; ++nb) *reinterpret_cast<f4*>(p + 1024 * (4 * mb + nb)) = acc[m8 + mb][nb];
+    };
+    if (grp == 0)
+      send(H, ex);
+    else
+      send(0, ex + 4096 * H);
+    __syncthreads();
+    auto take = [&](int m8, const char* p) Q4_INLINE {
+#pragma unroll
+      for (int mb = 0; mb < H; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) acc[mb][nb] = acc[m8 + mb][nb] + *reinterpret_cast<const f4*>(p + 1024 * (4 * mb + nb));
+    };
+    if (grp == 0)
+      take(0, ex + 4096 * H);
+    else
+      take(H, ex);
+    __syncthreads();
   }
 
-  // D (32 x 32 per block): lane holds column l32 and rows 8 (r / 4) + 4 hl + r % 4, r = 0..15.
-  // Columns >= N are skipped here; rows >= M fall outside the Y resource and are dropped.
-  const int wm = m0 + wr, wn = n0 + wc;
-  if constexpr (CH == 2) {
-    // This chunk's chains, fp32, to part[chunk][m][n] (rows >= M and columns >= N skipped).
-    float* const pc = part + (size_t)(u % chunks) * (size_t)M * (size_t)N;
+  // Output through LDS, kRows rows of a wavefront at a time: 16 stores of 16 bytes per lane in whole
+  // 128-byte lines instead of 128 stores of two bytes.  Lane (l16, kq) holds row 16 mb + l16, columns
+  // 16 nb + 4 kq .. +3.
+  constexpr int kMine = MF / G;                       // row fragments this wavefront finishes
+  constexpr int kRows = kMine >= 4 ? 64 : 16 * kMine;  // rows per pass
+  constexpr int kPer = G * kBytesA / (128 * kRows);    // wavefronts per X buffer
+  const int slot = gwave / kPer;
+  char* const stage = (slot == 0 ? sA0 : slot == 1 ? sA1 : slot == 2 ? sA2 : sA3) + 128 * kRows * (gwave % kPer);
+  const auto yrs = q4_rsrc(y, (uint32_t)M * (uint32_t)ldy * 2u);
+  const int row0 = m0 + wr + 16 * kMine * grp;
+  const int n_out = SWIGLU ? N >> 1 : N;
+  const int col0 = SWIGLU ? (n0 + wc) >> 1 : n0 + wc;
+  constexpr int kChunks = SWIGLU ? 4 : 8;  // 16-byte pieces of a row
+  auto at = [&](int row, int c) Q4_INLINE {
+    return stage + row * (16 * kChunks) + ((SWIGLU ? c ^ ((row >> 2) & 3) : c ^ ((row >> 1) & 7)) << 4);
+  };
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
-      const int n = wn + 32 * nb + l32;
-      if (n < N) {
+  for (int p = 0; p < 16 * kMine / kRows; ++p) {
 #pragma unroll
-        for (int mb = 0; mb < BM; ++mb)
+    for (int mb = 0; mb < kRows / 16; ++mb) {
+      const f4(&v)[4] = acc[p * (kRows / 16) + mb];
+      const int row = 16 * mb + l16;
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int m = wm + 32 * mb + 8 * (r >> 2) + 4 * hl + (r & 3);
-            if (m < M) pc[(size_t)m * N + n] = acc[mb][nb][r];
-          }
+      for (int nb = 0; nb < (SWIGLU ? 2 : 4); ++nb) {
+        u2 d;
+        if constexpr (SWIGLU) {  // columns 0-31: gate, 32-63: up, of the same 32 features
+          const f4 &g = v[nb], &t = v[nb + 2];
+          d = u2{q4_pack(swiglu_value((_Float16)g[0], (_Float16)t[0]), swiglu_value((_Float16)g[1], (_Float16)t[1])),
+                 q4_pack(swiglu_value((_Float16)g[2], (_Float16)t[2]), swiglu_value((_Float16)g[3], (_Float16)t[3]))};
+        } else {
+          const f4& f = v[nb];
+          d = u2{q4_pack((_Float16)f[0], (_Float16)f[1]), q4_pack((_Float16)f[2], (_Float16)f[3])};
+        }
+        *reinterpret_cast<u2*>(at(row, 2 * nb + (kq >> 1)) + 8 * (kq & 1)) = d;
       }
     }
-    return;
-  }
-  if constexpr (SWIGLU) {
-    // Block nb = 0 holds gate, nb = 1 up, of output features (n0 + wc) / 2 + l32.
-    const uint32_t n = (uint32_t)((wn >> 1) + l32);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    constexpr int kRowsPer = 64 / kChunks;  // rows per store instruction
 #pragma unroll
-    for (int mb = 0; mb < BM; ++mb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = wm + 32 * mb + 8 * (r >> 2) + 4 * hl + (r & 3);
-        const uint32_t off = m < M ? ((uint32_t)m * (uint32_t)ldy + n) * 2u : 0x80000000u;
-        q4_store_b16(swiglu_value((_Float16)acc[mb][0][r], (_Float16)acc[mb][1][r]), yrs, off);
+    for (int i = 0; i < kRows / kRowsPer; ++i) {
+      const int row = kRowsPer * i + lane / kChunks, c = lane % kChunks;
+      const u4 v = *reinterpret_cast<const u4*>(at(row, c));
+      const int m = row0 + kRows * p + row, n = col0 + 8 * c;
+      const uint32_t off = ((uint32_t)m * (uint32_t)ldy + (uint32_t)n) * 2u;
+      q4_store16(v, yrs, m < M && n + 8 <= n_out ? off : 0x80000000u);
+    }
+    // A last piece of fewer than 8 columns goes element by element.
+    const int part = (n_out - col0) >> 3;
+    if ((n_out & 7) && n_out > col0 && part < kChunks) {
+#pragma unroll 1
+      for (int i = 0; i < kRows / 8; ++i) {
+        const int row = 8 * i + (lane >> 3), m = row0 + kRows * p + row, n = col0 + 8 * part + (lane & 7);
+        const _Float16 v = *reinterpret_cast<const _Float16*>(at(row, part) + 2 * (lane & 7));
+        q4_store_b16(v, yrs, m < M && n < n_out ? ((uint32_t)m * (uint32_t)ldy + (uint32_t)n) * 2u : 0x80000000u);
       }
-    return;
-  }
-#pragma unroll
-  for (int nb = 0; nb < 2; ++nb) {
-    const int n = wn + 32 * nb + l32;
-    if (n < N) {
-#pragma unroll
-      for (int mb = 0; mb < BM; ++mb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = wm + 32 * mb + 8 * (r >> 2) + 4 * hl + (r & 3);
-          const uint32_t off = m < M ? ((uint32_t)m * (uint32_t)ldy + (uint32_t)n) * 2u : 0x80000000u;
-          q4_store_b16((_Float16)acc[mb][nb][r], yrs, off);
-        }
     }
   }
 }
 
+template <bool SWIGLU, int MF, int NWN, int G>
+void launch_q4_tile(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
+                    _Float16* y, int64_t ldy, hipStream_t stream) {
+  const int tiles_m = (M + 32 * MF - 1) / (32 * MF), tiles_n = (N + 64 * NWN - 1) / (64 * NWN);
+  const int tiles = tiles_m * tiles_n, per_xcd = (tiles + 7) / 8;
+  hipLaunchKernelGGL((q4_tile_kernel<SWIGLU, MF, NWN, G>), dim3((unsigned)(8 * per_xcd)), dim3(128 * NWN * G), 0, stream,
+                     x, ldx, M, K, w, w_bytes, N, y, ldy, q4_chunk_blocks(K), tiles_n, tiles, per_xcd);
+}
+
+// ---- medium launches.
+// 64 x 128 workgroup tiles, four wavefronts of 64 x 32 per group, each dequantising its own 32
+// columns straight into MFMA fragments; G = 2 (K above 1024): two groups, one per half of K.
+// What bounds it: with about one workgroup per CU, the latency of a K block.  An LDS weight tile
+// puts dequantise -> LDS write -> barrier -> LDS read in every K block's chain (0.37 us per pair of
+// halves); here only X goes through LDS, its barrier comes once per two blocks with loads six
+// blocks ahead, and weight records are loaded four blocks ahead.  A wavefront's block is about 75
+// instructions for 8 MFMAs, so VALU and MFMA issue are level.  Measured (us, before -> after):
+// 1419 x 2048 -> 1024 22.2 -> 13.2, 1500 x 3072 -> 1024 31.6 -> 17.8, 500 x 1024 -> 4096 12.8 -> 9.4,
+// 300 x 1024 -> 6144 with SwiGLU 12.6 -> 9.2.
+// The 8 weights of a 16x16x32 B fragment from quant bytes b0..b7: mask keeps the lane's nibbles,
+// mul / add take 1024 + byte to q - 8 (1, -1032 for low nibbles; 1/16, -72 for high ones).
+__device__ inline h8 dequant_frag(u2 q, uint32_t mask, h2 mul, h2 add, uint32_t scale_word) {
+  const _Float16 s = __builtin_bit_cast(h2, scale_word)[0];
+  const h2 scale = {s, s};
+  const uint32_t lo = q[0] & mask, hi = q[1] & mask;
+  const h2 p0 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, lo, 0x04010400u));
+  const h2 p1 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, lo, 0x04030402u));
+  const h2 p2 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, hi, 0x04010400u));
+  const h2 p3 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, hi, 0x04030402u));
+  const h2 c0 = __builtin_elementwise_fma(p0, mul, add) * scale, c1 = __builtin_elementwise_fma(p1, mul, add) * scale;
+  const h2 c2 = __builtin_elementwise_fma(p2, mul, add) * scale, c3 = __builtin_elementwise_fma(p3, mul, add) * scale;
+  return __builtin_bit_cast(h8, u4{__builtin_bit_cast(uint32_t, c0), __builtin_bit_cast(uint32_t, c1),
+                                   __builtin_bit_cast(uint32_t, c2), __builtin_bit_cast(uint32_t, c3)});
+}
+// A dword per lane whose 16-lane rows hold (s0 s1 s0 s1): s0 and s1 in every lane.
+__device__ inline u2 spread_rows(uint32_t s) {
+  const auto r = __builtin_amdgcn_permlane16_swap(s, s, false, false);
+  return u2{r[0], r[1]};
+}
+
+template <bool SWIGLU, int G>
+__global__ __launch_bounds__(256 * G, 3) void q4_mid_kernel(const _Float16* x, int64_t ldx, int M, int K,
+                                                            const uint8_t* w, uint32_t w_bytes, int N, _Float16* y,
+                                                            int64_t ldy, int chunk_blocks, int tiles_n,
+                                                            int tiles_total, int per_xcd) {
+  constexpr int kTileM = 64, kTileN = 128, kBlock = kTileM * 64, kStage = 2 * kBlock;
+  __shared__ __attribute__((aligned(1024))) char sA0[G * kStage];
+  __shared__ __attribute__((aligned(1024))) char sA1[G * kStage];
+  __shared__ __attribute__((aligned(1024))) char sA2[G * kStage];
+  __shared__ __attribute__((aligned(1024))) char sA3[G * kStage];
+
+  const int u = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (u >= tiles_total) return;
+  const int m0 = (u / tiles_n) * kTileM, n0 = (u % tiles_n) * kTileN;
+  const int gwave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = gwave >> 2, wave = gwave & 3;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+  const int kblocks = K >> 5;
+  const int kb0 = G == 1 ? 0 : grp * chunk_blocks, kn = G == 1 ? kblocks : chunk_blocks;
+  const int k_here = min(kn, kblocks - kb0);  // blocks from k_here on are read as zeros
+
+  const uint32_t x_bytes = (uint32_t)M * (uint32_t)ldx * 2u;
+  const int arow = 16 * wave + (lane >> 2);
+  const uint32_t a_src = (uint32_t)(m0 + arow) * (uint32_t)ldx * 2u + 16u * ((lane & 3) ^ ((arow >> 2) & 3));
+  const uint32_t a_dst = grp * kStage + 1024 * wave;
+  auto load_a = [&](char* dst, int kb) Q4_INLINE {  // K blocks kb, kb + 1
+    const auto r0 = q4_rsrc(x, kb < k_here ? x_bytes : 0u), r1 = q4_rsrc(x, kb + 1 < k_here ? x_bytes : 0u);
+    q4_dma16(r0, dst + a_dst, a_src, (uint32_t)(kb0 + kb) * 64u);
+    q4_dma16(r1, dst + a_dst + kBlock, a_src, (uint32_t)(kb0 + kb + 1) * 64u);
+  };
+  // Fragment nb of this wavefront: columns n0 + 32 wave + 16 nb + l16 (SWIGLU: the gate / up rows
+  // of features n0 / 2 + 16 wave + l16).
+  const int c0 = SWIGLU ? (n0 >> 1) + 16 * wave : n0 + 32 * wave;
+  const uint32_t tstride = (uint32_t)kblocks * 32u * kQ4Record;
+  const uint32_t rec0 = (uint32_t)(c0 >> 5) * tstride + (uint32_t)((c0 & 31) + l16) * kQ4Record;
+  const uint32_t rec1 = SWIGLU ? rec0 + (uint32_t)(N >> 6) * tstride : rec0 + 16u * kQ4Record;
+  const uint32_t q_off0 = rec0 + 4u + 8u * (kq & 1), q_off1 = rec1 + 4u + 8u * (kq & 1);
+  const uint32_t s_off = kq & 1 ? rec1 : rec0;
+  const uint32_t mask = kq < 2 ? 0x0F0F0F0Fu : 0xF0F0F0F0u;
+  const _Float16 mulc = (_Float16)(kq < 2 ? 1.0f : 0.0625f), addc = (_Float16)(kq < 2 ? -1032.0f : -72.0f);
+  const h2 mul = {mulc, mulc}, add = {addc, addc};
+  struct WRegs {
+    uint32_t s;
+    u2 q0, q1;
+  };
+  auto load_w = [&](WRegs& r, int kb) Q4_INLINE {
+    const auto rs = q4_rsrc(w, kb < k_here ? w_bytes : 0u);
+    const uint32_t so = (uint32_t)(kb0 + kb) * (32u * kQ4Record);
+    r.s = __builtin_amdgcn_raw_buffer_load_b32(rs, s_off, so, 0);
+    r.q0 = __builtin_amdgcn_raw_buffer_load_b64(rs, q_off0, so, 0);
+    r.q1 = __builtin_amdgcn_raw_buffer_load_b64(rs, q_off1, so, 0);
+  };
+  f4 acc[4][2];
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb) acc[mb][0] = acc[mb][1] = f4{};
+  const uint32_t a_rd = grp * kStage + q4_lds_off(l16, kq);
+  struct Frags {
+    h8 a[4], b[2];
+  };
+  Frags fe, fo;  // even and odd K blocks
+  auto read_a = [&](Frags& f, const char* p) Q4_INLINE {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f.a[i] = *reinterpret_cast<const h8*>(p + a_rd + 1024 * i);
+  };
+  auto weights = [&](Frags& f, const WRegs& r) Q4_INLINE {
+    const u2 sc = spread_rows(r.s);
+    f.b[0] = dequant_frag(r.q0, mask, mul, add, sc[0]);
+    f.b[1] = dequant_frag(r.q1, mask, mul, add, sc[1]);
+  };
+  auto mma = [&](const Frags& f) Q4_INLINE {
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = q4_mfma16(f.b[nb], f.a[mb], acc[mb][nb]);
+  };
+  WRegs wreg[4];
+  load_a(sA0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  load_a(sA1, 2);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) load_w(wreg[i], i);
+  __builtin_amdgcn_sched_barrier(0);
+  load_a(sA2, 4);
+  __builtin_amdgcn_sched_barrier(0);
+  load_a(sA3, 6);
+  q4_barrier<12 + 6>();  // X blocks 0, 1
+  read_a(fe, sA0);
+  weights(fe, wreg[0]);
+  load_w(wreg[0], 4);
+  __builtin_amdgcn_sched_barrier(0);
+  // Stage of K blocks kb, kb + 1 in `cur`.  The X blocks of stage + 1 have landed by its barrier,
+  // which also frees `cur` for stage + 4.  Vector-memory operations newer than that stage's last
+  // X load at the barrier: two stages' X loads (4) and at least five blocks' weight loads (15).
+  auto stage = [&](char* cur, const char* nxt, WRegs& w1, WRegs& w2, int kb) Q4_INLINE {
+    read_a(fo, cur + kBlock);
+    weights(fo, w1);
+    load_w(w1, kb + 5);
+    mma(fe);
+    q4_barrier<19>();
+    load_a(cur, kb + 8);
+    read_a(fe, nxt);
+    weights(fe, w2);
+    load_w(w2, kb + 6);
+    mma(fo);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (int kb = 0; kb < kn; kb += 8) {  // blocks past the end add zero products
+    stage(sA0, sA1, wreg[1], wreg[2], kb);
+    stage(sA1, sA2, wreg[3], wreg[0], kb + 2);
+    stage(sA2, sA3, wreg[1], wreg[2], kb + 4);
+    stage(sA3, sA0, wreg[3], wreg[0], kb + 6);
+  }
+  q4_barrier<0>();
+
+  // G = 2: the groups' chains meet; group g finishes row fragments 2 g, 2 g + 1.
+  if constexpr (G == 2) {
+    char* const ex = (wave == 0 ? sA0 : wave == 1 ? sA1 : wave == 2 ? sA2 : sA3) + 16 * lane;
+    if (grp == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<f4*>(ex + 1024 * i) = acc[2 + (i >> 1)][i & 1];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<f4*>(ex + 4096 + 1024 * i) = acc[i >> 1][i & 1];
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        acc[i >> 1][i & 1] = acc[i >> 1][i & 1] + *reinterpret_cast<const f4*>(ex + 4096 + 1024 * i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        acc[i >> 1][i & 1] = acc[2 + (i >> 1)][i & 1] + *reinterpret_cast<const f4*>(ex + 1024 * i);
+    }
+    __syncthreads();
+  }
+  // Output through LDS (rows 0-31 in sA0, 32-63 in sA1), stored as whole rows of the tile.  Lane
+  // (l16, kq) holds row 16 mb + l16, columns 16 nb + 4 kq .. +3 of the wavefront's 32.
+  constexpr int kPieces = SWIGLU ? 8 : 16;  // 16-byte pieces of a row
+  auto at = [&](int row, int c) Q4_INLINE {
+    return (row < 32 ? sA0 : sA1) + (row & 31) * (16 * kPieces) + ((SWIGLU ? c ^ ((row >> 1) & 7) : c ^ (row & 15)) << 4);
+  };
+#pragma unroll
+  for (int i = 0; i < 4 / G; ++i) {
+    const int row = 32 * grp + 16 * i + l16;
+    if constexpr (SWIGLU) {
+      const f4 &g = acc[i][0], &t = acc[i][1];
+      *reinterpret_cast<u2*>(at(row, 2 * wave + (kq >> 1)) + 8 * (kq & 1)) =
+          u2{q4_pack(swiglu_value((_Float16)g[0], (_Float16)t[0]), swiglu_value((_Float16)g[1], (_Float16)t[1])),
+             q4_pack(swiglu_value((_Float16)g[2], (_Float16)t[2]), swiglu_value((_Float16)g[3], (_Float16)t[3]))};
+    } else {
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) {
+        const f4& f = acc[i][nb];
+        *reinterpret_cast<u2*>(at(row, 4 * wave + 2 * nb + (kq >> 1)) + 8 * (kq & 1)) =
+            u2{q4_pack((_Float16)f[0], (_Float16)f[1]), q4_pack((_Float16)f[2], (_Float16)f[3])};
+      }
+    }
+  }
+  __syncthreads();
+  const auto yrs = q4_rsrc(y, (uint32_t)M * (uint32_t)ldy * 2u);
+  const int n_out = SWIGLU ? N >> 1 : N, col0 = SWIGLU ? n0 >> 1 : n0;
+  constexpr int kRowsPer = 256 * G / kPieces;  // rows per store of the workgroup
+#pragma unroll
+  for (int i = 0; i < kTileM / kRowsPer; ++i) {
+    const int row = kRowsPer * i + (int)threadIdx.x / kPieces, c = threadIdx.x % kPieces;
+    const int m = m0 + row, n = col0 + 8 * c;
+    q4_store16(*reinterpret_cast<const u4*>(at(row, c)), yrs,
+               m < M && n + 8 <= n_out ? ((uint32_t)m * (uint32_t)ldy + (uint32_t)n) * 2u : 0x80000000u);
+  }
+  // A last piece of fewer than 8 columns goes element by element.
+  const int part = (n_out - col0) >> 3;
+  if ((n_out & 7) && part < kPieces) {
+#pragma unroll 1
+    for (int i = threadIdx.x; i < kTileM * 8; i += 256 * G) {
+      const int row = i >> 3, m = m0 + row, n = col0 + 8 * part + (i & 7);
+      const _Float16 v = *reinterpret_cast<const _Float16*>(at(row, part) + 2 * (i & 7));
+      q4_store_b16(v, yrs, m < M && n < n_out ? ((uint32_t)m * (uint32_t)ldy + (uint32_t)n) * 2u : 0x80000000u);
+    }
+  }
+}
+
+template <bool SWIGLU, int G>
+void launch_q4_mid(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
+                   _Float16* y, int64_t ldy, hipStream_t stream) {
+  const int tiles_m = (M + 63) / 64, tiles_n = (N + 127) / 128, tiles = tiles_m * tiles_n, per_xcd = (tiles + 7) / 8;
+  hipLaunchKernelGGL((q4_mid_kernel<SWIGLU, G>), dim3((unsigned)(8 * per_xcd)), dim3(256 * G), 0, stream, x, ldx, M, K,
+                     w, w_bytes, N, y, ldy, q4_chunk_blocks(K), tiles_n, tiles, per_xcd);
+}
+
 // ---- small launches (at most kQ4DirectBlocks 32 x 32 output blocks): one wavefront per block,
-// one wavefront per workgroup, and no LDS.
-// At small M the tiled kernel's time is its K loop's latency chain -- dequantised weights to
-// LDS, barrier, fragment reads, MFMAs -- about 0.3 us per 32-column K block for every M up to
-// ~1,500, on as few as 8 workgroups.  Here each wavefront loads its own X rows and weight records
-// straight into MFMA fragment registers, kQ4Ahead K blocks ahead, dequantises them with the same
-// code and runs the same MFMA chain: per output element the same operands in the same order
-// (K block by K block, its 16-column step 0 then step 1, from a zero accumulator), so the result
-// is bit for bit the tiled kernel's and a row does not depend on the batch it is in.
+// one wavefront per workgroup, and no LDS.  Each wavefront loads its own X rows and weight records
+// straight into MFMA fragment registers, kQ4Ahead K blocks ahead, dequantises them with the same code
+// and runs the same MFMA chain: per output element the same operands in the same order, so the
+// result is bit for bit the other kernels' and a row does not depend on the batch it is in.
 // Lane (l32, hl) holds X row m0 + l32 and weight row n0 + l32, columns 16 s + 8 hl .. +7 of the
-// K block in step s (the tiled kernel's fragment layout).  SWIGLU: two chains, the gate rows
-// n0 + l32 and the up rows n_inter + n0 + l32 of the 32 output features n0 .. n0 + 31.
+// K block in step s.  SWIGLU: two chains, the gate rows n0 + l32 and the up rows n_inter + n0 + l32
+// of the 32 output features n0 .. n0 + 31.
 // A wavefront is bound by its own dequantisation VALU work (~0.11 us per K block, twice that
 // with SWIGLU's two chains) and its X loads, which touch one cache line per row: one wavefront
 // per workgroup spreads the blocks over as many CUs (measured 2x faster than four per
-// workgroup).  Up to 512 blocks (two per CU) it beats the tiled kernel on all four projection
-// shapes; deeper rings and coalesced X loads staged through LDS measured slower.
+// workgroup).  Up to 512 blocks (two per CU) it beats q4_mid_kernel (500 x 2048 -> 1024: 11.9
+// against 12.8 us; 64 x 1024 -> 4096: 6.0 against 8.5); deeper rings and coalesced X loads staged
+// through LDS measured slower.
 constexpr int kQ4DirectBlocks = 512;
 constexpr int kQ4Ahead = 8;  // K blocks in flight per wavefront (a ring of register stages)
 
-// One workgroup per output block.  CH = 0: K is one chunk.  CH = 1: one wavefront per K chunk;
-// wavefront c runs chunk c's chain, the chains meet in LDS and wavefront 0 sums them in chunk
-// order, as the tiled kernel does.  CH = 2: one wavefront runs the chunks in turn and folds each
-// finished chain into a second accumulator (launches whose chunk wavefronts would crowd the CUs).
+// One workgroup per output block.  CH = 0: K is one chain.  CH = 1: a wavefront per half of K; the
+// chains meet in LDS and wavefront 0 adds them.  CH = 2: one wavefront runs the halves in turn and
+// adds the second chain to the first (launches whose second wavefronts would crowd the CUs).
 // CH = 3 (SWIGLU, K one chunk): two wavefronts, the gate chain and the up chain, which meet in LDS
 // for the epilogue.
-constexpr int kQ4MaxChunks = 8;  // K <= 8192 on this path
+constexpr int kQ4MaxChunks = 2;
 // CH = 1 up to one output block per CU.  Measured at M = 15-240 for the output and down
 // projections: 25-46% faster than one wavefront folding the chunks; with more blocks the chunk
 // wavefronts share CUs and were up to 13% slower.
@@ -387,7 +643,7 @@ constexpr int kQ4ChunkParallelBlocks = 256;
 template <bool SWIGLU, int CH>
 __global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) void q4_direct_kernel(
     const _Float16* __restrict__ x, int64_t ldx, int M, int K, const uint8_t* __restrict__ w, uint32_t w_bytes, int N,
-    _Float16* __restrict__ y, int64_t ldy, int blocks_m, int blocks_total) {
+    _Float16* __restrict__ y, int64_t ldy, int chunk_blocks, int blocks_m, int blocks_total) {
   static_assert(CH != 3 || SWIGLU, "gate/up wavefront pairs are a SWIGLU form");
   const int lane = threadIdx.x & 63, l32 = lane & 31, hl = lane >> 5;
   constexpr bool CHUNKED = CH == 1;
@@ -401,8 +657,8 @@ __global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) v
   const int m0 = (g % blocks_m) * 32, n0 = (g / blocks_m) * 32;
   const int kblocks_all = K >> 5;
   // This wavefront's K blocks [kb0, kblocks): one chunk, or all of K.
-  const int kb0 = CHUNKED ? chunk * kQ4ChunkBlocks : 0;
-  const int kblocks = CHUNKED ? min(kb0 + kQ4ChunkBlocks, kblocks_all) : kblocks_all;
+  const int kb0 = CHUNKED ? chunk * chunk_blocks : 0;
+  const int kblocks = CHUNKED ? min(kb0 + chunk_blocks, kblocks_all) : kblocks_all;
   const int n_out = SWIGLU ? N >> 1 : N;  // output columns
 
   const auto xrs = q4_rsrc(x, (uint32_t)M * (uint32_t)ldx * 2u);  // rows >= M read as zeros
@@ -462,7 +718,6 @@ __global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) v
   // kb + kQ4Ahead.
   constexpr int kWait = (kQ4Ahead - 1) * kOps;
   static_assert(kWait < 64, "vmcnt is 6 bits");
-  static_assert(kQ4ChunkBlocks % kQ4Ahead == 0, "chunk ends fall between ring passes");
   f16x tot_g = {}, tot_u = {};
   for (int kb = kb0; kb < kblocks; kb += kQ4Ahead) {
 #pragma unroll
@@ -475,11 +730,11 @@ __global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) v
     }
     if constexpr (CH == 2) {
       // End of a chunk (or of K): fold the chain into the sum and start the next from zero.
-      if ((kb + kQ4Ahead) % kQ4ChunkBlocks == 0 || kb + kQ4Ahead >= kblocks) {
-        tot_g = kb < kQ4ChunkBlocks ? acc_g : tot_g + acc_g;
+      if (kb + kQ4Ahead == chunk_blocks || kb + kQ4Ahead >= kblocks) {
+        tot_g = kb < chunk_blocks ? acc_g : tot_g + acc_g;
         acc_g = f16x{};
         if constexpr (BOTH) {
-          tot_u = kb < kQ4ChunkBlocks ? acc_u : tot_u + acc_u;
+          tot_u = kb < chunk_blocks ? acc_u : tot_u + acc_u;
           acc_u = f16x{};
         }
       }
@@ -494,14 +749,13 @@ __global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) v
     // The chains of chunks 1.. meet wavefront 0's (chunk 0) in LDS; it adds them in chunk order.
     __shared__ f16x part_g[kQ4MaxChunks - 1][64];
     __shared__ f16x part_u[SWIGLU ? kQ4MaxChunks - 1 : 1][SWIGLU ? 64 : 1];
-    const int nch = (kblocks_all + kQ4ChunkBlocks - 1) / kQ4ChunkBlocks;
     if (chunk > 0) {
       part_g[chunk - 1][lane] = acc_g;
       if constexpr (SWIGLU) part_u[chunk - 1][lane] = acc_u;
     }
     __syncthreads();
     if (chunk > 0) return;
-    for (int c = 1; c < nch; ++c) {
+    for (int c = 1; c < kQ4MaxChunks; ++c) {
       acc_g = acc_g + part_g[c - 1][lane];
       if constexpr (SWIGLU) acc_u = acc_u + part_u[c - 1][lane];
     }
@@ -533,116 +787,69 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
                       _Float16* y, int64_t ldy, hipStream_t stream) {
   const int n_out = SWIGLU ? N / 2 : N;
   const int blocks_m = (M + 31) / 32, blocks = blocks_m * ((n_out + 31) / 32);
-  const int chunks = (K / 32 + kQ4ChunkBlocks - 1) / kQ4ChunkBlocks;
+  const int cb = q4_chunk_blocks(K), chunks = cb < K / 32 ? 2 : 1;
   if (chunks > 1 && blocks <= kQ4ChunkParallelBlocks)
     hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, 1>), dim3((unsigned)blocks), dim3(64 * chunks), 0, stream, x, ldx,
-                       M, K, w, w_bytes, N, y, ldy, blocks_m, blocks);
+                       M, K, w, w_bytes, N, y, ldy, cb, blocks_m, blocks);
   else if (chunks > 1)
     hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, 2>), dim3((unsigned)blocks), dim3(64), 0, stream, x, ldx, M, K, w,
-                       w_bytes, N, y, ldy, blocks_m, blocks);
+                       w_bytes, N, y, ldy, cb, blocks_m, blocks);
   else if (SWIGLU && blocks <= kQ4ChunkParallelBlocks)
     hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, SWIGLU ? 3 : 0>), dim3((unsigned)blocks), dim3(128), 0, stream, x,
-                       ldx, M, K, w, w_bytes, N, y, ldy, blocks_m, blocks);
+                       ldx, M, K, w, w_bytes, N, y, ldy, cb, blocks_m, blocks);
   else
     hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, 0>), dim3((unsigned)blocks), dim3(64), 0, stream, x, ldx, M,
-                       K, w, w_bytes, N, y, ldy, blocks_m, blocks);
+                       K, w, w_bytes, N, y, ldy, cb, blocks_m, blocks);
 }
 
-// y = f16(part[0] + part[1] + ...), summed in chunk order (part: chunks x M x N fp32).  Thread =
-// four consecutive columns of row blockIdx.y (16-byte partial loads and an 8-byte store when the
-// alignment allows; the same fp32 additions either way).
-__global__ __launch_bounds__(256) void q4_reduce_kernel(const float* __restrict__ part, int chunks, int M, int N,
-                                                        _Float16* __restrict__ y, int64_t ldy) {
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-  const int m = blockIdx.y;
-  const int n0 = (blockIdx.x * 256 + threadIdx.x) * 4;
-  if (n0 >= N) return;
-  const size_t plane = (size_t)M * (size_t)N;
-  const float* p = part + (size_t)m * N + n0;
-  _Float16* yr = y + (int64_t)m * ldy + n0;
-  if ((N & 3) == 0) {  // rows, planes and this thread's columns start 16-byte aligned
-    f4 s = *reinterpret_cast<const f4*>(p);
-    for (int c = 1; c < chunks; ++c) s = s + *reinterpret_cast<const f4*>(p + (size_t)c * plane);
-    const h4 v = {(_Float16)s[0], (_Float16)s[1], (_Float16)s[2], (_Float16)s[3]};
-    if ((reinterpret_cast<uintptr_t>(yr) & 7) == 0) {
-      *reinterpret_cast<h4*>(yr) = v;
-    } else {
-      yr[0] = v[0];
-      yr[1] = v[1];
-      yr[2] = v[2];
-      yr[3] = v[3];
-    }
-  } else {
-    for (int j = 0; j < 4 && n0 + j < N; ++j) {
-      float s = p[j];
-      for (int c = 1; c < chunks; ++c) s = s + p[(size_t)c * plane + j];
-      yr[j] = (_Float16)s;
-    }
-  }
-}
-
-// Grid: 8 * ceil(tiles / 8) workgroups of 256 threads (the surplus ones exit at once), 128 x 128
-// tiles, or 64 x 128 when the launch has fewer than kQ4SmallLaunch 128 x 128 tiles.
-template <bool SWIGLU, int BM, int CH>
-void launch_q4_shape(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
-                     _Float16* y, int64_t ldy, hipStream_t stream, float* part = nullptr, int chunks = 1) {
-  const int tiles_m = (M + 64 * BM - 1) / (64 * BM), tiles_n = (N + kQ4TileN - 1) / kQ4TileN;
-  const int units = tiles_m * tiles_n * (CH == 2 ? chunks : 1), per_xcd = (units + 7) / 8;
-  hipLaunchKernelGGL((q4_matmul_kernel<SWIGLU, BM, CH>), dim3((unsigned)(8 * per_xcd)), dim3(256), 0, stream, x, ldx,
-                     M, K, w, w_bytes, N, y, ldy, tiles_n, units, per_xcd, part, chunks);
-}
-template <bool SWIGLU, int BM>
-void launch_q4_tiled(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
-                     _Float16* y, int64_t ldy, hipStream_t stream) {
-  if (K / 32 > kQ4ChunkBlocks)
-    launch_q4_shape<SWIGLU, BM, 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
-  else
-    launch_q4_shape<SWIGLU, BM, 0>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
-}
-
-size_t q4_split_bytes(int M, int K, int N) {
-  const int chunks = (K / 32 + kQ4ChunkBlocks - 1) / kQ4ChunkBlocks;
-  const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + kQ4TileN - 1) / kQ4TileN);
-  if (chunks < 2 || tiles >= kQ4SplitTiles) return 0;
-  return (size_t)chunks * (size_t)M * (size_t)N * sizeof(float);
-}
-
+// The kernel and tile by the number of tiles, i.e. by how a launch fills the 256 CUs (times in us).
+// K up to 1024:
+//   * up to 512 tiles of 64 x 128: q4_mid_kernel (N = 4096: M = 1,000 14.7, 256 x 128 tiles 17.0;
+//     M = 1,500, 768 tiles, 19.6 against 18.1);
+//   * then 256 x 128 tiles while they are at most one per CU (N = 6144: M = 1,000 18.2, 256 x 256
+//     tiles 26.5);
+//   * then 256 x 256 tiles where their last round of 256 is mostly full (N = 4096: M = 2,400 27.5
+//     against 29.5, M = 8,000 65 against 68), else 256 x 128 tiles, whose second workgroup per CU
+//     fills the gap (N = 6144, M = 4,000: 1.5 rounds, 60 against 53).
+// K above 1024 (N = 1024, K = 2048):
+//   * up to 256 tiles of 64 x 128: q4_mid_kernel (M = 1,419 13.2, 128 x 128 tiles 19.8);
+//   * then 128 x 128 tiles while at most one per CU (M = 2,400 20.3, mid 25.4, 256 x 128 27.6);
+//   * then 256 x 128 or 128 x 128 tiles by the rounds each needs (M = 8,000: one round of 38.8 against
+//     two of 22.7).
 template <bool SWIGLU>
 hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
-                     _Float16* y, int64_t ldy, hipStream_t stream, float* ws, size_t ws_bytes,
-                     const RowNorm* norm = nullptr, bool* normed = nullptr) {
-  const int64_t big_tiles = (int64_t)((M + 127) / 128) * ((N + kQ4TileN - 1) / kQ4TileN);
+                     _Float16* y, int64_t ldy, hipStream_t stream) {
   const int n_out = SWIGLU ? N / 2 : N;
-  const size_t split = SWIGLU ? 0 : q4_split_bytes(M, K, N);
-  const int chunks = (K / 32 + kQ4ChunkBlocks - 1) / kQ4ChunkBlocks;
-  if ((int64_t)((M + 31) / 32) * ((n_out + 31) / 32) <= kQ4DirectBlocks && chunks <= kQ4MaxChunks) {
+  const auto tiles = [&](int tm, int tn) { return (int64_t)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
+  const auto rounds = [](int64_t t) { return (t + 255) / 256; };
+#define Q4_TILE(MF, NWN, G) launch_q4_tile<SWIGLU, MF, NWN, G>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream)
+  if ((int64_t)((M + 31) / 32) * ((n_out + 31) / 32) <= kQ4DirectBlocks) {
     launch_q4_direct<SWIGLU>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
-  } else if (split && ws && split <= ws_bytes) {
-    launch_q4_shape<SWIGLU, 1, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream, ws, chunks);
-    if (norm && N % 8 == 0 && N <= kRmsMaxWidth) {
-      // the sums go straight into the residual add + RMSNorm that follows the projection
-      const hipError_t e = launch_reduce_rmsnorm(ws, chunks, M, N, *norm, stream);
-      if (e != hipSuccess) return e;
-      if (normed) *normed = true;
-    } else {
-      // one row per grid row (M < 64 * kQ4SplitTiles here), 1024 columns per workgroup
-      hipLaunchKernelGGL(q4_reduce_kernel, dim3((unsigned)((N + 1023) / 1024), (unsigned)M), dim3(256), 0, stream,
-                         ws, chunks, M, N, y, ldy);
-    }
-  } else if (big_tiles < kQ4SmallLaunch) {
-    launch_q4_tiled<SWIGLU, 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+  } else if (q4_chunk_blocks(K) == K / 32) {
+    const int64_t t = tiles(256, 256);
+    if (tiles(64, 128) <= 512)
+      launch_q4_mid<SWIGLU, 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+    else if (tiles(256, 128) <= 256 || (t > 256 && 256 * rounds(t) * 100 > 115 * t))
+      Q4_TILE(8, 2, 1);
+    else
+      Q4_TILE(8, 4, 1);
   } else {
-    launch_q4_tiled<SWIGLU, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+    const int64_t big = rounds(tiles(256, 128)), small = rounds(tiles(128, 128));
+    if (tiles(64, 128) <= 256)
+      launch_q4_mid<SWIGLU, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+    else if (small > 1 && 5 * big <= 3 * small)
+      Q4_TILE(8, 2, 2);
+    else
+      Q4_TILE(4, 2, 2);
   }
+#undef Q4_TILE
   return hipGetLastError();
 }
 
 hipError_t launch_q4_matmul(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
-                            _Float16* y, int64_t ldy, hipStream_t stream, float* ws, size_t ws_bytes,
-                            const RowNorm* norm, bool* normed) {
+                            _Float16* y, int64_t ldy, hipStream_t stream) {
   if (M <= 0 || N <= 0) return hipSuccess;
-  return launch_q4<false>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream, ws, ws_bytes, norm, normed);
+  return launch_q4<false>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
 }
 
 // y [M, n_inter] = swiglu of the [gate | up] projection; the weight has 2 n_inter rows and
@@ -650,7 +857,7 @@ hipError_t launch_q4_matmul(const _Float16* x, int64_t ldx, int M, int K, const 
 hipError_t launch_q4_matmul_swiglu(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes,
                                    int n_inter, _Float16* y, int64_t ldy, hipStream_t stream) {
   if (M <= 0 || n_inter <= 0) return hipSuccess;
-  return launch_q4<true>(x, ldx, M, K, w, w_bytes, 2 * n_inter, y, ldy, stream, nullptr, 0);
+  return launch_q4<true>(x, ldx, M, K, w, w_bytes, 2 * n_inter, y, ldy, stream);
 }
 
 }  // namespace qattn

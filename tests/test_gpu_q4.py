@@ -195,3 +195,36 @@ def test_q4_matmul_invalid_arguments(ctx, qattn):
             ctx.q4_matmul_swiglu(buf.ptr, 4, 64, buf.ptr, w_bytes, n_inter, buf.ptr, ldy=ldy)
         assert e.value.code == qattn.EINVAL, (n_inter, ldy, w_bytes)
     buf.free()
+
+
+# (m, k, n): each launch takes another kernel or tile of the dispatch, at its edges: ragged last tiles
+# in M and N, K blocks that are no multiple of the loops' four and eight, N no multiple of 8.
+TILE_CASES = [
+    (65, 96, 6001, False),      # 64 x 128 tiles, one row past a tile, N odd
+    (1025, 1024, 4096, False),  # 256 x 128
+    (500, 160, 12300, False),   # 256 x 128, K padded to 8 blocks, N = 8 k + 4
+    (4100, 64, 4352, False),    # 256 x 128 for its fuller last round
+    (2100, 1024, 4096, False),  # 256 x 256
+    (2570, 32, 4100, False),    # 256 x 256, one K block
+    (1900, 1056, 520, False),   # halves of 24 and 9 K blocks, 64 x 128
+    (2100, 2048, 1024, False),  # halves, 128 x 128
+    (4200, 3072, 1000, False),  # halves, 256 x 128
+    (200, 1024, 6144, True), (1030, 1024, 6144, True), (1300, 1024, 6144, True),  # n: gate + up rows
+    (2100, 96, 6144, True), (23000, 32, 384, True), (5000, 1120, 384, True), (700, 2048, 6144, True),
+]
+
+
+@pytest.mark.parametrize("m,k,n,swiglu", TILE_CASES)
+def test_q4_tiled_launches_equal_small_launches_bit_for_bit(ctx, m, k, n, swiglu):
+    """All rows of a launch against the same rows in 32-row launches, which take the
+    one-wavefront-per-block kernel (itself checked against the oracle above): equal bit for bit."""
+    rng = np.random.default_rng(m + k + n)
+    packed = random_compact(rng, n, k)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    run = (lambda v: run_q4_swiglu(ctx, v, packed, k, n // 2)) if swiglu else (lambda v: run_q4(ctx, v, packed, k, n))
+    cols = n // 2 if swiglu else n
+    whole = run(x)[:, :cols].view(np.uint16)
+    starts = sorted(set(list(range(0, m, 32 * max(1, m // 512))) + [max(0, m - 32)]))
+    for a in starts:
+        small = run(x[a:a + 32])[:, :cols].view(np.uint16)
+        assert np.array_equal(whole[a:a + 32], small), (a, np.argwhere(whole[a:a + 32] != small)[:4])
