@@ -8,7 +8,7 @@
 // The weight is f16(scale * (q - 8)), as the reference dequantises it; the products and sums run
 // in fp32 on the matrix cores (the reference accumulates in f16).
 //
-// Three kernels, one result: every output element is the same MFMA chain (its K blocks in turn from
+// Four kernels, one result: every output element is the same MFMA chain (its K blocks in turn from
 // a zero accumulator, the two halves of a K above 1024 columns added at the end), so a row does not
 // depend on the launch it is in.  v_mfma_f32_16x16x32_f16 on a K block equals two chained
 // v_mfma_f32_32x32x16_f16 on its halves bit for bit, which lets each kernel take the shape it needs.
@@ -16,8 +16,9 @@
 //     LDS-DMA, every weight record dequantised once per workgroup into an LDS tile;
 //   * q4_mid_kernel, medium launches: 64 x 128 tiles, X by LDS-DMA, the weights dequantised
 //     straight into each wavefront's MFMA fragments;
-//   * q4_direct_kernel, at most kQ4DirectBlocks 32 x 32 output blocks: one workgroup per block, no
-//     tile staging.
+//   * q4_direct_kernel, K above 1024 and at most kQ4DirectBlocks 32 x 32 output blocks: a wavefront
+//     per block, no tile staging;
+//   * q4_small_kernel, the smallest launches: a workgroup per 16- or 32-row block, K shared out.
 // Tiles are numbered so that consecutive workgroups on one XCD (workgroup b runs on XCD b % 8)
 // walk the N tiles of one M tile: its X rows stay in that XCD's L2.  The SWIGLU variants (the FFN's
 // gate/up projection, model.ts:126-127) map B rows onto a feature's gate and up rows and write
@@ -98,6 +99,12 @@ __device__ inline void q4_dma16(__amdgpu_buffer_rsrc_t rs, char* dst, uint32_t o
 }
 __device__ inline void q4_store16(u4 v, __amdgpu_buffer_rsrc_t rs, uint32_t off) {
   __builtin_amdgcn_raw_buffer_store_b128(v, rs, off, 0, 0);
+}
+__device__ inline u4 q4_load16(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  return __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
+}
+__device__ inline void q4_store8(u2 v, __amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  __builtin_amdgcn_raw_buffer_store_b64(v, rs, off, 0, 0);
 }
 __device__ inline uint32_t q4_pack(_Float16 a, _Float16 b) {
   return (uint32_t)__builtin_bit_cast(unsigned short, a) | (uint32_t)__builtin_bit_cast(unsigned short, b) << 16;
@@ -613,52 +620,177 @@ void launch_q4_mid(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* 
                      w, w_bytes, N, y, ldy, q4_chunk_blocks(K), tiles_n, tiles, per_xcd);
 }
 
-// ---- small launches (at most kQ4DirectBlocks 32 x 32 output blocks): one wavefront per block,
-// one wavefront per workgroup, and no LDS.  Each wavefront loads its own X rows and weight records
-// straight into MFMA fragment registers, kQ4Ahead K blocks ahead, dequantises them with the same code
-// and runs the same MFMA chain: per output element the same operands in the same order, so the
-// result is bit for bit the other kernels' and a row does not depend on the batch it is in.
+// ---- the smallest launches: one workgroup per 16 MB x 32 block of output (SWIGLU: 16 features),
+// its wavefronts sharing K.  Wavefront p of a chain loads and dequantises K blocks NKB p .. + NKB - 1,
+// all at once; then the chain runs through the wavefronts in turn, the accumulators passing from one
+// to the next through LDS, so the sums are the same as in one wavefront.  H = 2 (K above 1024): both
+// halves of K run side by side and are added at the end.
+// What bounds it: a launch's fixed 3 us or so, one memory round trip, and P hand-overs of about 0.2 us;
+// one wavefront running the whole chain dequantised 32 blocks in sequence instead.  Weight records
+// come in as they lie in memory (three 1 KiB loads per four blocks, not twelve of scattered 4- and
+// 8-byte pieces, whose address work alone took 2 us per CU) and are taken apart in LDS.
+// Measured (us, before -> after): 15 x 1024 -> 4096 5.9 -> 4.5, 15 rows gate/up 6.6 -> 4.6,
+// 50 x 2048 -> 1024 7.5 -> 5.4, 50 x 3072 -> 1024 10.3 -> 6.7.
+template <bool SWIGLU, int MB, int NKB, int H>
+__global__ __launch_bounds__(1024) void q4_small_kernel(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w,
+                                                        uint32_t w_bytes, int N, _Float16* y, int64_t ldy,
+                                                        int chunk_blocks, int P, int blocks_m) {
+  __shared__ f4 hand[H][2 * MB][64];
+  const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = H == 2 && wv >= P ? 1 : 0, p = wv - h * P;
+  const int m0 = (int)(blockIdx.x % (unsigned)blocks_m) * 16 * MB, nblk = (int)(blockIdx.x / (unsigned)blocks_m);
+  const int kblocks = K >> 5;
+  const int kb0 = h * chunk_blocks + p * NKB, k_end = min(kblocks, (h + 1) * chunk_blocks);
+
+  const uint32_t x_bytes = (uint32_t)M * (uint32_t)ldx * 2u;
+  const uint32_t x_off = (uint32_t)(m0 + l16) * (uint32_t)ldx * 2u + 16u * kq;
+  const int c0 = SWIGLU ? 16 * nblk : 32 * nblk;
+  const uint32_t tstride = (uint32_t)kblocks * 32u * kQ4Record;
+  const uint32_t rec0 = (uint32_t)(c0 >> 5) * tstride + (uint32_t)(c0 & 31) * kQ4Record;
+  const uint32_t rec1 = SWIGLU ? rec0 + (uint32_t)(N >> 6) * tstride : rec0 + 16u * kQ4Record;
+  const uint32_t mask = kq < 2 ? 0x0F0F0F0Fu : 0xF0F0F0F0u;
+  const _Float16 mulc = (_Float16)(kq < 2 ? 1.0f : 0.0625f), addc = (_Float16)(kq < 2 ? -1032.0f : -72.0f);
+  const h2 mul = {mulc, mulc}, add = {addc, addc};
+
+  // This wavefront's weight records (32 rows x NKB blocks of 20 bytes) go to LDS as they lie in
+  // memory, 16 bytes per lane; blocks past the chain's end are read as zeros.
+  constexpr int kRaw = (NKB * 640 + 1023) / 1024;
+  __shared__ __attribute__((aligned(1024))) char raw[16][kRaw * 1024];
+  const auto wrs = q4_rsrc(w, w_bytes);
+  u4 piece[kRaw];
+#pragma unroll
+  for (int j = 0; j < kRaw; ++j) {
+    const int unit = 64 * j + lane, kb = unit / 40, r = unit % 40;
+    const uint32_t off = (r < 20 ? rec0 + 16u * r : rec1 + 16u * (r - 20)) + (uint32_t)(kb0 + kb) * 640u;
+    piece[j] = q4_load16(wrs, kb < NKB && kb0 + kb < k_end ? off : 0x80000000u);
+  }
+  h8 a[NKB][MB];
+#pragma unroll
+  for (int i = 0; i < NKB; ++i) {
+    const auto xs = q4_rsrc(x, kb0 + i < k_end ? x_bytes : 0u);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+      a[i][mb] = __builtin_bit_cast(
+          h8, __builtin_amdgcn_raw_buffer_load_b128(xs, x_off + (uint32_t)(16 * mb) * (uint32_t)ldx * 2u,
+                                                    (uint32_t)(kb0 + i) * 64u, 0));
+  }
+#pragma unroll
+  for (int j = 0; j < kRaw; ++j) *reinterpret_cast<u4*>(raw[wv] + 1024 * j + 16 * lane) = piece[j];
+  h8 b[NKB][2];
+  const char* const mine = raw[wv] + l16 * kQ4Record + 8 * (kq & 1) + 4;
+  const char* const scales = raw[wv] + (l16 + 16 * (kq & 1)) * kQ4Record;
+#pragma unroll
+  for (int i = 0; i < NKB; ++i) {
+    const u2 sc = spread_rows(*reinterpret_cast<const uint32_t*>(scales + 640 * i));
+    const uint32_t* const q0 = reinterpret_cast<const uint32_t*>(mine + 640 * i);
+    const uint32_t* const q1 = reinterpret_cast<const uint32_t*>(mine + 640 * i + 320);
+    b[i][0] = dequant_frag(u2{q0[0], q0[1]}, mask, mul, add, sc[0]);
+    b[i][1] = dequant_frag(u2{q1[0], q1[1]}, mask, mul, add, sc[1]);
+  }
+  f4 acc[MB][2];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) acc[mb][0] = acc[mb][1] = f4{};
+  for (int t = 0; t < P; ++t) {
+    if (t == p) {
+      if (t > 0)
+#pragma unroll
+        for (int i = 0; i < 2 * MB; ++i) acc[i >> 1][i & 1] = hand[h][i][lane];
+#pragma unroll
+      for (int i = 0; i < NKB; ++i)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = q4_mfma16(b[i][nb], a[i][mb], acc[mb][nb]);
+      if (t < P - 1 || h == 1)
+#pragma unroll
+        for (int i = 0; i < 2 * MB; ++i) hand[h][i][lane] = acc[i >> 1][i & 1];
+    }
+    if (t < P - 1 || H == 2) __syncthreads();
+  }
+  if (h != 0 || p != P - 1) return;
+  if constexpr (H == 2)
+#pragma unroll
+    for (int i = 0; i < 2 * MB; ++i) acc[i >> 1][i & 1] = acc[i >> 1][i & 1] + hand[1][i][lane];
+
+  const auto yrs = q4_rsrc(y, (uint32_t)M * (uint32_t)ldy * 2u);
+  const int n_out = SWIGLU ? N >> 1 : N;
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    const int m = m0 + 16 * mb + l16;
+#pragma unroll
+    for (int nb = 0; nb < (SWIGLU ? 1 : 2); ++nb) {
+      const int n = c0 + 16 * nb + 4 * kq;
+      _Float16 v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[e] = SWIGLU ? swiglu_value((_Float16)acc[mb][0][e], (_Float16)acc[mb][1][e]) : (_Float16)acc[mb][nb][e];
+      const uint32_t off = m < M ? ((uint32_t)m * (uint32_t)ldy + (uint32_t)n) * 2u : 0x80000000u;
+      if (c0 + 32 <= n_out || n + 4 <= n_out) {
+        q4_store8(u2{q4_pack(v[0], v[1]), q4_pack(v[2], v[3])}, yrs, off);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < n_out) q4_store_b16(v[e], yrs, off + 2u * e);
+      }
+    }
+  }
+}
+
+template <bool SWIGLU, int MB>
+void launch_q4_small(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
+                     _Float16* y, int64_t ldy, hipStream_t stream) {
+  const int n_out = SWIGLU ? N / 2 : N, cb = q4_chunk_blocks(K), halves = cb < K / 32 ? 2 : 1;
+  const int blocks_m = (M + 16 * MB - 1) / (16 * MB), cols = SWIGLU ? 16 : 32, blocks = blocks_m * ((n_out + cols - 1) / cols);
+  const int nkb = cb <= 32 ? 4 : cb <= 48 ? 6 : 8, P = (cb + nkb - 1) / nkb;
+#define Q4_SMALL(NKB, H) \
+  hipLaunchKernelGGL((q4_small_kernel<SWIGLU, MB, NKB, H>), dim3((unsigned)blocks), dim3(64 * P * H), 0, stream, x, \
+                     ldx, M, K, w, w_bytes, N, y, ldy, cb, P, blocks_m)
+  if (halves == 1) {
+    Q4_SMALL(4, 1);
+  } else if constexpr (MB == 1) {
+    if (nkb == 4) Q4_SMALL(4, 2);
+    else if (nkb == 6) Q4_SMALL(6, 2);
+    else Q4_SMALL(8, 2);
+  }
+#undef Q4_SMALL
+}
+
+// ---- K above 1024, at most kQ4DirectBlocks 32 x 32 output blocks beyond q4_small_kernel's: one
+// wavefront per block (two where both halves of K run at once), and no LDS tiles.  Each wavefront
+// loads its own X rows and weight records straight into MFMA fragment registers, kQ4Ahead K blocks
+// ahead, dequantises them with the same code and runs the same MFMA chain.
 // Lane (l32, hl) holds X row m0 + l32 and weight row n0 + l32, columns 16 s + 8 hl .. +7 of the
 // K block in step s.  SWIGLU: two chains, the gate rows n0 + l32 and the up rows n_inter + n0 + l32
 // of the 32 output features n0 .. n0 + 31.
-// A wavefront is bound by its own dequantisation VALU work (~0.11 us per K block, twice that
-// with SWIGLU's two chains) and its X loads, which touch one cache line per row: one wavefront
-// per workgroup spreads the blocks over as many CUs (measured 2x faster than four per
-// workgroup).  Up to 512 blocks (two per CU) it beats q4_mid_kernel (500 x 2048 -> 1024: 11.9
-// against 12.8 us; 64 x 1024 -> 4096: 6.0 against 8.5); deeper rings and coalesced X loads staged
-// through LDS measured slower.
+// A wavefront is bound by its own dequantisation VALU work (~0.08 us per K block, twice that with
+// SWIGLU's two chains) and its X loads, which touch one cache line per row: one wavefront per
+// workgroup spreads the blocks over as many CUs.  Up to 512 blocks (two per CU) it beats
+// q4_mid_kernel (us: 500 x 2048 -> 1024 11.9 against 12.9, 250 x 3072 -> 1024 9.9 against 17.2).
 constexpr int kQ4DirectBlocks = 512;
 constexpr int kQ4Ahead = 8;  // K blocks in flight per wavefront (a ring of register stages)
 
-// One workgroup per output block.  CH = 0: K is one chain.  CH = 1: a wavefront per half of K; the
-// chains meet in LDS and wavefront 0 adds them.  CH = 2: one wavefront runs the halves in turn and
-// adds the second chain to the first (launches whose second wavefronts would crowd the CUs).
-// CH = 3 (SWIGLU, K one chunk): two wavefronts, the gate chain and the up chain, which meet in LDS
-// for the epilogue.
-constexpr int kQ4MaxChunks = 2;
-// CH = 1 up to one output block per CU.  Measured at M = 15-240 for the output and down
-// projections: 25-46% faster than one wavefront folding the chunks; with more blocks the chunk
-// wavefronts share CUs and were up to 13% slower.
-constexpr int kQ4ChunkParallelBlocks = 256;
-template <bool SWIGLU, int CH>
-__global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) void q4_direct_kernel(
+// One workgroup per output block.  PAR: a wavefront per half of K; the chains meet in LDS and
+// wavefront 0 adds them.  Otherwise one wavefront runs the halves in turn and adds the second chain
+// to the first (launches whose second wavefronts would crowd the CUs).
+// PAR up to one output block per CU.  Measured at M = 15-240 for the output and down projections:
+// 25-46% faster than one wavefront; with more blocks the second wavefronts share CUs and were up to
+// 13% slower.
+constexpr int kQ4ParallelBlocks = 256;
+template <bool SWIGLU, bool PAR>
+__global__ __launch_bounds__(PAR ? 128 : 64) void q4_direct_kernel(
     const _Float16* __restrict__ x, int64_t ldx, int M, int K, const uint8_t* __restrict__ w, uint32_t w_bytes, int N,
     _Float16* __restrict__ y, int64_t ldy, int chunk_blocks, int blocks_m, int blocks_total) {
-  static_assert(CH != 3 || SWIGLU, "gate/up wavefront pairs are a SWIGLU form");
   const int lane = threadIdx.x & 63, l32 = lane & 31, hl = lane >> 5;
-  constexpr bool CHUNKED = CH == 1;
-  constexpr bool PAIR = CH == 3;          // this wavefront runs one of the two SWIGLU chains
-  constexpr bool BOTH = SWIGLU && !PAIR;  // this wavefront runs the gate and the up chain
-  const int half = PAIR ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;  // 0 gate, 1 up
-  const int chunk = CHUNKED ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const int chunk = PAR ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   // block g: the M blocks of one N block are consecutive (they share weight records in L2)
   const int g = blockIdx.x;
   if (g >= blocks_total) return;  // the whole workgroup: its barrier below stays uniform
   const int m0 = (g % blocks_m) * 32, n0 = (g / blocks_m) * 32;
   const int kblocks_all = K >> 5;
-  // This wavefront's K blocks [kb0, kblocks): one chunk, or all of K.
-  const int kb0 = CHUNKED ? chunk * chunk_blocks : 0;
-  const int kblocks = CHUNKED ? min(kb0 + chunk_blocks, kblocks_all) : kblocks_all;
+  // This wavefront's K blocks [kb0, kblocks): one half, or all of K.
+  const int kb0 = PAR ? chunk * chunk_blocks : 0;
+  const int kblocks = PAR ? min(kb0 + chunk_blocks, kblocks_all) : kblocks_all;
   const int n_out = SWIGLU ? N >> 1 : N;  // output columns
 
   const auto xrs = q4_rsrc(x, (uint32_t)M * (uint32_t)ldx * 2u);  // rows >= M read as zeros
@@ -669,8 +801,7 @@ __global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) v
     return ((uint32_t)(n >> 5) * (uint32_t)kblocks_all * 32u + (uint32_t)(n & 31)) * kQ4Record;
   };
   const uint32_t wu_rec = SWIGLU ? w_rec(n_out + n0 + l32) : 0u;
-  // The first chain's records: the gate rows (the up rows for the second wavefront of a pair).
-  const uint32_t wg_rec = PAIR && half ? wu_rec : w_rec(n0 + l32);
+  const uint32_t wg_rec = w_rec(n0 + l32);
   const uint32_t w_step = 32u * kQ4Record;
 
   struct Stage {
@@ -678,7 +809,7 @@ __global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) v
     uint32_t sg, su;
     u2 qg, qu;
   };
-  constexpr int kOps = BOTH ? 6 : 4;  // vector-memory instructions per K block
+  constexpr int kOps = SWIGLU ? 6 : 4;  // vector-memory instructions per K block
   auto load = [&](Stage& st, int kb) {
     kb = kb < kblocks ? kb : kblocks - 1;  // past the end: re-read the last block (never used)
     const uint32_t xo = x_row + (uint32_t)kb * 64u;
@@ -687,7 +818,7 @@ __global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) v
     const uint32_t go = wg_rec + (uint32_t)kb * w_step;
     st.sg = __builtin_amdgcn_raw_buffer_load_b32(wrs, go, 0, 0);
     st.qg = __builtin_amdgcn_raw_buffer_load_b64(wrs, go + 4u + 8u * hl, 0, 0);
-    if constexpr (BOTH) {
+    if constexpr (SWIGLU) {
       const uint32_t uo = wu_rec + (uint32_t)kb * w_step;
       st.su = __builtin_amdgcn_raw_buffer_load_b32(wrs, uo, 0, 0);
       st.qu = __builtin_amdgcn_raw_buffer_load_b64(wrs, uo + 4u + 8u * hl, 0, 0);
@@ -699,7 +830,7 @@ __global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) v
     const h2 scale_g = {sg, sg};
     acc_g = q4_mfma(st.a[0], dequant8<false>(st.qg, scale_g), acc_g);
     acc_g = q4_mfma(st.a[1], dequant8<true>(st.qg, scale_g), acc_g);
-    if constexpr (BOTH) {
+    if constexpr (SWIGLU) {
       const _Float16 su = __builtin_bit_cast(h2, st.su)[0];
       const h2 scale_u = {su, su};
       acc_u = q4_mfma(st.a[0], dequant8<false>(st.qu, scale_u), acc_u);
@@ -728,12 +859,12 @@ __global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) v
       load(ring[j], kb + j + kQ4Ahead);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (CH == 2) {
-      // End of a chunk (or of K): fold the chain into the sum and start the next from zero.
+    if constexpr (!PAR) {
+      // End of a half: add the chain to the sum and start the next from zero.
       if (kb + kQ4Ahead == chunk_blocks || kb + kQ4Ahead >= kblocks) {
         tot_g = kb < chunk_blocks ? acc_g : tot_g + acc_g;
         acc_g = f16x{};
-        if constexpr (BOTH) {
+        if constexpr (SWIGLU) {
           tot_u = kb < chunk_blocks ? acc_u : tot_u + acc_u;
           acc_u = f16x{};
         }
@@ -741,34 +872,24 @@ __global__ __launch_bounds__(CH == 1 ? 64 * kQ4MaxChunks : CH == 3 ? 128 : 64) v
     }
   }
   __builtin_amdgcn_s_waitcnt(0);
-  if constexpr (CH == 2) {
+  if constexpr (!PAR) {
     acc_g = tot_g;
     acc_u = tot_u;
   }
-  if constexpr (CHUNKED) {
-    // The chains of chunks 1.. meet wavefront 0's (chunk 0) in LDS; it adds them in chunk order.
-    __shared__ f16x part_g[kQ4MaxChunks - 1][64];
-    __shared__ f16x part_u[SWIGLU ? kQ4MaxChunks - 1 : 1][SWIGLU ? 64 : 1];
+  if constexpr (PAR) {
+    __shared__ f16x part_g[64];
+    __shared__ f16x part_u[SWIGLU ? 64 : 1];
     if (chunk > 0) {
-      part_g[chunk - 1][lane] = acc_g;
-      if constexpr (SWIGLU) part_u[chunk - 1][lane] = acc_u;
+      part_g[lane] = acc_g;
+      if constexpr (SWIGLU) part_u[lane] = acc_u;
     }
     __syncthreads();
     if (chunk > 0) return;
-    for (int c = 1; c < kQ4MaxChunks; ++c) {
-      acc_g = acc_g + part_g[c - 1][lane];
-      if constexpr (SWIGLU) acc_u = acc_u + part_u[c - 1][lane];
-    }
-  }
-  if constexpr (PAIR) {
-    __shared__ f16x up[64];
-    if (half) up[lane] = acc_g;
-    __syncthreads();
-    if (half) return;
-    acc_u = up[lane];
+    acc_g = acc_g + part_g[lane];
+    if constexpr (SWIGLU) acc_u = acc_u + part_u[lane];
   }
 
-  // D (32 x 32): lane holds column l32 and rows 8 (r / 4) + 4 hl + r % 4 -- as the tiled kernel.
+  // D (32 x 32): lane holds column l32 and rows 8 (r / 4) + 4 hl + r % 4.
   const int n = n0 + l32;
   if (n >= n_out) return;
 #pragma unroll
@@ -787,23 +908,19 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
                       _Float16* y, int64_t ldy, hipStream_t stream) {
   const int n_out = SWIGLU ? N / 2 : N;
   const int blocks_m = (M + 31) / 32, blocks = blocks_m * ((n_out + 31) / 32);
-  const int cb = q4_chunk_blocks(K), chunks = cb < K / 32 ? 2 : 1;
-  if (chunks > 1 && blocks <= kQ4ChunkParallelBlocks)
-    hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, 1>), dim3((unsigned)blocks), dim3(64 * chunks), 0, stream, x, ldx,
-                       M, K, w, w_bytes, N, y, ldy, cb, blocks_m, blocks);
-  else if (chunks > 1)
-    hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, 2>), dim3((unsigned)blocks), dim3(64), 0, stream, x, ldx, M, K, w,
+  const int cb = q4_chunk_blocks(K);
+  if (blocks <= kQ4ParallelBlocks)
+    hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, true>), dim3((unsigned)blocks), dim3(128), 0, stream, x, ldx, M, K, w,
                        w_bytes, N, y, ldy, cb, blocks_m, blocks);
-  else if (SWIGLU && blocks <= kQ4ChunkParallelBlocks)
-    hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, SWIGLU ? 3 : 0>), dim3((unsigned)blocks), dim3(128), 0, stream, x,
-                       ldx, M, K, w, w_bytes, N, y, ldy, cb, blocks_m, blocks);
   else
-    hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, 0>), dim3((unsigned)blocks), dim3(64), 0, stream, x, ldx, M,
-                       K, w, w_bytes, N, y, ldy, cb, blocks_m, blocks);
+    hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, false>), dim3((unsigned)blocks), dim3(64), 0, stream, x, ldx, M, K, w,
+                       w_bytes, N, y, ldy, cb, blocks_m, blocks);
 }
 
 // The kernel and tile by the number of tiles, i.e. by how a launch fills the 256 CUs (times in us).
 // K up to 1024:
+//   * q4_small_kernel while its 16-row blocks are at most one per CU, with 32-row blocks while those are
+//     at most two (N = 4096: M = 50 5.2, mid 8.5; M = 100 7.3 against 8.6);
 //   * up to 512 tiles of 64 x 128: q4_mid_kernel (N = 4096: M = 1,000 14.7, 256 x 128 tiles 17.0;
 //     M = 1,500, 768 tiles, 19.6 against 18.1);
 //   * then 256 x 128 tiles while they are at most one per CU (N = 6144: M = 1,000 18.2, 256 x 256
@@ -812,6 +929,9 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
 //     against 29.5, M = 8,000 65 against 68), else 256 x 128 tiles, whose second workgroup per CU
 //     fills the gap (N = 6144, M = 4,000: 1.5 rounds, 60 against 53).
 // K above 1024 (N = 1024, K = 2048):
+//   * q4_small_kernel while its 16-row blocks are at most one per CU (M = 100 6.2, direct 7.5;
+//     M = 150, 320 blocks, 10.4 against 7.8) and a half's blocks fit its eight wavefronts;
+//   * q4_direct_kernel up to kQ4DirectBlocks;
 //   * up to 256 tiles of 64 x 128: q4_mid_kernel (M = 1,419 13.2, 128 x 128 tiles 19.8);
 //   * then 128 x 128 tiles while at most one per CU (M = 2,400 20.3, mid 25.4, 256 x 128 27.6);
 //   * then 256 x 128 or 128 x 128 tiles by the rounds each needs (M = 8,000: one round of 38.8 against
@@ -819,15 +939,17 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
 template <bool SWIGLU>
 hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
                      _Float16* y, int64_t ldy, hipStream_t stream) {
-  const int n_out = SWIGLU ? N / 2 : N;
+  const int n_out = SWIGLU ? N / 2 : N, cb = q4_chunk_blocks(K);
   const auto tiles = [&](int tm, int tn) { return (int64_t)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
   const auto rounds = [](int64_t t) { return (t + 255) / 256; };
 #define Q4_TILE(MF, NWN, G) launch_q4_tile<SWIGLU, MF, NWN, G>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream)
-  if ((int64_t)((M + 31) / 32) * ((n_out + 31) / 32) <= kQ4DirectBlocks) {
-    launch_q4_direct<SWIGLU>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
-  } else if (q4_chunk_blocks(K) == K / 32) {
+  if (cb == K / 32) {
     const int64_t t = tiles(256, 256);
-    if (tiles(64, 128) <= 512)
+    if (tiles(16, 32) <= 256)
+      launch_q4_small<SWIGLU, 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+    else if (tiles(32, 32) <= 512)
+      launch_q4_small<SWIGLU, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+    else if (tiles(64, 128) <= 512)
       launch_q4_mid<SWIGLU, 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if (tiles(256, 128) <= 256 || (t > 256 && 256 * rounds(t) * 100 > 115 * t))
       Q4_TILE(8, 2, 1);
@@ -835,7 +957,11 @@ hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t
       Q4_TILE(8, 4, 1);
   } else {
     const int64_t big = rounds(tiles(256, 128)), small = rounds(tiles(128, 128));
-    if (tiles(64, 128) <= 256)
+    if (tiles(16, 32) <= 256 && cb <= 64)
+      launch_q4_small<SWIGLU, 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+    else if ((int64_t)((M + 31) / 32) * ((n_out + 31) / 32) <= kQ4DirectBlocks)
+      launch_q4_direct<SWIGLU>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+    else if (tiles(64, 128) <= 256)
       launch_q4_mid<SWIGLU, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if (small > 1 && 5 * big <= 3 * small)
       Q4_TILE(8, 2, 2);

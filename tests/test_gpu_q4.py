@@ -200,6 +200,9 @@ def test_q4_matmul_invalid_arguments(ctx, qattn):
 # (m, k, n): each launch takes another kernel or tile of the dispatch, at its edges: ragged last tiles
 # in M and N, K blocks that are no multiple of the loops' four and eight, N no multiple of 8.
 TILE_CASES = [
+    (50, 1024, 4096, False), (50, 992, 1501, False), (33, 1024, 6144, True),  # 32-row blocks
+    (300, 2048, 1024, False), (500, 3072, 1023, False), (150, 1056, 384, True),  # one wavefront per block
+    (150, 3072, 2048, True), (33, 4160, 96, False),  # halves of 72 K blocks
     (65, 96, 6001, False),      # 64 x 128 tiles, one row past a tile, N odd
     (1025, 1024, 4096, False),  # 256 x 128
     (500, 160, 12300, False),   # 256 x 128, K padded to 8 blocks, N = 8 k + 4
@@ -216,8 +219,8 @@ TILE_CASES = [
 
 @pytest.mark.parametrize("m,k,n,swiglu", TILE_CASES)
 def test_q4_tiled_launches_equal_small_launches_bit_for_bit(ctx, m, k, n, swiglu):
-    """All rows of a launch against the same rows in 32-row launches, which take the
-    one-wavefront-per-block kernel (itself checked against the oracle above): equal bit for bit."""
+    """All rows of a launch against the same rows in launches of at most 32, which take the kernel
+    for the smallest launches (itself checked against the oracle above): equal bit for bit."""
     rng = np.random.default_rng(m + k + n)
     packed = random_compact(rng, n, k)
     x = rng.standard_normal((m, k)).astype(np.float16)
