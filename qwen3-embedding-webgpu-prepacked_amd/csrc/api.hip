@@ -447,6 +447,7 @@ int install_plan(qattn_run* run, const qattn_run_desc* d) {
   fill_params(&p, d, mask, info.slots, run->plan_dev[next], items_bytes, heads_bytes);
   p.partials = static_cast<float*>(run->split_dev);
   p.n_splits = plan.splits;
+  p.one_entry = plan.one_entry;
   run->params = p;
   run->cur = next;
   run->info = info;
@@ -591,6 +592,7 @@ int qattn_prefill_static(qattn_ctx* ctx, const qattn_run_desc* desc, qattn_strea
   std::memcpy(host.data() + items_bytes, plan.slot_begin.data(), slots_bytes);
   AttnParams p{};
   fill_params(&p, &d, mask, info.slots, ctx->scratch, items_bytes, 0);
+  p.one_entry = plan.one_entry;
   DeviceGuard g(ctx->device);
   hipStream_t st = pick_stream(ctx, stream);
   HIP_TRY(ctx, hipMemcpyAsync(ctx->scratch, host.data(), host.size(), hipMemcpyHostToDevice, st));

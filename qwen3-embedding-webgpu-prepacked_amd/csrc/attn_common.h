@@ -172,6 +172,7 @@ struct AttnParams {
   const WorkItem* work;       // work items grouped by slot
   const int32_t* slot_begin;  // slot b owns work[slot_begin[b] .. slot_begin[b+1])
   int32_t n_slots;            // workgroups launched
+  int32_t one_entry;          // no slot holds more than one entry
   MaskSpec mask;
   float scale_log2;           // (1/sqrt(128)) * log2(e)
   float* partials;            // split chunks' partial results (one record set per chunk)

@@ -334,6 +334,9 @@ void plan_work(const qattn_run_desc* d, int max_slots, Plan* out, qattn_run_info
         for (const WorkItem& w : lists[g][j]) out->items.push_back(w);
       out->slot_begin.push_back((int32_t)out->items.size());
     }
+  out->one_entry = true;
+  for (size_t j = 1; j < out->slot_begin.size(); ++j)
+    out->one_entry = out->one_entry && out->slot_begin[j] - out->slot_begin[j - 1] <= 1;
   info.slots = (int32_t)out->slot_begin.size() - 1;
   info.split_items = out->splits;
   info.flops = 4ll * kHeadDim * kQHeads * info.pairs;

@@ -35,6 +35,7 @@ struct Plan {
   std::vector<int32_t> slot_begin;   // n_slots + 1 offsets into items
   std::vector<WorkItem> split_heads; // chunk 0 of each split item, by split id
   int32_t splits = 0;                // items spread over several chunks
+  bool one_entry = false;            // no slot holds more than one entry
   int32_t partials = 0;              // chunk partial-result records the workspace holds
 };
 

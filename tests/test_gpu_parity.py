@@ -417,6 +417,28 @@ def test_varlen_equals_solo_and_isolation(ctx, qattn, oracle):
     assert np.array_equal(pert[s:e], Case(ctx, qattn, q, k, v, cu).run()[s:e])
 
 
+@pytest.mark.parametrize("mask", [0, 1])
+@pytest.mark.parametrize("length", [1, 33, 64, 65, 128, 129, 250, 700])
+def test_one_entry_launch_equals_the_packed_launch(ctx, qattn, oracle, length, mask):
+    """A launch whose slots hold one entry each (the variant without a next entry to load) against
+    the same sequence packed with enough others that slots hold several: equal bit for bit, with the
+    last-token row."""
+    lengths = [length] + [640] * 8
+    cu = cu_of(lengths)
+    q, k, v = oracle.gen_qkv(1, 0, cu)
+    inv = qattn.FLAG_BATCH_INVARIANT
+    solo = Case(ctx, qattn, q[:length].copy(), k[:length].copy(), v[:length].copy(), cu_of([length]), mask=mask,
+                o_last=True, flags=inv)
+    packed = Case(ctx, qattn, q, k, v, cu, mask=mask, o_last=True, flags=inv)
+    slots = lambda c: qattn.plan_slots(c.desc)  # noqa: E731
+    assert np.diff(slots(solo)).max() == 1 and np.diff(slots(packed)).max() > 1
+    a, b = solo.run(), packed.run()
+    assert np.array_equal(a, b[:length])
+    assert np.array_equal(solo.last()[0], a[-1]) and np.array_equal(packed.last()[0], a[-1])
+    solo.free()
+    packed.free()
+
+
 def test_workgroups_reach_xcds_round_robin(ctx):
     # The planner keeps every KV head's entries on slots b with one value of b % 8 and expects
     # round-robin dispatch to put them on one XCD, so the head's K/V tiles share one L2.
