@@ -723,7 +723,9 @@ int qattn_plan_mask(int32_t L, int32_t mask, int32_t prefix, int32_t window, uin
 
 // ---- producer + generator ---------------------------------------------------------------------
 
-namespace {
+}  // extern "C"
+
+namespace qattn {
 // The context's RoPE table covering `positions` positions for `theta` (model.ts:76-81: angle =
 // pos * theta^(-i/64) in f64, cos / sin rounded to f32), rebuilt only when it must grow or theta
 // changes.  A rebuild uploads synchronously; every other call only reads it.
@@ -768,7 +770,9 @@ int32_t longest(const int32_t* cu, int32_t nseq) {
   for (int32_t s = 0; s < nseq; ++s) m = std::max(m, cu[s + 1] - cu[s]);
   return m;
 }
-}  // namespace
+}  // namespace qattn
+
+extern "C" {
 
 int qattn_qk_norm_rope(qattn_ctx* ctx, void* x, int64_t row_stride, int64_t col0, int32_t heads,
                        const int32_t* cu_seqlens, int32_t nseq, const float* weight, double eps,

@@ -60,4 +60,8 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // Host cu_seqlens: nseq in [1, QATTN_MAX_SEQS], cu[0] = 0, non-decreasing.
 int validate_cu(qattn_ctx* ctx, const int32_t* cu, int32_t nseq);
 
+// The context's RoPE table of at least `positions` positions, and the longest sequence of cu (api.hip).
+int rope_table(qattn_ctx* ctx, int32_t positions, double theta, const float2** out);
+int32_t longest(const int32_t* cu, int32_t nseq);
+
 }  // namespace qattn

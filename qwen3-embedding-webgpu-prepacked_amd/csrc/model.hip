@@ -42,6 +42,7 @@ struct qattn_model_plan {
   int32_t max_tokens = 0, max_seqs = 0;
   int32_t* ids = nullptr;      // device int32 [max_tokens]
   void* x = nullptr;           // residual stream     [T][1024]
+  void* x2 = nullptr;          // its other copy      [min(T, kFusedTokens)][1024] (fused small forward)
   void* normalized = nullptr;  // norm output          [T][1024]
   void* qkv = nullptr;         // qkvRaw               [T][4096]
   void* q = nullptr;           // roped Q              [T][2048]
@@ -174,7 +175,7 @@ void free_plan(qattn_model_plan* p) {
   qattn_ctx* ctx = p->model->ctx;
   DeviceGuard g(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
-  void* bufs[] = {p->ids, p->x, p->normalized, p->qkv, p->q, p->k, p->attn, p->delta, p->ffn};
+  void* bufs[] = {p->ids, p->x, p->x2, p->normalized, p->qkv, p->q, p->k, p->attn, p->delta, p->ffn};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   delete p;
@@ -205,6 +206,83 @@ struct Recorder {
   }
 };
 
+// The layers and the pool of a batch of at most kFusedTokens tokens, whose embedding rows are in p->x:
+// the QKV and gate/up projections normalise their own rows (each norm's time falls in its
+// consumer's stage) and QKV applies the QK norm and RoPE, so a layer is five launches instead of eight.
+// Same arithmetic, row for row, as the separate launches of a larger batch.
+int enqueue_fused(qattn_model_plan* p, const int32_t* cu, int32_t nseq, float* out, int64_t out_row_stride,
+                  hipStream_t stream, Recorder* rec) {
+  const qattn_model* m = p->model;
+  qattn_ctx* ctx = m->ctx;
+  const qattn_model_desc& d = m->desc;
+  const int32_t T = cu[nseq];
+  const qattn_stream_t s = reinterpret_cast<qattn_stream_t>(stream);
+  const auto stage = [&](int i) {
+    if (rec) rec->begin(i);
+  };
+  const auto done = [&]() {
+    if (rec) rec->end();
+  };
+  const float2* table = nullptr;
+  int rc = rope_table(ctx, longest(cu, nseq), d.rope_theta, &table);
+  if (rc) return rc;
+  half_t *x = static_cast<half_t*>(p->x), *x_next = static_cast<half_t*>(p->x2);
+  half_t* const delta = static_cast<half_t*>(p->delta);
+  FusedQkv heads{static_cast<half_t*>(p->q), static_cast<half_t*>(p->k), static_cast<half_t*>(p->qkv), nullptr, nullptr,
+                 table, (float)d.eps, nseq, {}};
+  std::copy(cu, cu + nseq + 1, heads.cu);
+  for (int32_t l = 0; l < d.n_layers; ++l) {
+    const qattn_layer_weights& w = m->layers[l];
+    stage(QATTN_STAGE_QKV);
+    heads.weight_q = w.attn_q_norm;
+    heads.weight_k = w.attn_k_norm;
+    HIP_TRY(ctx, launch_q4_norm_qkv({x, l ? delta : nullptr, x_next, w.attn_norm, (float)d.eps, T},
+                                    static_cast<const uint8_t*>(w.attn_qkv), (uint32_t)w.attn_qkv_bytes, heads, stream));
+    if (l) std::swap(x, x_next);
+    done();
+    stage(QATTN_STAGE_ROPE_ATTENTION);
+    rc = qattn_run_encode(p->run, s);
+    if (rc) return rc;
+    done();
+    stage(QATTN_STAGE_ATTENTION_OUTPUT);
+    rc = qattn_q4_matmul(ctx, p->attn, kQWidth, T, kQWidth, w.attn_output, w.attn_output_bytes, kHidden, delta, kHidden, s);
+    if (rc) return rc;
+    done();
+    stage(QATTN_STAGE_POST_ATTENTION_NORM);
+    done();
+    stage(QATTN_STAGE_FFN_UP_GATE);
+    HIP_TRY(ctx, launch_q4_norm_swiglu({x, delta, x_next, w.ffn_norm, (float)d.eps, T},
+                                       static_cast<const uint8_t*>(w.ffn_gate_up), (uint32_t)w.ffn_gate_up_bytes, kInter,
+                                       static_cast<half_t*>(p->ffn), kInter, stream));
+    std::swap(x, x_next);
+    done();
+    stage(QATTN_STAGE_SWIGLU);
+    done();
+    stage(QATTN_STAGE_FFN_DOWN);
+    rc = qattn_q4_matmul(ctx, p->ffn, kInter, T, kInter, w.ffn_down, w.ffn_down_bytes, kHidden, delta, kHidden, s);
+    if (rc) return rc;
+    done();
+    stage(QATTN_STAGE_POST_FFN_NORM);
+    if (l + 1 == d.n_layers)
+      rc = qattn_rmsnorm(ctx, x, kHidden, delta, kHidden, d.output_norm, p->normalized, kHidden, T, kHidden, d.eps, s);
+    if (rc) return rc;
+    done();
+  }
+  stage(QATTN_STAGE_POOL);
+  rc = qattn_pool_last_l2(ctx, p->normalized, kHidden, kHidden, cu, nseq, out, out_row_stride, s);
+  done();
+  return rc;
+}
+
+// The batches enqueue_fused takes.  Weights past 32-bit offsets go to the separate entry points, which
+// refuse them.
+bool fused_batch(const qattn_model* m, int64_t T, int32_t nseq) {
+  return T > 0 && T <= kFusedTokens && nseq <= kFusedSeqs &&
+         std::all_of(m->layers.begin(), m->layers.end(), [](const qattn_layer_weights& w) {
+           return w.attn_qkv_bytes <= 0x7FFFFFFFll && w.ffn_gate_up_bytes <= 0x7FFFFFFFll;
+         });
+}
+
 // Everything after the checks: enqueues one batch of T tokens.
 int enqueue(qattn_model_plan* p, const int32_t* cu, int32_t nseq, float* out, int64_t out_row_stride,
             hipStream_t stream, Recorder* rec) {
@@ -227,6 +305,10 @@ int enqueue(qattn_model_plan* p, const int32_t* cu, int32_t nseq, float* out, in
   } while (0)
   begin(QATTN_STAGE_EMBEDDING_NORM);
   STAGE_TRY(qattn_embed_q6k(ctx, p->ids, T, d.token_embd, d.token_embd_bytes, kHidden, p->x, kHidden, s));
+  if (fused_batch(m, T, nseq)) {
+    end();
+    return enqueue_fused(p, cu, nseq, out, out_row_stride, stream, rec);
+  }
   STAGE_TRY(qattn_rmsnorm(ctx, p->x, kHidden, nullptr, 0, m->layers[0].attn_norm, p->normalized, kHidden, T, kHidden,
                           d.eps, s));
   end();
@@ -327,6 +409,7 @@ int qattn_model_plan_create(qattn_model* model, int32_t max_tokens, int32_t max_
       void** ptr;
       size_t bytes;
     } bufs[] = {{reinterpret_cast<void**>(&p->ids), T * 4},   {&p->x, T * kHidden * 2},
+                {&p->x2, std::min<size_t>(T, kFusedTokens) * kHidden * 2},
                 {&p->normalized, T * kHidden * 2},             {&p->qkv, T * kQkvWidth * 2},
                 {&p->q, T * kQWidth * 2},                      {&p->k, T * kKWidth * 2},
                 {&p->attn, T * kQWidth * 2},                   {&p->delta, T * kHidden * 2},

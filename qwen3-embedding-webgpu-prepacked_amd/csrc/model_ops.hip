@@ -12,7 +12,7 @@ namespace qattn {
 
 namespace {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef half8 h8;
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 
 // ---- Q6_K token embedding (EmbeddingLookupKernel, ops.ts:381-423) ------------------------------
@@ -52,57 +52,7 @@ __global__ __launch_bounds__(256) void embed_q6k_kernel(const int32_t* ids, int6
   *reinterpret_cast<h8*>(out + t * out_stride + c0) = v;
 }
 
-// ---- residual add + RMSNorm (RmsNormKernel, ops.ts:21-72) -------------------------------------
-// One wavefront per row; lane l owns columns 8l + 512j.  With a residual: v = f32(x) + f32(r),
-// x <- f16(v) (the residual stream is updated in place, ops.ts:41), and the sum of squares takes
-// the unrounded v (ops.ts:42); without: v = f32(x).  normalized = f16(f32(x) * inv * w) with the
-// stored (rounded) x and inv = 1 / sqrt(sum / width + eps) (ops.ts:52-55).  residual_at(c) gives
-// the residual's 8 values at columns c..c+7.
-template <bool RESIDUAL, typename ResidualAt>
-__device__ inline void rmsnorm_row(half_t* xr, ResidualAt residual_at, const float* weight, half_t* out_row,
-                                   int width, float eps, int lane) {
-  constexpr int kMaxChunks = kRmsMaxWidth / 512;
-  h8 xs[kMaxChunks];
-  float ss = 0.f;
-#pragma unroll
-  for (int j = 0; j < kMaxChunks; ++j) {
-    const int c = 8 * lane + 512 * j;
-    if (c < width) {
-      h8 a = *reinterpret_cast<const h8*>(xr + c);
-      if (RESIDUAL) {
-        const h8 b = residual_at(c);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float s = (float)a[e] + (float)b[e];
-          ss += s * s;
-          a[e] = (_Float16)s;
-        }
-        *reinterpret_cast<h8*>(xr + c) = a;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) ss += (float)a[e] * (float)a[e];
-      }
-      xs[j] = a;
-    }
-  }
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
-  const float inv = 1.f / sqrtf(ss / (float)width + eps);
-#pragma unroll
-  for (int j = 0; j < kMaxChunks; ++j) {
-    const int c = 8 * lane + 512 * j;
-    if (c < width) {
-      const float4 w0 = *reinterpret_cast<const float4*>(weight + c);
-      const float4 w1 = *reinterpret_cast<const float4*>(weight + c + 4);
-      const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-      h8 o;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = (_Float16)((float)xs[j][e] * inv * w[e]);
-      *reinterpret_cast<h8*>(out_row + c) = o;
-    }
-  }
-}
-
+// ---- residual add + RMSNorm (RmsNormKernel, ops.ts:21-72): rmsnorm_row (model_ops.h), a wavefront per row.
 __global__ __launch_bounds__(256) void rmsnorm_kernel(half_t* x, const half_t* residual, const float* weight,
                                                       half_t* out, int64_t rows, int width, int64_t x_stride,
                                                       int64_t r_stride, int64_t out_stride, float eps) {
@@ -110,12 +60,13 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(half_t* x, const half_t* r
   if (row >= rows) return;
   const int lane = threadIdx.x & 63;
   half_t* xr = x + row * x_stride;
+  half_t* const out_row = out + row * out_stride;
+  const auto put = [&](int c, h8 v) { *reinterpret_cast<h8*>(out_row + c) = v; };
   if (residual) {
     const half_t* rr = residual + row * r_stride;
-    rmsnorm_row<true>(xr, [&](int c) { return *reinterpret_cast<const h8*>(rr + c); }, weight, out + row * out_stride,
-                      width, eps, lane);
+    rmsnorm_row(xr, rr, xr, weight, put, width, eps, lane);
   } else {
-    rmsnorm_row<false>(xr, [](int) { return h8{}; }, weight, out + row * out_stride, width, eps, lane);
+    rmsnorm_row(xr, nullptr, nullptr, weight, put, width, eps, lane);
   }
 }
 

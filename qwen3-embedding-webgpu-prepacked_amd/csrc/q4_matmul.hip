@@ -28,6 +28,7 @@
 
 
 #include "model_ops.h"
+#include "qk_rope.h"
 
 namespace qattn {
 
@@ -754,6 +755,176 @@ void launch_q4_small(const _Float16* x, int64_t ldx, int M, int K, const uint8_t
     else Q4_SMALL(8, 2);
   }
 #undef Q4_SMALL
+}
+
+// ---- the small forward's fused projections: q4_small_kernel for K = 1024 whose workgroups normalise
+// their own rows and, for QKV, apply the QK norm and RoPE to the head they hold.
+// A workgroup's wavefronts first load their weight records, then RMSNorm the block's rows into LDS (a
+// wavefront per row, repeated by every workgroup of the row block; workgroup 0 also writes the
+// residual sum, to another buffer, since the others still read x), then run the chain as
+// q4_small_kernel does.  QKV: 16 wavefronts hold the 128 columns of one head for 16 rows; the head goes
+// through LDS to the 16-lane layout of rope_vector.
+// What bounds the small forward is its launches: each costs 3 us or more whatever it does, and this
+// takes three of eight out of every layer.  Measured (us, 28 layers, before -> after): 1 token 1,122 ->
+// 875, 15 tokens 1,200 -> 1,070, 32 tokens 1,264 -> 1,175.  The rows normalised in every workgroup are
+// VALU work that grows with the tokens: at 33 to 64 the separate launches are as fast (1,378 against
+// 1,385 at 50), hence kFusedTokens.
+template <bool QKV, int MB>
+__global__ __launch_bounds__(QKV ? 1024 : 512) void q4_fused_kernel(FusedNorm n, const uint8_t* w, uint32_t w_bytes,
+                                                                     int N, _Float16* y, int64_t ldy, int blocks_m,
+                                                                     FusedQkv out) {
+  constexpr int kBlocks = 32, P = QKV ? 4 : 8, NKB = kBlocks / P, G = QKV ? 4 : 1, W = P * G, kRows = 16 * MB;
+  constexpr int kRaw = (NKB * 640 + 1023) / 1024;
+  __shared__ __attribute__((aligned(1024))) char raw[W][kRaw * 1024];
+  __shared__ __attribute__((aligned(1024))) char rows[kRows][2048];  // 16-byte chunk c of row r at c ^ (r & 15)
+  __shared__ f4 hand[G][2 * MB][64];
+  const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = wv / P, p = wv % P;
+  const int m0 = (int)(blockIdx.x % (unsigned)blocks_m) * kRows, nblk = (int)(blockIdx.x / (unsigned)blocks_m);
+
+  const int c0 = QKV ? 128 * nblk + 32 * g : 16 * nblk;
+  const uint32_t rec0 = ((uint32_t)(c0 >> 5) * (kBlocks * 32u) + (uint32_t)(c0 & 31)) * kQ4Record;
+  const uint32_t rec1 = rec0 + (QKV ? 16u : (uint32_t)(N >> 6) * (kBlocks * 32u)) * kQ4Record;
+  const auto wrs = q4_rsrc(w, w_bytes);
+  u4 piece[kRaw];
+#pragma unroll
+  for (int j = 0; j < kRaw; ++j) {
+    const int unit = 64 * j + lane, kb = unit / 40, r = unit % 40;
+    const uint32_t off = (r < 20 ? rec0 + 16u * r : rec1 + 16u * (r - 20)) + (uint32_t)(NKB * p + kb) * 640u;
+    piece[j] = q4_load16(wrs, kb < NKB ? off : 0x80000000u);
+  }
+#pragma unroll
+  for (int i = 0; i < kRows / W; ++i) {
+    const int r = W * i + wv, m = m0 + r;
+    const auto put = [&](int c, half8 v) { *reinterpret_cast<half8*>(rows[r] + (((c >> 3) ^ (r & 15)) << 4)) = v; };
+    if (m < n.tokens) {
+      const half_t* const xr = n.x + (size_t)m * 1024;
+      if (n.residual)
+        rmsnorm_row(xr, n.residual + (size_t)m * 1024, nblk == 0 ? n.x_out + (size_t)m * 1024 : nullptr, n.weight, put,
+                    1024, n.eps, lane);
+      else
+        rmsnorm_row(xr, nullptr, nullptr, n.weight, put, 1024, n.eps, lane);
+    } else {
+      put(8 * lane, half8{});
+      put(8 * lane + 512, half8{});
+    }
+  }
+  const uint32_t mask = kq < 2 ? 0x0F0F0F0Fu : 0xF0F0F0F0u;
+  const _Float16 mulc = (_Float16)(kq < 2 ? 1.0f : 0.0625f), addc = (_Float16)(kq < 2 ? -1032.0f : -72.0f);
+  const h2 mul = {mulc, mulc}, add = {addc, addc};
+#pragma unroll
+  for (int j = 0; j < kRaw; ++j) *reinterpret_cast<u4*>(raw[wv] + 1024 * j + 16 * lane) = piece[j];
+  h8 b[NKB][2];
+  const char* const mine = raw[wv] + l16 * kQ4Record + 8 * (kq & 1) + 4;
+  const char* const scales = raw[wv] + (l16 + 16 * (kq & 1)) * kQ4Record;
+#pragma unroll
+  for (int i = 0; i < NKB; ++i) {
+    const u2 sc = spread_rows(*reinterpret_cast<const uint32_t*>(scales + 640 * i));
+    const uint32_t* const q0 = reinterpret_cast<const uint32_t*>(mine + 640 * i);
+    const uint32_t* const q1 = reinterpret_cast<const uint32_t*>(mine + 640 * i + 320);
+    b[i][0] = dequant_frag(u2{q0[0], q0[1]}, mask, mul, add, sc[0]);
+    b[i][1] = dequant_frag(u2{q1[0], q1[1]}, mask, mul, add, sc[1]);
+  }
+  __syncthreads();
+  h8 a[NKB][MB];
+#pragma unroll
+  for (int i = 0; i < NKB; ++i)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+      a[i][mb] = *reinterpret_cast<const h8*>(rows[16 * mb + l16] + (((4 * (NKB * p + i) + kq) ^ l16) << 4));
+  f4 acc[MB][2];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) acc[mb][0] = acc[mb][1] = f4{};
+  for (int t = 0; t < P; ++t) {
+    if (t == p) {
+      if (t > 0)
+#pragma unroll
+        for (int i = 0; i < 2 * MB; ++i) acc[i >> 1][i & 1] = hand[g][i][lane];
+#pragma unroll
+      for (int i = 0; i < NKB; ++i)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = q4_mfma16(b[i][nb], a[i][mb], acc[mb][nb]);
+      if (t < P - 1)
+#pragma unroll
+        for (int i = 0; i < 2 * MB; ++i) hand[g][i][lane] = acc[i >> 1][i & 1];
+    }
+    if (t < P - 1) __syncthreads();
+  }
+  if constexpr (!QKV) {
+    if (p != P - 1) return;
+    const int n_inter = N >> 1, f = c0 + 4 * kq;
+    const auto yrs = q4_rsrc(y, (uint32_t)n.tokens * (uint32_t)ldy * 2u);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const int m = m0 + 16 * mb + l16;
+      _Float16 v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = swiglu_value((_Float16)acc[mb][0][e], (_Float16)acc[mb][1][e]);
+      q4_store8(u2{q4_pack(v[0], v[1]), q4_pack(v[2], v[3])}, yrs,
+                m < n.tokens && f < n_inter ? ((uint32_t)m * (uint32_t)ldy + (uint32_t)f) * 2u : 0x80000000u);
+    }
+  } else {
+    // The head's 16 rows of 128 columns, chunk c of row r at c ^ r, over the weight records (read by
+    // their own wavefronts before the first barrier).
+    char* const tile = raw[0];
+    if (p == P - 1) {
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) {
+        const f4& v = acc[0][nb];
+        *reinterpret_cast<u2*>(tile + l16 * 256 + (((4 * g + 2 * nb + (kq >> 1)) ^ l16) << 4) + 8 * (kq & 1)) =
+            u2{q4_pack((_Float16)v[0], (_Float16)v[1]), q4_pack((_Float16)v[2], (_Float16)v[3])};
+      }
+    }
+    __syncthreads();
+    if (wv >= 4) return;
+    // Wavefront wv: rows 4 wv .. + 3, lane (row 4 wv + lane / 16, j = lane % 16): columns 8 j .. + 7.
+    const int row = 4 * wv + kq, t = m0 + row;
+    const rope_h8 x = *reinterpret_cast<const rope_h8*>(tile + row * 256 + ((l16 ^ row) << 4));
+    if (nblk >= 24) {
+      if (t < n.tokens)
+        *reinterpret_cast<rope_h8*>(out.qkv + (size_t)t * 4096 + 3072 + (nblk - 24) * 128 + 8 * l16) = x;
+      return;
+    }
+    // Sequence of each token: the number of sequences that end at or before it.
+    const int end = lane < out.nseq ? out.cu[lane + 1] : 0x7fffffff;
+    int s = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = __popcll(__ballot(end <= m0 + 4 * wv + i));
+      s = kq == i ? c : s;
+    }
+    const int pos = t < n.tokens ? t - out.cu[s] : 0;
+    const float* const gains = nblk < 16 ? out.weight_q : out.weight_k;
+    const float4 g0 = reinterpret_cast<const float4*>(gains)[2 * l16], g1 = reinterpret_cast<const float4*>(gains)[2 * l16 + 1];
+    const float4* const cs = reinterpret_cast<const float4*>(out.rope + (int64_t)pos * 64 + 8 * (l16 & 7));
+    const float4 c4[4] = {cs[0], cs[1], cs[2], cs[3]};
+    const rope_h8 r = rope_vector(x, g0, g1, c4, l16, out.eps);
+    half_t* const dst = nblk < 16 ? out.q + (size_t)t * 2048 + nblk * 128 : out.k + (size_t)t * 1024 + (nblk - 16) * 128;
+    if (t < n.tokens) *reinterpret_cast<rope_h8*>(dst + 8 * l16) = r;
+  }
+}
+
+hipError_t launch_q4_norm_qkv(const FusedNorm& n, const uint8_t* w, uint32_t w_bytes, const FusedQkv& out,
+                              hipStream_t stream) {
+  const int blocks_m = (n.tokens + 15) / 16;
+  hipLaunchKernelGGL((q4_fused_kernel<true, 1>), dim3((unsigned)(32 * blocks_m)), dim3(1024), 0, stream, n, w, w_bytes,
+                     4096, nullptr, (int64_t)0, blocks_m, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_q4_norm_swiglu(const FusedNorm& n, const uint8_t* w, uint32_t w_bytes, int n_inter, half_t* y,
+                                 int64_t ldy, hipStream_t stream) {
+  const int mb = n.tokens <= 16 ? 1 : 2, blocks_m = (n.tokens + 16 * mb - 1) / (16 * mb);
+  const dim3 grid((unsigned)(n_inter / 16 * blocks_m));
+  if (mb == 1)
+    hipLaunchKernelGGL((q4_fused_kernel<false, 1>), grid, dim3(512), 0, stream, n, w, w_bytes, 2 * n_inter, y, ldy,
+                       blocks_m, FusedQkv{});
+  else
+    hipLaunchKernelGGL((q4_fused_kernel<false, 2>), grid, dim3(512), 0, stream, n, w, w_bytes, 2 * n_inter, y, ldy,
+                       blocks_m, FusedQkv{});
+  return hipGetLastError();
 }
 
 // ---- K above 1024, at most kQ4DirectBlocks 32 x 32 output blocks beyond q4_small_kernel's: one

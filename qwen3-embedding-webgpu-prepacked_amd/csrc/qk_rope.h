@@ -8,6 +8,38 @@ namespace qattn {
 
 typedef _Float16 half_t;
 
+typedef half_t rope_h8 __attribute__((ext_vector_type(8)));
+// QK RMSNorm + RoPE of one 128-wide head vector held by 16 lanes (lane j: elements 8j..8j+7) with gains
+// g0, g1 and c4 = (cos, sin) of slots 8 (j & 7) .. +7 (ops.ts:125-147, f32).  The sum of squares is
+// reduced over the 16 lanes by xor-shuffles in a fixed order; the rotate-half partner of element d
+// (d +- 64) sits in lane j ^ 8 at the same slot.  The one formula of qk_norm_rope_kernel and of the
+// fused small projection, so the two agree bit for bit.
+__device__ inline rope_h8 rope_vector(rope_h8 x, float4 g0, float4 g1, const float4 (&c4)[4], int j, float eps) {
+  float v[8], ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    v[e] = (float)x[e];
+    ss = fmaf(v[e], v[e], ss);
+  }
+#pragma unroll
+  for (int m = 8; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 16);
+  const float inv = __frsqrt_rn(fmaf(ss, 1.0f / 128.0f, eps));
+  const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+  float n[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) n[e] = v[e] * inv * g[e];
+  rope_h8 r;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float4 c = c4[e >> 1];  // (cos, sin) of slots e & ~1 and e | 1
+    const float partner = __shfl_xor(n[e], 8, 16);
+    float o = fmaf(j < 8 ? -partner : partner, e & 1 ? c.w : c.y, n[e] * (e & 1 ? c.z : c.x));
+    asm volatile("" : "+v"(o));  // rounded to fp32, then to fp16, in every caller
+    r[e] = (half_t)o;
+  }
+  return r;
+}
+
 constexpr int kRopeSeqs = 64;
 constexpr int kRopeMaxHeads = 32;
 struct RopeArgs {

@@ -58,7 +58,7 @@ __global__ void fill_normal_kernel(half_t* dst, int64_t rows, int64_t row_elems,
 // offsets come by value, the token's sequence found by one ballot over them.
 template <int ITERS>
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(RopeArgs a) {
-  typedef half_t h8v __attribute__((ext_vector_type(8)));
+  typedef rope_h8 h8v;
   const int lane = threadIdx.x & 63, grp = lane >> 4, j = lane & 15;
   const int t = a.cu[0] + (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (t >= a.cu[a.nseq]) return;
@@ -92,30 +92,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(RopeArgs a) {
   for (int it = 0; it < ITERS; ++it) {
     const int h = 4 * it + grp;
     const bool isq = h < a.split;
-    float v[8], ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      v[e] = (float)x[it][e];
-      ss = fmaf(v[e], v[e], ss);
-    }
-#pragma unroll
-    for (int m = 8; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 16);
-    const float inv = __frsqrt_rn(ss / 128.0f + a.eps);
-    float n[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float4 g = isq ? wq[e >> 2] : wk[e >> 2];
-      n[e] = v[e] * inv * ((e & 3) == 0 ? g.x : (e & 3) == 1 ? g.y : (e & 3) == 2 ? g.z : g.w);
-    }
-    h8v r;
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      const float4 c = c4[e >> 1];  // (cos, sin) of slots e and e+1
-      const float p0 = __shfl_xor(n[e], 8, 16), p1 = __shfl_xor(n[e + 1], 8, 16);
-      const float rot0 = j < 8 ? -p0 : p0, rot1 = j < 8 ? -p1 : p1;
-      r[e] = (half_t)(n[e] * c.x + rot0 * c.y);
-      r[e + 1] = (half_t)(n[e + 1] * c.z + rot1 * c.w);
-    }
+    const h8v r = rope_vector(x[it], isq ? wq[0] : wk[0], isq ? wq[1] : wk[1], c4, j, a.eps);
     half_t* dst = isq ? a.out_q + (int64_t)t * a.out_stride_q + h * 128
                       : a.out_k + (int64_t)t * a.out_stride_k + (h - a.split) * 128;
     *reinterpret_cast<h8v*>(dst + 8 * j) = r;

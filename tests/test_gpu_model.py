@@ -196,6 +196,26 @@ def test_model_rows_do_not_depend_on_the_batch(ctx, weights):
         m.free()
 
 
+@pytest.mark.parametrize("lengths", [[1], [15], [16], [17, 0, 3], [7, 1, 9, 14], [32], [33]])
+def test_fused_small_forward_equals_the_packed_forward(ctx, weights, lengths):
+    """Batches of up to 32 tokens take projections that normalise their own rows (and rotate Q and K);
+    the same requests packed with others take the separate launches: the same bits."""
+    m = DeviceModel(ctx, weights, flags=1)
+    rng = np.random.default_rng(sum(lengths))
+    ids = rng.integers(0, weights["vocab"], sum(lengths)).astype(np.int32)
+    more = rng.integers(0, weights["vocab"], 70).astype(np.int32)
+    cu = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    try:
+        small = _run(ctx, m, ids, cu, max_tokens=200, max_seqs=8)
+        packed = _run(ctx, m, np.concatenate([ids, more]), np.append(cu, cu[-1] + 70).astype(np.int32), max_tokens=200,
+                      max_seqs=8)
+        keep = [i for i, n in enumerate(lengths) if n]
+        assert np.array_equal(small[keep].view(np.uint32), packed[:-1][keep].view(np.uint32))
+        _check_embeddings(small[keep], mr.forward(weights, ids, cu)[keep])
+    finally:
+        m.free()
+
+
 def test_model_plan_reuse_and_rejects(ctx, qattn, weights, dmodel):
     rng = np.random.default_rng(9)
     plan = dmodel.model.plan(400, 4)

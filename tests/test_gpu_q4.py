@@ -231,3 +231,19 @@ def test_q4_tiled_launches_equal_small_launches_bit_for_bit(ctx, m, k, n, swiglu
     for a in starts:
         small = run(x[a:a + 32])[:, :cols].view(np.uint16)
         assert np.array_equal(whole[a:a + 32], small), (a, np.argwhere(whole[a:a + 32] != small)[:4])
+
+
+@pytest.mark.parametrize("m,k,n", [(15, 1024, 4096), (50, 2048, 1000), (300, 3072, 1024), (1419, 1024, 4096),
+                                   (2100, 2048, 1024)])
+def test_q4_weights_need_only_4_byte_alignment(ctx, m, k, n):
+    rng = np.random.default_rng(m + k)
+    packed = random_compact(rng, n, k)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    bx, bw = ctx.upload(x.view(np.uint16)), ctx.upload(np.concatenate([np.zeros(4, np.uint8), packed]))
+    by = ctx.alloc(m * n * 2)
+    ctx.q4_matmul(bx.ptr, m, k, bw.ptr + 4, packed.size, n, by.ptr)
+    ctx.synchronize()
+    y = by.read(np.uint16, (m, n))
+    for b in (bx, bw, by):
+        b.free()
+    assert np.array_equal(y, run_q4(ctx, x, packed, k, n).view(np.uint16))
