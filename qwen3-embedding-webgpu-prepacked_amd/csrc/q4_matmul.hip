@@ -621,7 +621,7 @@ void launch_q4_mid(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* 
                      w, w_bytes, N, y, ldy, q4_chunk_blocks(K), tiles_n, tiles, per_xcd);
 }
 
-// ---- the smallest launches: one workgroup per 16 MB x 32 block of output (SWIGLU: 16 features),
+// ---- the smallest launches: one workgroup per 16 MB x 16 NB block of output (SWIGLU: 16 features),
 // its wavefronts sharing K.  Wavefront p of a chain loads and dequantises K blocks NKB p .. + NKB - 1,
 // all at once; then the chain runs through the wavefronts in turn, the accumulators passing from one
 // to the next through LDS, so the sums are the same as in one wavefront.  H = 2 (K above 1024): both
@@ -631,12 +631,12 @@ void launch_q4_mid(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* 
 // come in as they lie in memory (three 1 KiB loads per four blocks, not twelve of scattered 4- and
 // 8-byte pieces, whose address work alone took 2 us per CU) and are taken apart in LDS.
 // Measured (us, before -> after): 15 x 1024 -> 4096 5.9 -> 4.5, 15 rows gate/up 6.6 -> 4.6,
-// 50 x 2048 -> 1024 7.5 -> 5.4, 50 x 3072 -> 1024 10.3 -> 6.7.
-template <bool SWIGLU, int MB, int NKB, int H>
+// 50 x 2048 -> 1024 7.5 -> 4.6, 50 x 3072 -> 1024 10.3 -> 6.0.
+template <bool SWIGLU, int MB, int NB, int NKB, int H>
 __global__ __launch_bounds__(1024) void q4_small_kernel(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w,
                                                         uint32_t w_bytes, int N, _Float16* y, int64_t ldy,
                                                         int chunk_blocks, int P, int blocks_m) {
-  __shared__ f4 hand[H][2 * MB][64];
+  __shared__ f4 hand[H][NB * MB][64];
   const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = H == 2 && wv >= P ? 1 : 0, p = wv - h * P;
@@ -646,7 +646,7 @@ __global__ __launch_bounds__(1024) void q4_small_kernel(const _Float16* x, int64
 
   const uint32_t x_bytes = (uint32_t)M * (uint32_t)ldx * 2u;
   const uint32_t x_off = (uint32_t)(m0 + l16) * (uint32_t)ldx * 2u + 16u * kq;
-  const int c0 = SWIGLU ? 16 * nblk : 32 * nblk;
+  const int c0 = SWIGLU ? 16 * nblk : 16 * NB * nblk;
   const uint32_t tstride = (uint32_t)kblocks * 32u * kQ4Record;
   const uint32_t rec0 = (uint32_t)(c0 >> 5) * tstride + (uint32_t)(c0 & 31) * kQ4Record;
   const uint32_t rec1 = SWIGLU ? rec0 + (uint32_t)(N >> 6) * tstride : rec0 + 16u * kQ4Record;
@@ -654,15 +654,16 @@ __global__ __launch_bounds__(1024) void q4_small_kernel(const _Float16* x, int64
   const _Float16 mulc = (_Float16)(kq < 2 ? 1.0f : 0.0625f), addc = (_Float16)(kq < 2 ? -1032.0f : -72.0f);
   const h2 mul = {mulc, mulc}, add = {addc, addc};
 
-  // This wavefront's weight records (32 rows x NKB blocks of 20 bytes) go to LDS as they lie in
+  // This wavefront's weight records (16 NB rows x NKB blocks of 20 bytes) go to LDS as they lie in
   // memory, 16 bytes per lane; blocks past the chain's end are read as zeros.
-  constexpr int kRaw = (NKB * 640 + 1023) / 1024;
+  constexpr int kBytes = 320 * NB, kUnits = kBytes / 16;  // one K block's records
+  constexpr int kRaw = (NKB * kBytes + 1023) / 1024;
   __shared__ __attribute__((aligned(1024))) char raw[16][kRaw * 1024];
   const auto wrs = q4_rsrc(w, w_bytes);
   u4 piece[kRaw];
 #pragma unroll
   for (int j = 0; j < kRaw; ++j) {
-    const int unit = 64 * j + lane, kb = unit / 40, r = unit % 40;
+    const int unit = 64 * j + lane, kb = unit / kUnits, r = unit % kUnits;
     const uint32_t off = (r < 20 ? rec0 + 16u * r : rec1 + 16u * (r - 20)) + (uint32_t)(kb0 + kb) * 640u;
     piece[j] = q4_load16(wrs, kb < NKB && kb0 + kb < k_end ? off : 0x80000000u);
   }
@@ -678,41 +679,43 @@ __global__ __launch_bounds__(1024) void q4_small_kernel(const _Float16* x, int64
   }
 #pragma unroll
   for (int j = 0; j < kRaw; ++j) *reinterpret_cast<u4*>(raw[wv] + 1024 * j + 16 * lane) = piece[j];
-  h8 b[NKB][2];
+  h8 b[NKB][NB];
   const char* const mine = raw[wv] + l16 * kQ4Record + 8 * (kq & 1) + 4;
-  const char* const scales = raw[wv] + (l16 + 16 * (kq & 1)) * kQ4Record;
+  const char* const scales = raw[wv] + (l16 + (NB == 2 ? 16 * (kq & 1) : 0)) * kQ4Record;
 #pragma unroll
   for (int i = 0; i < NKB; ++i) {
-    const u2 sc = spread_rows(*reinterpret_cast<const uint32_t*>(scales + 640 * i));
-    const uint32_t* const q0 = reinterpret_cast<const uint32_t*>(mine + 640 * i);
-    const uint32_t* const q1 = reinterpret_cast<const uint32_t*>(mine + 640 * i + 320);
-    b[i][0] = dequant_frag(u2{q0[0], q0[1]}, mask, mul, add, sc[0]);
-    b[i][1] = dequant_frag(u2{q1[0], q1[1]}, mask, mul, add, sc[1]);
-  }
-  f4 acc[MB][2];
+    const uint32_t sw = *reinterpret_cast<const uint32_t*>(scales + kBytes * i);
+    const u2 sc = NB == 2 ? spread_rows(sw) : u2{sw, sw};
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) acc[mb][0] = acc[mb][1] = f4{};
+    for (int nb = 0; nb < NB; ++nb) {
+      const uint32_t* const q = reinterpret_cast<const uint32_t*>(mine + kBytes * i + 320 * nb);
+      b[i][nb] = dequant_frag(u2{q[0], q[1]}, mask, mul, add, sc[nb]);
+    }
+  }
+  f4 acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < NB * MB; ++i) acc[i / NB][i % NB] = f4{};
   for (int t = 0; t < P; ++t) {
     if (t == p) {
       if (t > 0)
 #pragma unroll
-        for (int i = 0; i < 2 * MB; ++i) acc[i >> 1][i & 1] = hand[h][i][lane];
+        for (int i = 0; i < NB * MB; ++i) acc[i / NB][i % NB] = hand[h][i][lane];
 #pragma unroll
       for (int i = 0; i < NKB; ++i)
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-          for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = q4_mfma16(b[i][nb], a[i][mb], acc[mb][nb]);
+          for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = q4_mfma16(b[i][nb], a[i][mb], acc[mb][nb]);
       if (t < P - 1 || h == 1)
 #pragma unroll
-        for (int i = 0; i < 2 * MB; ++i) hand[h][i][lane] = acc[i >> 1][i & 1];
+        for (int i = 0; i < NB * MB; ++i) hand[h][i][lane] = acc[i / NB][i % NB];
     }
     if (t < P - 1 || H == 2) __syncthreads();
   }
   if (h != 0 || p != P - 1) return;
   if constexpr (H == 2)
 #pragma unroll
-    for (int i = 0; i < 2 * MB; ++i) acc[i >> 1][i & 1] = acc[i >> 1][i & 1] + hand[1][i][lane];
+    for (int i = 0; i < NB * MB; ++i) acc[i / NB][i % NB] = acc[i / NB][i % NB] + hand[1][i][lane];
 
   const auto yrs = q4_rsrc(y, (uint32_t)M * (uint32_t)ldy * 2u);
   const int n_out = SWIGLU ? N >> 1 : N;
@@ -720,12 +723,12 @@ __global__ __launch_bounds__(1024) void q4_small_kernel(const _Float16* x, int64
   for (int mb = 0; mb < MB; ++mb) {
     const int m = m0 + 16 * mb + l16;
 #pragma unroll
-    for (int nb = 0; nb < (SWIGLU ? 1 : 2); ++nb) {
+    for (int nb = 0; nb < (SWIGLU ? 1 : NB); ++nb) {
       const int n = c0 + 16 * nb + 4 * kq;
       _Float16 v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        v[e] = SWIGLU ? swiglu_value((_Float16)acc[mb][0][e], (_Float16)acc[mb][1][e]) : (_Float16)acc[mb][nb][e];
+        v[e] = SWIGLU ? swiglu_value((_Float16)acc[mb][0][e], (_Float16)acc[mb][NB - 1][e]) : (_Float16)acc[mb][nb][e];
       const uint32_t off = m < M ? ((uint32_t)m * (uint32_t)ldy + (uint32_t)n) * 2u : 0x80000000u;
       if (c0 + 32 <= n_out || n + 4 <= n_out) {
         q4_store8(u2{q4_pack(v[0], v[1]), q4_pack(v[2], v[3])}, yrs, off);
@@ -738,20 +741,21 @@ __global__ __launch_bounds__(1024) void q4_small_kernel(const _Float16* x, int64
   }
 }
 
-template <bool SWIGLU, int MB>
+template <bool SWIGLU, int MB, int NB>
 void launch_q4_small(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
                      _Float16* y, int64_t ldy, hipStream_t stream) {
   const int n_out = SWIGLU ? N / 2 : N, cb = q4_chunk_blocks(K), halves = cb < K / 32 ? 2 : 1;
-  const int blocks_m = (M + 16 * MB - 1) / (16 * MB), cols = SWIGLU ? 16 : 32, blocks = blocks_m * ((n_out + cols - 1) / cols);
-  const int nkb = cb <= 32 ? 4 : cb <= 48 ? 6 : 8, P = (cb + nkb - 1) / nkb;
+  const int blocks_m = (M + 16 * MB - 1) / (16 * MB), cols = SWIGLU ? 16 : 16 * NB, blocks = blocks_m * ((n_out + cols - 1) / cols);
+  // K blocks per wavefront: few, so that its loads and dequantising are short, but each turn of the chain
+  // costs a barrier: at K = 2048 four turns of eight blocks beat eight of four (50 rows: 5.1 against 5.4 us).
+  const int nkb = halves == 1 ? 4 : cb <= 32 ? 8 : cb <= 48 ? 6 : 8, P = (cb + nkb - 1) / nkb;
 #define Q4_SMALL(NKB, H) \
-  hipLaunchKernelGGL((q4_small_kernel<SWIGLU, MB, NKB, H>), dim3((unsigned)blocks), dim3(64 * P * H), 0, stream, x, \
+  hipLaunchKernelGGL((q4_small_kernel<SWIGLU, MB, NB, NKB, H>), dim3((unsigned)blocks), dim3(64 * P * H), 0, stream, x, \
                      ldx, M, K, w, w_bytes, N, y, ldy, cb, P, blocks_m)
   if (halves == 1) {
     Q4_SMALL(4, 1);
   } else if constexpr (MB == 1) {
-    if (nkb == 4) Q4_SMALL(4, 2);
-    else if (nkb == 6) Q4_SMALL(6, 2);
+    if (nkb == 6) Q4_SMALL(6, 2);
     else Q4_SMALL(8, 2);
   }
 #undef Q4_SMALL
@@ -1100,8 +1104,9 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
 //     against 29.5, M = 8,000 65 against 68), else 256 x 128 tiles, whose second workgroup per CU
 //     fills the gap (N = 6144, M = 4,000: 1.5 rounds, 60 against 53).
 // K above 1024 (N = 1024, K = 2048):
-//   * q4_small_kernel while its 16-row blocks are at most one per CU (M = 100 6.2, direct 7.5;
-//     M = 150, 320 blocks, 10.4 against 7.8) and a half's blocks fit its eight wavefronts;
+//   * q4_small_kernel while its 16 x 16 blocks are at most one per CU (M = 50 4.6, 16 x 32 blocks 5.1;
+//     K = 3072 6.0 against 6.7), then while its 16 x 32 blocks are (M = 100 5.9, direct 7.5; M = 150,
+//     320 blocks, 10.4 against 7.8) and a half's blocks fit its eight wavefronts;
 //   * q4_direct_kernel up to kQ4DirectBlocks;
 //   * up to 256 tiles of 64 x 128: q4_mid_kernel (M = 1,419 13.2, 128 x 128 tiles 19.8);
 //   * then 128 x 128 tiles while at most one per CU (M = 2,400 20.3, mid 25.4, 256 x 128 27.6);
@@ -1117,9 +1122,9 @@ hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t
   if (cb == K / 32) {
     const int64_t t = tiles(256, 256);
     if (tiles(16, 32) <= 256)
-      launch_q4_small<SWIGLU, 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+      launch_q4_small<SWIGLU, 1, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if (tiles(32, 32) <= 512)
-      launch_q4_small<SWIGLU, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+      launch_q4_small<SWIGLU, 2, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if (tiles(64, 128) <= 512)
       launch_q4_mid<SWIGLU, 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if (tiles(256, 128) <= 256 || (t > 256 && 256 * rounds(t) * 100 > 115 * t))
@@ -1128,8 +1133,10 @@ hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t
       Q4_TILE(8, 4, 1);
   } else {
     const int64_t big = rounds(tiles(256, 128)), small = rounds(tiles(128, 128));
-    if (tiles(16, 32) <= 256 && cb <= 64)
-      launch_q4_small<SWIGLU, 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+    if (tiles(16, 16) <= 256 && cb <= 64 && !SWIGLU)
+      launch_q4_small<SWIGLU, 1, SWIGLU ? 2 : 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+    else if (tiles(16, 32) <= 256 && cb <= 64)
+      launch_q4_small<SWIGLU, 1, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if ((int64_t)((M + 31) / 32) * ((n_out + 31) / 32) <= kQ4DirectBlocks)
       launch_q4_direct<SWIGLU>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if (tiles(64, 128) <= 256)

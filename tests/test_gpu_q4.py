@@ -203,6 +203,8 @@ TILE_CASES = [
     (50, 1024, 4096, False), (50, 992, 1501, False), (33, 1024, 6144, True),  # 32-row blocks
     (300, 2048, 1024, False), (500, 3072, 1023, False), (150, 1056, 384, True),  # one wavefront per block
     (150, 3072, 2048, True), (33, 4160, 96, False),  # halves of 72 K blocks
+    (50, 2048, 1000, False), (64, 3072, 1023, False), (40, 4096, 9, False),  # 16 x 16 blocks
+    (65, 2048, 1000, False), (33, 4096, 1400, False),  # 16 x 32 blocks
     (65, 96, 6001, False),      # 64 x 128 tiles, one row past a tile, N odd
     (1025, 1024, 4096, False),  # 256 x 128
     (500, 160, 12300, False),   # 256 x 128, K padded to 8 blocks, N = 8 k + 4
