@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "attn_common.h"
+#include "qk_rope.h"
 
 namespace qattn {
 
@@ -52,8 +53,7 @@ __device__ inline void rmsnorm_row(const half_t* xr, const half_t* rr, half_t* x
       xs[j] = a;
     }
   }
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+  ss = wave_sum(ss);
   const float inv = 1.f / sqrtf(ss / (float)width + eps);
 #pragma unroll
   for (int j = 0; j < kMaxChunks; ++j) {

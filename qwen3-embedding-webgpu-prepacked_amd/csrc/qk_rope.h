@@ -9,9 +9,33 @@ namespace qattn {
 typedef _Float16 half_t;
 
 typedef half_t rope_h8 __attribute__((ext_vector_type(8)));
+// The value of lane l ^ N (N = 8), or one equal to it where values already repeat every 2 N lanes, as in
+// a sum over xor distances from 8 down: a rotation within the 16 lanes of a row, one VALU operation
+// where a shuffle goes through LDS (us, shuffles -> this: QK norm + RoPE of 8,000 tokens, twelve of them
+// per vector, 20.9 -> 20.1; forward of 15 tokens 1,024 -> 1,010, of 500 2,275 -> 2,241).
+template <int N>
+__device__ inline float row_rotate(float v) {
+  const int i = __float_as_int(v);
+  return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x120 + N, 0xf, 0xf, false));
+}
+// The sum over the 16 lanes of a row: xor distances 8, 4, 2, 1 in turn.
+__device__ inline float row_sum(float v) {
+  v += row_rotate<8>(v);
+  v += row_rotate<4>(v);
+  v += row_rotate<2>(v);
+  return v + row_rotate<1>(v);
+}
+// The sum over the wavefront: xor distances 32, 16, then the row's.
+__device__ inline float wave_sum(float v) {
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return row_sum(__uint_as_float(rows[0]) + __uint_as_float(rows[1]));
+}
+
 // QK RMSNorm + RoPE of one 128-wide head vector held by 16 lanes (lane j: elements 8j..8j+7) with gains
 // g0, g1 and c4 = (cos, sin) of slots 8 (j & 7) .. +7 (ops.ts:125-147, f32).  The sum of squares is
-// reduced over the 16 lanes by xor-shuffles in a fixed order; the rotate-half partner of element d
+// reduced over the 16 lanes in a fixed order; the rotate-half partner of element d
 // (d +- 64) sits in lane j ^ 8 at the same slot.  The one formula of qk_norm_rope_kernel and of the
 // fused small projection, so the two agree bit for bit.
 __device__ inline rope_h8 rope_vector(rope_h8 x, float4 g0, float4 g1, const float4 (&c4)[4], int j, float eps) {
@@ -21,8 +45,7 @@ __device__ inline rope_h8 rope_vector(rope_h8 x, float4 g0, float4 g1, const flo
     v[e] = (float)x[e];
     ss = fmaf(v[e], v[e], ss);
   }
-#pragma unroll
-  for (int m = 8; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 16);
+  ss = row_sum(ss);
   const float inv = __frsqrt_rn(fmaf(ss, 1.0f / 128.0f, eps));
   const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
   float n[8];
@@ -32,7 +55,7 @@ __device__ inline rope_h8 rope_vector(rope_h8 x, float4 g0, float4 g1, const flo
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const float4 c = c4[e >> 1];  // (cos, sin) of slots e & ~1 and e | 1
-    const float partner = __shfl_xor(n[e], 8, 16);
+    const float partner = row_rotate<8>(n[e]);
     float o = fmaf(j < 8 ? -partner : partner, e & 1 ? c.w : c.y, n[e] * (e & 1 ? c.z : c.x));
     asm volatile("" : "+v"(o));  // rounded to fp32, then to fp16, in every caller
     r[e] = (half_t)o;
