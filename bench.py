@@ -375,7 +375,7 @@ def q4_timing(reps, ms=(8000,)):
         ctx.synchronize()
         us = e0.elapsed_ms(e1) * 1000.0 / reps
         flop = 2.0 * M * N * K
-        print(json.dumps({"kernel": "q4_matmul_kernel", "shape": name, "M": M, "K": K, "N": N, "launches": reps,
+        print(json.dumps({"kernel": "qattn_q4_matmul", "shape": name, "M": M, "K": K, "N": N, "launches": reps,
                           "us_per_launch": round(us, 2), "TFLOP/s": round(flop / us / 1e6, 1),
                           "frac_of_fp16_peak": round(flop / us / 1e6 / PEAK_FP16_TFLOPS, 3)}), flush=True)
         for b in (bw, bx, by):

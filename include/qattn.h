@@ -435,7 +435,8 @@ enum qattn_model_stage {
 };
 /* qattn_model_plan_run with a HIP event pair around every stage of every layer, then a wait for
  * the stream: stage_ms[s] receives stage s's total over all layers in milliseconds
- * (Qwen3ExecutionPlan.profile, model.ts:141-182). */
+ * (Qwen3ExecutionPlan.profile, model.ts:141-182).  A batch of at most 32 tokens runs the norms and
+ * the QK norm + RoPE inside the projections that read or write them: their time is in those stages. */
 int qattn_model_plan_profile(qattn_model_plan* plan, const int32_t* ids, const int32_t* cu_seqlens,
                              int32_t nseq, float* out, int64_t out_row_stride, qattn_stream_t stream,
                              float stage_ms[QATTN_STAGE_COUNT]);

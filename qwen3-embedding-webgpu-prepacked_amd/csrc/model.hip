@@ -5,8 +5,9 @@
 //
 // The plan enqueues the reference's sequence of dispatches (model.ts:117-131) over a packed
 // varlen batch: no padding rows, RoPE positions restart per sequence, attention restricted to
-// each sequence.  Every stage is one launch of this library's gfx950 kernels; the plan keeps its
-// buffers between batches and re-plans only the attention work list.
+// each sequence.  Every stage is one launch of this library's gfx950 kernels (the smallest batches
+// merge the norms and RoPE into the projections); the plan keeps its buffers between batches and
+// re-plans only the attention work list.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
