@@ -523,13 +523,17 @@ __global__ __launch_bounds__(256 * G, 3) void q4_mid_kernel(const _Float16* x, i
   __builtin_amdgcn_sched_barrier(0);
   // Stage of K blocks kb, kb + 1 in `cur`.  The X blocks of stage + 1 have landed by its barrier,
   // which also frees `cur` for stage + 4.  Vector-memory operations newer than that stage's last
-  // X load at the barrier: two stages' X loads (4) and at least five blocks' weight loads (15).
+  // X load at the barrier, wherever the compiler puts the weight loads within a half stage:
+  //   steady state: two stages' X loads (4) and at least five blocks' weight loads (15);
+  //   kb = 0 (X loaded before W0-3 by the prologue): W0-3 12, X 4-7 4, W4-5 6 = 22;
+  //   kb = 2 (X 4, 5 loaded after W0-3): X 6-9 4, W4-7 12 = 16, the fewest;
+  //   kb = 4: X 8-11 4, W4-9 18 = 22.
   auto stage = [&](char* cur, const char* nxt, WRegs& w1, WRegs& w2, int kb) Q4_INLINE {
     read_a(fo, cur + kBlock);
     weights(fo, w1);
     load_w(w1, kb + 5);
     mma(fe);
-    q4_barrier<19>();
+    q4_barrier<16>();
     load_a(cur, kb + 8);
     read_a(fe, nxt);
     weights(fe, w2);
