@@ -8,8 +8,8 @@
 // The weight is f16(scale * (q - 8)), as the reference dequantises it; the products and sums run
 // in fp32 on the matrix cores (the reference accumulates in f16).
 //
-// Four kernels, one result: every output element is the same MFMA chain (its K blocks in turn from
-// a zero accumulator, the two halves of a K above 1024 columns added at the end), so a row does not
+// Four kernels, one result: every output element is the same MFMA chains (one per 1,024 columns of K,
+// its K blocks in turn from a zero accumulator; the chains' sums added in order), so a row does not
 // depend on the launch it is in.  v_mfma_f32_16x16x32_f16 on a K block equals two chained
 // v_mfma_f32_32x32x16_f16 on its halves bit for bit, which lets each kernel take the shape it needs.
 //   * q4_tile_kernel, large launches: 256 x 256 / 256 x 128 / 128 x 128 workgroup tiles, X by
@@ -39,14 +39,13 @@ typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
 constexpr int kQ4Record = 20;  // bytes per (row, 32-column block)
-// Every output element is the fp32 sum of at most two MFMA chains, each from a zero accumulator:
-// one over all of K up to 1024 columns, else one per half, y = f16(c0 + c1).  The split depends on
-// K alone, so a row's result does not depend on the batch, and the halves of a launch with few
-// tiles run side by side.
-// K blocks per chain (a multiple of 8 where there are two).
-__host__ __device__ constexpr int q4_chunk_blocks(int K) {
-  return K <= 1024 ? K / 32 : ((K / 32 + 1) / 2 + 7) / 8 * 8;
-}
+// Every output element is the fp32 sum, in order, of MFMA chains over chunks of kQ4Chunk K blocks
+// (1,024 columns), each chain from a zero accumulator: y = f16((c0 + c1) + c2) for K = 3072.  The
+// split depends on K alone, so a row's result does not depend on the batch, the length of a chain
+// (and with it the bound of its rounding error) does not grow with K, and the chunks of a launch
+// with few tiles run side by side.
+constexpr int kQ4Chunk = 32;
+__host__ __device__ constexpr int q4_chunks(int K) { return (K / 32 + kQ4Chunk - 1) / kQ4Chunk; }
 __device__ inline __amdgpu_buffer_rsrc_t q4_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
 }
@@ -124,8 +123,9 @@ __device__ inline void q4_barrier() {
 #define Q4_INLINE __attribute__((always_inline))
 
 // ---- large launches.
-// Workgroup tile 32 MF x 64 NWN, 2 x NWN wavefronts of 16 MF x 64 per group; G = 2 (K above 1024): two
-// such groups, one per half of K, whose chains meet through LDS at the end.
+// Workgroup tile 32 MF x 64 NWN, 2 x NWN wavefronts of 16 MF x 64 per group.  K above 1024: G = 2 or 3
+// such groups, one per chunk of K, whose chains meet through LDS at the end, or (FOLD) one group that
+// runs the chunks in turn and adds each finished chain to a second set of accumulators.
 //
 // What bounds it: LDS bandwidth (128 B per clock and CU, measured) and power.  A 128 x 64 wavefront
 // (MF = 8) reads 12 KiB of fragments per K block for 512 clocks of MFMA, so two per SIMD keep LDS
@@ -137,17 +137,17 @@ __device__ inline void q4_barrier() {
 // 68.1 us).  Not kept: weights dequantised into registers at this size (VALU power: 73 us), four
 // wavefronts of 128 x 128 (one per SIMD cannot issue the dequantisation beside its MFMAs: 65 us).
 // Measured (us, before -> after): 8000 x 1024 -> 4096 80.4 -> 65.5; 20000 x 1024 -> 6144 with SwiGLU
-// 292 -> 254; 8000 x 2048 -> 1024 44.8 -> 38.8; 8000 x 3072 -> 1024 64.9 -> 53.2.
+// 292 -> 254; 8000 x 2048 -> 1024 44.8 -> 38.8; 8000 x 3072 -> 1024, folding in 128 x 256, 66.7 -> 55.5.
 //
 // Step kb (X tile and weight tile kb in LDS; the first half's fragments in registers): half 1 reads
 // the other row fragments, dequantises weight tile kb + 1 into the free B buffer and runs the first
 // half's MFMAs; the barrier publishes that tile and X tile kb + 1 (loaded two steps ago); half 2
 // reads the next step's fragments under the other half's MFMAs.  X tile kb + 3 goes into the buffer
 // that tile kb - 1 left at the previous barrier.
-template <bool SWIGLU, int MF, int NWN, int G>
+template <bool SWIGLU, int MF, int NWN, int G, bool FOLD>
 __global__ __launch_bounds__(128 * NWN * G, 2) void q4_tile_kernel(
     const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N, _Float16* y, int64_t ldy,
-    int chunk_blocks, int tiles_n, int tiles_total, int per_xcd) {
+    int tiles_n, int tiles_total, int per_xcd) {
   constexpr int kWaves = 2 * NWN;                            // per group
   constexpr int kTileM = 32 * MF, kTileN = 64 * NWN;
   constexpr int kBytesA = kTileM * 64, kBytesB = kTileN * 64;  // one K block's tiles
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(128 * NWN * G, 2) void q4_tile_kernel(
   const int l16 = lane & 15, kq = lane >> 4;
   const int wr = 16 * MF * (wave & 1), wc = 64 * (wave >> 1);
   const int kblocks = K >> 5;
-  const int kb0 = G == 1 ? 0 : grp * chunk_blocks, kn = G == 1 ? kblocks : chunk_blocks;
+  const int kb0 = G == 1 ? 0 : grp * kQ4Chunk, kn = G == 1 ? kblocks : kQ4Chunk;
   const int k_here = min(kn, kblocks - kb0);  // blocks from k_here on are read as zeros
 
   const uint32_t x_bytes = (uint32_t)M * (uint32_t)ldx * 2u;
@@ -296,16 +296,37 @@ __global__ __launch_bounds__(128 * NWN * G, 2) void q4_tile_kernel(
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  for (int kb = 0; kb < kn; kb += 4) {  // blocks past the end add zero products
+  auto steps = [&](int kb) Q4_INLINE {  // blocks past the end add zero products
     step(sA0, sA1, sA3, sB1, b0, b1, wreg[1], wreg[3], kb);
     step(sA1, sA2, sA0, sB0, b1, b0, wreg[2], wreg[0], kb + 1);
     step(sA2, sA3, sA1, sB1, b0, b1, wreg[3], wreg[1], kb + 2);
     step(sA3, sA0, sA2, sB0, b1, b0, wreg[0], wreg[2], kb + 3);
+  };
+  if constexpr (FOLD) {
+    f4 sum[MF][4];
+    for (int c = 0; c < kn; c += kQ4Chunk) {
+      const int end = min(c + kQ4Chunk, kn);
+      for (int kb = c; kb < end; kb += 4) steps(kb);
+#pragma unroll
+      for (int mb = 0; mb < MF; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) {
+          sum[mb][nb] = c ? sum[mb][nb] + acc[mb][nb] : acc[mb][nb];
+          acc[mb][nb] = f4{};
+        }
+    }
+#pragma unroll
+    for (int mb = 0; mb < MF; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) acc[mb][nb] = sum[mb][nb];
+  } else {
+#pragma unroll 1
+    for (int kb = 0; kb < kn; kb += 4) steps(kb);
   }
   q4_barrier<0>();
 
-  // G = 2: the groups' chains meet.  Group g finishes the rows of half g of every wavefront's tile.
-  if constexpr (G == 2) {
+  // G > 1: the groups' chains meet.  Group g < 2 finishes the rows of half g of every wavefront's tile.
+  if constexpr (G > 1) {
     char* const ex = (wave == 0 ? sA0 : wave == 1 ? sA1 : wave == 2 ? sA2 : sA3) + 16 * lane;
     auto send = [&](int m8, char* p) Q4_INLINE {
 #pragma unroll
@@ -315,7 +336,7 @@ __global__ __launch_bounds__(128 * NWN * G, 2) void q4_tile_kernel(
     };
     if (grp == 0)
       send(H, ex);
-    else
+    else if (G == 2 || grp == 1)
       send(0, ex + 4096 * H);
     __syncthreads();
     auto take = [&](int m8, const char* p) Q4_INLINE {
@@ -326,17 +347,30 @@ __global__ __launch_bounds__(128 * NWN * G, 2) void q4_tile_kernel(
     };
     if (grp == 0)
       take(0, ex + 4096 * H);
-    else
+    else if (G == 2 || grp == 1)
       take(H, ex);
     __syncthreads();
+    if constexpr (G == 3) {
+      if (grp == 2) {
+        send(0, ex);
+        send(H, ex + 4096 * H);
+      }
+      __syncthreads();
+      if (grp < 2) take(0, ex + 4096 * H * grp);
+      __syncthreads();
+      if (grp == 2) return;
+    }
   }
 
   // Output through LDS, kRows rows of a wavefront at a time: 16 stores of 16 bytes per lane in whole
   // 128-byte lines instead of 128 stores of two bytes.  Lane (l16, kq) holds row 16 mb + l16, columns
   // 16 nb + 4 kq .. +3.
-  constexpr int kMine = MF / G;                       // row fragments this wavefront finishes
-  constexpr int kRows = kMine >= 4 ? 64 : 16 * kMine;  // rows per pass
+  constexpr int kMine = G > 1 ? H : MF;               // row fragments this wavefront finishes
+  constexpr int kWriters = kWaves * (G > 1 ? 2 : 1);
+  // rows per pass: at most 64, and as many as the X buffers hold for every writer
+  constexpr int kRows = 16 * kMine < 64 ? 16 * kMine : G * kBytesA / 32 / kWriters < 64 ? G * kBytesA / 32 / kWriters : 64;
   constexpr int kPer = G * kBytesA / (128 * kRows);    // wavefronts per X buffer
+  static_assert(4 * kPer >= kWriters && 16 * kMine % kRows == 0 && kRows % 16 == 0, "a stage per writer, whole fragments");
   const int slot = gwave / kPer;
   char* const stage = (slot == 0 ? sA0 : slot == 1 ? sA1 : slot == 2 ? sA2 : sA3) + 128 * kRows * (gwave % kPer);
   const auto yrs = q4_rsrc(y, (uint32_t)M * (uint32_t)ldy * 2u);
@@ -390,24 +424,25 @@ __global__ __launch_bounds__(128 * NWN * G, 2) void q4_tile_kernel(
   }
 }
 
-template <bool SWIGLU, int MF, int NWN, int G>
+template <bool SWIGLU, int MF, int NWN, int G, bool FOLD = false>
 void launch_q4_tile(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
                     _Float16* y, int64_t ldy, hipStream_t stream) {
   const int tiles_m = (M + 32 * MF - 1) / (32 * MF), tiles_n = (N + 64 * NWN - 1) / (64 * NWN);
   const int tiles = tiles_m * tiles_n, per_xcd = (tiles + 7) / 8;
-  hipLaunchKernelGGL((q4_tile_kernel<SWIGLU, MF, NWN, G>), dim3((unsigned)(8 * per_xcd)), dim3(128 * NWN * G), 0, stream,
-                     x, ldx, M, K, w, w_bytes, N, y, ldy, q4_chunk_blocks(K), tiles_n, tiles, per_xcd);
+  hipLaunchKernelGGL((q4_tile_kernel<SWIGLU, MF, NWN, G, FOLD>), dim3((unsigned)(8 * per_xcd)), dim3(128 * NWN * G), 0,
+                     stream, x, ldx, M, K, w, w_bytes, N, y, ldy, tiles_n, tiles, per_xcd);
 }
 
 // ---- medium launches.
 // 64 x 128 workgroup tiles, four wavefronts of 64 x 32 per group, each dequantising its own 32
-// columns straight into MFMA fragments; G = 2 (K above 1024): two groups, one per half of K.
+// columns straight into MFMA fragments.  K above 1024: G = 2 or 3 groups, one per chunk of K, or FOLD as
+// in q4_tile_kernel.
 // What bounds it: with about one workgroup per CU, the latency of a K block.  An LDS weight tile
 // puts dequantise -> LDS write -> barrier -> LDS read in every K block's chain (0.37 us per pair of
 // halves); here only X goes through LDS, its barrier comes once per two blocks with loads six
 // blocks ahead, and weight records are loaded four blocks ahead.  A wavefront's block is about 75
 // instructions for 8 MFMAs, so VALU and MFMA issue are level.  Measured (us, before -> after):
-// 1419 x 2048 -> 1024 22.2 -> 13.2, 1500 x 3072 -> 1024 31.6 -> 17.8, 500 x 1024 -> 4096 12.8 -> 9.4,
+// 1419 x 2048 -> 1024 22.2 -> 13.2, 1500 x 3072 -> 1024 31.2 -> 18.3, 500 x 1024 -> 4096 12.8 -> 9.4,
 // 300 x 1024 -> 6144 with SwiGLU 12.6 -> 9.2.
 // The 8 weights of a 16x16x32 B fragment from quant bytes b0..b7: mask keeps the lane's nibbles,
 // mul / add take 1024 + byte to q - 8 (1, -1032 for low nibbles; 1/16, -72 for high ones).
@@ -430,11 +465,10 @@ __device__ inline u2 spread_rows(uint32_t s) {
   return u2{r[0], r[1]};
 }
 
-template <bool SWIGLU, int G>
+template <bool SWIGLU, int G, bool FOLD>
 __global__ __launch_bounds__(256 * G, 3) void q4_mid_kernel(const _Float16* x, int64_t ldx, int M, int K,
                                                             const uint8_t* w, uint32_t w_bytes, int N, _Float16* y,
-                                                            int64_t ldy, int chunk_blocks, int tiles_n,
-                                                            int tiles_total, int per_xcd) {
+                                                            int64_t ldy, int tiles_n, int tiles_total, int per_xcd) {
   constexpr int kTileM = 64, kTileN = 128, kBlock = kTileM * 64, kStage = 2 * kBlock;
   __shared__ __attribute__((aligned(1024))) char sA0[G * kStage];
   __shared__ __attribute__((aligned(1024))) char sA1[G * kStage];
@@ -448,7 +482,7 @@ __global__ __launch_bounds__(256 * G, 3) void q4_mid_kernel(const _Float16* x, i
   const int grp = gwave >> 2, wave = gwave & 3;
   const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
   const int kblocks = K >> 5;
-  const int kb0 = G == 1 ? 0 : grp * chunk_blocks, kn = G == 1 ? kblocks : chunk_blocks;
+  const int kb0 = G == 1 ? 0 : grp * kQ4Chunk, kn = G == 1 ? kblocks : kQ4Chunk;
   const int k_here = min(kn, kblocks - kb0);  // blocks from k_here on are read as zeros
 
   const uint32_t x_bytes = (uint32_t)M * (uint32_t)ldx * 2u;
@@ -541,33 +575,59 @@ __global__ __launch_bounds__(256 * G, 3) void q4_mid_kernel(const _Float16* x, i
     mma(fo);
     __builtin_amdgcn_sched_barrier(0);
   };
-  for (int kb = 0; kb < kn; kb += 8) {  // blocks past the end add zero products
+  auto stages = [&](int kb) Q4_INLINE {  // blocks past the end add zero products
     stage(sA0, sA1, wreg[1], wreg[2], kb);
     stage(sA1, sA2, wreg[3], wreg[0], kb + 2);
     stage(sA2, sA3, wreg[1], wreg[2], kb + 4);
     stage(sA3, sA0, wreg[3], wreg[0], kb + 6);
+  };
+  if constexpr (FOLD) {
+    f4 sum[4][2];
+    for (int c = 0; c < kn; c += kQ4Chunk) {
+      const int end = min(c + kQ4Chunk, kn);
+      for (int kb = c; kb < end; kb += 8) stages(kb);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        sum[i >> 1][i & 1] = c ? sum[i >> 1][i & 1] + acc[i >> 1][i & 1] : acc[i >> 1][i & 1];
+        acc[i >> 1][i & 1] = f4{};
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i >> 1][i & 1] = sum[i >> 1][i & 1];
+  } else {
+#pragma unroll 1
+    for (int kb = 0; kb < kn; kb += 8) stages(kb);
   }
   q4_barrier<0>();
 
-  // G = 2: the groups' chains meet; group g finishes row fragments 2 g, 2 g + 1.
-  if constexpr (G == 2) {
+  // G > 1: the groups' chains meet; group g < 2 finishes row fragments 2 g, 2 g + 1.
+  if constexpr (G > 1) {
     char* const ex = (wave == 0 ? sA0 : wave == 1 ? sA1 : wave == 2 ? sA2 : sA3) + 16 * lane;
     if (grp == 0) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) *reinterpret_cast<f4*>(ex + 1024 * i) = acc[2 + (i >> 1)][i & 1];
-    } else {
+    } else if (G == 2 || grp == 1) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) *reinterpret_cast<f4*>(ex + 4096 + 1024 * i) = acc[i >> 1][i & 1];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) *reinterpret_cast<f4*>(ex + 8192 + 1024 * i) = acc[i >> 1][i & 1];
     }
     __syncthreads();
     if (grp == 0) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         acc[i >> 1][i & 1] = acc[i >> 1][i & 1] + *reinterpret_cast<const f4*>(ex + 4096 + 1024 * i);
-    } else {
+    } else if (G == 2 || grp == 1) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         acc[i >> 1][i & 1] = acc[2 + (i >> 1)][i & 1] + *reinterpret_cast<const f4*>(ex + 1024 * i);
+    }
+    if constexpr (G == 3) {
+      if (grp < 2)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc[i >> 1][i & 1] = acc[i >> 1][i & 1] + *reinterpret_cast<const f4*>(ex + 8192 + 4096 * grp + 1024 * i);
     }
     __syncthreads();
   }
@@ -577,8 +637,10 @@ __global__ __launch_bounds__(256 * G, 3) void q4_mid_kernel(const _Float16* x, i
   auto at = [&](int row, int c) Q4_INLINE {
     return (row < 32 ? sA0 : sA1) + (row & 31) * (16 * kPieces) + ((SWIGLU ? c ^ ((row >> 1) & 7) : c ^ (row & 15)) << 4);
   };
+  constexpr int kGroups = G > 1 ? 2 : 1;  // that finish and store rows
+  if (grp < kGroups)
 #pragma unroll
-  for (int i = 0; i < 4 / G; ++i) {
+  for (int i = 0; i < 4 / kGroups; ++i) {
     const int row = 32 * grp + 16 * i + l16;
     if constexpr (SWIGLU) {
       const f4 &g = acc[i][0], &t = acc[i][1];
@@ -595,9 +657,10 @@ __global__ __launch_bounds__(256 * G, 3) void q4_mid_kernel(const _Float16* x, i
     }
   }
   __syncthreads();
+  if (grp >= kGroups) return;
   const auto yrs = q4_rsrc(y, (uint32_t)M * (uint32_t)ldy * 2u);
   const int n_out = SWIGLU ? N >> 1 : N, col0 = SWIGLU ? n0 >> 1 : n0;
-  constexpr int kRowsPer = 256 * G / kPieces;  // rows per store of the workgroup
+  constexpr int kRowsPer = 256 * kGroups / kPieces;  // rows per store of the workgroup
 #pragma unroll
   for (int i = 0; i < kTileM / kRowsPer; ++i) {
     const int row = kRowsPer * i + (int)threadIdx.x / kPieces, c = threadIdx.x % kPieces;
@@ -609,7 +672,7 @@ __global__ __launch_bounds__(256 * G, 3) void q4_mid_kernel(const _Float16* x, i
   const int part = (n_out - col0) >> 3;
   if ((n_out & 7) && part < kPieces) {
 #pragma unroll 1
-    for (int i = threadIdx.x; i < kTileM * 8; i += 256 * G) {
+    for (int i = threadIdx.x; i < kTileM * 8; i += 256 * kGroups) {
       const int row = i >> 3, m = m0 + row, n = col0 + 8 * part + (i & 7);
       const _Float16 v = *reinterpret_cast<const _Float16*>(at(row, part) + 2 * (i & 7));
       q4_store_b16(v, yrs, m < M && n < n_out ? ((uint32_t)m * (uint32_t)ldy + (uint32_t)n) * 2u : 0x80000000u);
@@ -617,36 +680,36 @@ __global__ __launch_bounds__(256 * G, 3) void q4_mid_kernel(const _Float16* x, i
   }
 }
 
-template <bool SWIGLU, int G>
+template <bool SWIGLU, int G, bool FOLD = false>
 void launch_q4_mid(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
                    _Float16* y, int64_t ldy, hipStream_t stream) {
   const int tiles_m = (M + 63) / 64, tiles_n = (N + 127) / 128, tiles = tiles_m * tiles_n, per_xcd = (tiles + 7) / 8;
-  hipLaunchKernelGGL((q4_mid_kernel<SWIGLU, G>), dim3((unsigned)(8 * per_xcd)), dim3(256 * G), 0, stream, x, ldx, M, K,
-                     w, w_bytes, N, y, ldy, q4_chunk_blocks(K), tiles_n, tiles, per_xcd);
+  hipLaunchKernelGGL((q4_mid_kernel<SWIGLU, G, FOLD>), dim3((unsigned)(8 * per_xcd)), dim3(256 * G), 0, stream, x, ldx, M,
+                     K, w, w_bytes, N, y, ldy, tiles_n, tiles, per_xcd);
 }
 
 // ---- the smallest launches: one workgroup per 16 MB x 16 NB block of output (SWIGLU: 16 features),
 // its wavefronts sharing K.  Wavefront p of a chain loads and dequantises K blocks NKB p .. + NKB - 1,
 // all at once; then the chain runs through the wavefronts in turn, the accumulators passing from one
-// to the next through LDS, so the sums are the same as in one wavefront.  H = 2 (K above 1024): both
-// halves of K run side by side and are added at the end.
+// to the next through LDS, so the sums are the same as in one wavefront.  C > 1 (K above 1024): up to C
+// chunks of K run side by side and are added in order at the end.
 // What bounds it: a launch's fixed 3 us or so, one memory round trip, and P hand-overs of about 0.2 us;
 // one wavefront running the whole chain dequantised 32 blocks in sequence instead.  Weight records
 // come in as they lie in memory (three 1 KiB loads per four blocks, not twelve of scattered 4- and
 // 8-byte pieces, whose address work alone took 2 us per CU) and are taken apart in LDS.
 // Measured (us, before -> after): 15 x 1024 -> 4096 5.9 -> 4.5, 15 rows gate/up 6.6 -> 4.6,
-// 50 x 2048 -> 1024 7.5 -> 4.6, 50 x 3072 -> 1024 10.3 -> 6.0.
-template <bool SWIGLU, int MB, int NB, int NKB, int H>
-__global__ __launch_bounds__(1024) void q4_small_kernel(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w,
-                                                        uint32_t w_bytes, int N, _Float16* y, int64_t ldy,
-                                                        int chunk_blocks, int P, int blocks_m) {
-  __shared__ f4 hand[H][NB * MB][64];
+// 50 x 2048 -> 1024 7.5 -> 4.6, 50 x 3072 -> 1024 10.4 -> 6.1.
+template <bool SWIGLU, int MB, int NB, int NKB, int C>
+__global__ __launch_bounds__(64 * C * kQ4Chunk / NKB) void q4_small_kernel(
+    const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N, _Float16* y, int64_t ldy,
+    int P, int blocks_m) {
+  __shared__ f4 hand[C][NB * MB][64];
   const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int h = H == 2 && wv >= P ? 1 : 0, p = wv - h * P;
+  const int h = C > 1 ? wv / P : 0, p = wv - h * P;  // chunk, turn
   const int m0 = (int)(blockIdx.x % (unsigned)blocks_m) * 16 * MB, nblk = (int)(blockIdx.x / (unsigned)blocks_m);
   const int kblocks = K >> 5;
-  const int kb0 = h * chunk_blocks + p * NKB, k_end = min(kblocks, (h + 1) * chunk_blocks);
+  const int kb0 = h * kQ4Chunk + p * NKB, k_end = min(kblocks, (h + 1) * kQ4Chunk);
 
   const uint32_t x_bytes = (uint32_t)M * (uint32_t)ldx * 2u;
   const uint32_t x_off = (uint32_t)(m0 + l16) * (uint32_t)ldx * 2u + 16u * kq;
@@ -662,7 +725,7 @@ __global__ __launch_bounds__(1024) void q4_small_kernel(const _Float16* x, int64
   // memory, 16 bytes per lane; blocks past the chain's end are read as zeros.
   constexpr int kBytes = 320 * NB, kUnits = kBytes / 16;  // one K block's records
   constexpr int kRaw = (NKB * kBytes + 1023) / 1024;
-  __shared__ __attribute__((aligned(1024))) char raw[16][kRaw * 1024];
+  __shared__ __attribute__((aligned(1024))) char raw[C * kQ4Chunk / NKB][kRaw * 1024];
   const auto wrs = q4_rsrc(w, w_bytes);
   u4 piece[kRaw];
 #pragma unroll
@@ -710,16 +773,17 @@ __global__ __launch_bounds__(1024) void q4_small_kernel(const _Float16* x, int64
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
           for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = q4_mfma16(b[i][nb], a[i][mb], acc[mb][nb]);
-      if (t < P - 1 || h == 1)
+      if (t < P - 1 || h > 0)
 #pragma unroll
         for (int i = 0; i < NB * MB; ++i) hand[h][i][lane] = acc[i / NB][i % NB];
     }
-    if (t < P - 1 || H == 2) __syncthreads();
+    if (t < P - 1 || C > 1) __syncthreads();
   }
   if (h != 0 || p != P - 1) return;
-  if constexpr (H == 2)
+  if constexpr (C > 1)
+    for (int c = 1; kQ4Chunk * c < kblocks; ++c)
 #pragma unroll
-    for (int i = 0; i < NB * MB; ++i) acc[i / NB][i % NB] = acc[i / NB][i % NB] + hand[1][i][lane];
+      for (int i = 0; i < NB * MB; ++i) acc[i / NB][i % NB] = acc[i / NB][i % NB] + hand[c][i][lane];
 
   const auto yrs = q4_rsrc(y, (uint32_t)M * (uint32_t)ldy * 2u);
   const int n_out = SWIGLU ? N >> 1 : N;
@@ -745,22 +809,22 @@ __global__ __launch_bounds__(1024) void q4_small_kernel(const _Float16* x, int64
   }
 }
 
+constexpr int kQ4SmallChunks = 4;  // 16 wavefronts
 template <bool SWIGLU, int MB, int NB>
 void launch_q4_small(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
                      _Float16* y, int64_t ldy, hipStream_t stream) {
-  const int n_out = SWIGLU ? N / 2 : N, cb = q4_chunk_blocks(K), halves = cb < K / 32 ? 2 : 1;
+  const int n_out = SWIGLU ? N / 2 : N, chunks = q4_chunks(K);
   const int blocks_m = (M + 16 * MB - 1) / (16 * MB), cols = SWIGLU ? 16 : 16 * NB, blocks = blocks_m * ((n_out + cols - 1) / cols);
   // K blocks per wavefront: few, so that its loads and dequantising are short, but each turn of the chain
   // costs a barrier: at K = 2048 four turns of eight blocks beat eight of four (50 rows: 5.1 against 5.4 us).
-  const int nkb = halves == 1 ? 4 : cb <= 32 ? 8 : cb <= 48 ? 6 : 8, P = (cb + nkb - 1) / nkb;
-#define Q4_SMALL(NKB, H) \
-  hipLaunchKernelGGL((q4_small_kernel<SWIGLU, MB, NB, NKB, H>), dim3((unsigned)blocks), dim3(64 * P * H), 0, stream, x, \
-                     ldx, M, K, w, w_bytes, N, y, ldy, cb, P, blocks_m)
-  if (halves == 1) {
-    Q4_SMALL(4, 1);
-  } else if constexpr (MB == 1) {
-    if (nkb == 6) Q4_SMALL(6, 2);
-    else Q4_SMALL(8, 2);
+#define Q4_SMALL(NKB, C, P) \
+  hipLaunchKernelGGL((q4_small_kernel<SWIGLU, MB, NB, NKB, C>), dim3((unsigned)blocks), dim3(64 * (P) * chunks), 0, \
+                     stream, x, ldx, M, K, w, w_bytes, N, y, ldy, P, blocks_m)
+  if constexpr (NB == 2) {
+    if (chunks == 1) Q4_SMALL(4, 1, (K / 32 + 3) / 4);
+  }
+  if constexpr (MB == 1) {
+    if (chunks > 1) Q4_SMALL(8, kQ4SmallChunks, 4);
   }
 #undef Q4_SMALL
 }
@@ -936,7 +1000,7 @@ hipError_t launch_q4_norm_swiglu(const FusedNorm& n, const uint8_t* w, uint32_t 
 }
 
 // ---- K above 1024, at most kQ4DirectBlocks 32 x 32 output blocks beyond q4_small_kernel's: one
-// wavefront per block (two where both halves of K run at once), and no LDS tiles.  Each wavefront
+// wavefront per block (or one per chunk of K), and no LDS tiles.  Each wavefront
 // loads its own X rows and weight records straight into MFMA fragment registers, kQ4Ahead K blocks
 // ahead, dequantises them with the same code and runs the same MFMA chain.
 // Lane (l32, hl) holds X row m0 + l32 and weight row n0 + l32, columns 16 s + 8 hl .. +7 of the
@@ -949,17 +1013,18 @@ hipError_t launch_q4_norm_swiglu(const FusedNorm& n, const uint8_t* w, uint32_t 
 constexpr int kQ4DirectBlocks = 512;
 constexpr int kQ4Ahead = 8;  // K blocks in flight per wavefront (a ring of register stages)
 
-// One workgroup per output block.  PAR: a wavefront per half of K; the chains meet in LDS and
-// wavefront 0 adds them.  Otherwise one wavefront runs the halves in turn and adds the second chain
-// to the first (launches whose second wavefronts would crowd the CUs).
+// One workgroup per output block.  PAR: a wavefront per chunk of K; the chains meet in LDS and
+// wavefront 0 adds them in order.  Otherwise one wavefront runs the chunks in turn and adds each
+// finished chain to the sum (launches whose chunk wavefronts would crowd the CUs).
 // PAR up to one output block per CU.  Measured at M = 15-240 for the output and down projections:
 // 25-46% faster than one wavefront; with more blocks the second wavefronts share CUs and were up to
 // 13% slower.
 constexpr int kQ4ParallelBlocks = 256;
+constexpr int kQ4ParallelChunks = 8;
 template <bool SWIGLU, bool PAR>
-__global__ __launch_bounds__(PAR ? 128 : 64) void q4_direct_kernel(
+__global__ __launch_bounds__(PAR ? 64 * kQ4ParallelChunks : 64) void q4_direct_kernel(
     const _Float16* __restrict__ x, int64_t ldx, int M, int K, const uint8_t* __restrict__ w, uint32_t w_bytes, int N,
-    _Float16* __restrict__ y, int64_t ldy, int chunk_blocks, int blocks_m, int blocks_total) {
+    _Float16* __restrict__ y, int64_t ldy, int blocks_m, int blocks_total) {
   const int lane = threadIdx.x & 63, l32 = lane & 31, hl = lane >> 5;
   const int chunk = PAR ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   // block g: the M blocks of one N block are consecutive (they share weight records in L2)
@@ -967,9 +1032,9 @@ __global__ __launch_bounds__(PAR ? 128 : 64) void q4_direct_kernel(
   if (g >= blocks_total) return;  // the whole workgroup: its barrier below stays uniform
   const int m0 = (g % blocks_m) * 32, n0 = (g / blocks_m) * 32;
   const int kblocks_all = K >> 5;
-  // This wavefront's K blocks [kb0, kblocks): one half, or all of K.
-  const int kb0 = PAR ? chunk * chunk_blocks : 0;
-  const int kblocks = PAR ? min(kb0 + chunk_blocks, kblocks_all) : kblocks_all;
+  // This wavefront's K blocks [kb0, kblocks): one chunk, or all of K.
+  const int kb0 = PAR ? chunk * kQ4Chunk : 0;
+  const int kblocks = PAR ? min(kb0 + kQ4Chunk, kblocks_all) : kblocks_all;
   const int n_out = SWIGLU ? N >> 1 : N;  // output columns
 
   const auto xrs = q4_rsrc(x, (uint32_t)M * (uint32_t)ldx * 2u);  // rows >= M read as zeros
@@ -1028,6 +1093,7 @@ __global__ __launch_bounds__(PAR ? 128 : 64) void q4_direct_kernel(
   // kb + kQ4Ahead.
   constexpr int kWait = (kQ4Ahead - 1) * kOps;
   static_assert(kWait < 64, "vmcnt is 6 bits");
+  static_assert(kQ4Chunk % kQ4Ahead == 0, "chunks end between ring passes");
   f16x tot_g = {}, tot_u = {};
   for (int kb = kb0; kb < kblocks; kb += kQ4Ahead) {
 #pragma unroll
@@ -1039,12 +1105,12 @@ __global__ __launch_bounds__(PAR ? 128 : 64) void q4_direct_kernel(
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (!PAR) {
-      // End of a half: add the chain to the sum and start the next from zero.
-      if (kb + kQ4Ahead == chunk_blocks || kb + kQ4Ahead >= kblocks) {
-        tot_g = kb < chunk_blocks ? acc_g : tot_g + acc_g;
+      // End of a chunk: add the chain to the sum and start the next from zero.
+      if ((kb + kQ4Ahead) % kQ4Chunk == 0 || kb + kQ4Ahead >= kblocks) {
+        tot_g = kb < kQ4Chunk ? acc_g : tot_g + acc_g;
         acc_g = f16x{};
         if constexpr (SWIGLU) {
-          tot_u = kb < chunk_blocks ? acc_u : tot_u + acc_u;
+          tot_u = kb < kQ4Chunk ? acc_u : tot_u + acc_u;
           acc_u = f16x{};
         }
       }
@@ -1056,16 +1122,18 @@ __global__ __launch_bounds__(PAR ? 128 : 64) void q4_direct_kernel(
     acc_u = tot_u;
   }
   if constexpr (PAR) {
-    __shared__ f16x part_g[64];
-    __shared__ f16x part_u[SWIGLU ? 64 : 1];
+    __shared__ f16x part_g[kQ4ParallelChunks - 1][64];
+    __shared__ f16x part_u[SWIGLU ? kQ4ParallelChunks - 1 : 1][SWIGLU ? 64 : 1];
     if (chunk > 0) {
-      part_g[lane] = acc_g;
-      if constexpr (SWIGLU) part_u[lane] = acc_u;
+      part_g[chunk - 1][lane] = acc_g;
+      if constexpr (SWIGLU) part_u[chunk - 1][lane] = acc_u;
     }
     __syncthreads();
     if (chunk > 0) return;
-    acc_g = acc_g + part_g[lane];
-    if constexpr (SWIGLU) acc_u = acc_u + part_u[lane];
+    for (int c = 1; kQ4Chunk * c < kblocks_all; ++c) {
+      acc_g = acc_g + part_g[c - 1][lane];
+      if constexpr (SWIGLU) acc_u = acc_u + part_u[c - 1][lane];
+    }
   }
 
   // D (32 x 32): lane holds column l32 and rows 8 (r / 4) + 4 hl + r % 4.
@@ -1087,13 +1155,13 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
                       _Float16* y, int64_t ldy, hipStream_t stream) {
   const int n_out = SWIGLU ? N / 2 : N;
   const int blocks_m = (M + 31) / 32, blocks = blocks_m * ((n_out + 31) / 32);
-  const int cb = q4_chunk_blocks(K);
-  if (blocks <= kQ4ParallelBlocks)
-    hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, true>), dim3((unsigned)blocks), dim3(128), 0, stream, x, ldx, M, K, w,
-                       w_bytes, N, y, ldy, cb, blocks_m, blocks);
+  const int chunks = q4_chunks(K);
+  if (blocks <= kQ4ParallelBlocks && chunks <= kQ4ParallelChunks)
+    hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, true>), dim3((unsigned)blocks), dim3(64 * chunks), 0, stream, x, ldx, M,
+                       K, w, w_bytes, N, y, ldy, blocks_m, blocks);
   else
     hipLaunchKernelGGL((q4_direct_kernel<SWIGLU, false>), dim3((unsigned)blocks), dim3(64), 0, stream, x, ldx, M, K, w,
-                       w_bytes, N, y, ldy, cb, blocks_m, blocks);
+                       w_bytes, N, y, ldy, blocks_m, blocks);
 }
 
 // The kernel and tile by the number of tiles, i.e. by how a launch fills the 256 CUs (times in us).
@@ -1107,49 +1175,69 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
 //   * then 256 x 256 tiles where their last round of 256 is mostly full (N = 4096: M = 2,400 27.5
 //     against 29.5, M = 8,000 65 against 68), else 256 x 128 tiles, whose second workgroup per CU
 //     fills the gap (N = 6144, M = 4,000: 1.5 rounds, 60 against 53).
-// K above 1024 (N = 1024, K = 2048):
-//   * q4_small_kernel while its 16 x 16 blocks are at most one per CU (M = 50 4.6, 16 x 32 blocks 5.1;
-//     K = 3072 6.0 against 6.7), then while its 16 x 32 blocks are (M = 100 5.9, direct 7.5; M = 150,
-//     320 blocks, 10.4 against 7.8) and a half's blocks fit its eight wavefronts;
-//   * q4_direct_kernel up to kQ4DirectBlocks;
-//   * up to 256 tiles of 64 x 128: q4_mid_kernel (M = 1,419 13.2, 128 x 128 tiles 19.8);
-//   * then 128 x 128 tiles while at most one per CU (M = 2,400 20.3, mid 25.4, 256 x 128 27.6);
-//   * then 256 x 128 or 128 x 128 tiles by the rounds each needs (M = 8,000: one round of 38.8 against
-//     two of 22.7).
+// K above 1024 (N = 1024):
+//   * q4_small_kernel while its 16 x 16 blocks are at most one per CU (K = 2048, M = 50 4.6, 16 x 32 blocks
+//     5.1; K = 3072 6.2 against 7.0), then while its 16 x 32 blocks are (K = 3072, M = 100 7.2, direct 10.5;
+//     M = 150, 320 blocks, 12.2 against 10.7) and a workgroup holds a wavefront for every part of K;
+//   * q4_direct_kernel up to kQ4DirectBlocks (K = 3072, M = 500 16.5, mid 17.5);
+//   * up to 256 tiles of 64 x 128: q4_mid_kernel, a group per chunk (K = 2048, M = 1,419 13.2, 128 x 128
+//     tiles 19.8; K = 3072 18.4);
+//   * K up to 2048: 128 x 128 tiles while at most one per CU (M = 2,400 20.3, mid 25.4, 256 x 128 27.6),
+//     then 256 x 128 or 128 x 128 tiles by the rounds each needs (M = 8,000: one round of 38.8 against two
+//     of 22.7);
+//   * K up to 3072: 128 x 128 tiles with three groups while at most one per CU (M = 4,000 31.9; mid 37.1,
+//     128 x 256 folding 49.5); beyond, three groups of larger tiles do not fit in LDS;
+//   * K above 3072: folding q4_mid_kernel up to 512 tiles, two workgroups per CU (K = 4096, M = 4,000 47.2,
+//     128 x 256 tiles 64.4; M = 5,000, 632 tiles, 66.1 against 64.8);
+//   * the rest folds the chunks in 128 x 256 tiles where their last round of 256 is mostly full (K = 3072,
+//     M = 8,000 55 against 61 with 128 x 128 tiles, M = 16,000 114 against 120), else in 128 x 128 tiles, whose
+//     second workgroup per CU fills the gap (M = 12,000, 1.5 rounds, 92 against 106).
 template <bool SWIGLU>
 hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
                      _Float16* y, int64_t ldy, hipStream_t stream) {
-  const int n_out = SWIGLU ? N / 2 : N, cb = q4_chunk_blocks(K);
+  const int n_out = SWIGLU ? N / 2 : N, chunks = q4_chunks(K);
   const auto tiles = [&](int tm, int tn) { return (int64_t)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
   const auto rounds = [](int64_t t) { return (t + 255) / 256; };
-#define Q4_TILE(MF, NWN, G) launch_q4_tile<SWIGLU, MF, NWN, G>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream)
-  if (cb == K / 32) {
+#define Q4_TILE(...) launch_q4_tile<SWIGLU, __VA_ARGS__>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream)
+#define Q4_MID(...) launch_q4_mid<SWIGLU, __VA_ARGS__>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream)
+  if (chunks == 1) {
     const int64_t t = tiles(256, 256);
     if (tiles(16, 32) <= 256)
       launch_q4_small<SWIGLU, 1, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if (tiles(32, 32) <= 512)
       launch_q4_small<SWIGLU, 2, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if (tiles(64, 128) <= 512)
-      launch_q4_mid<SWIGLU, 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+      Q4_MID(1);
     else if (tiles(256, 128) <= 256 || (t > 256 && 256 * rounds(t) * 100 > 115 * t))
       Q4_TILE(8, 2, 1);
     else
       Q4_TILE(8, 4, 1);
   } else {
-    const int64_t big = rounds(tiles(256, 128)), small = rounds(tiles(128, 128));
-    if (tiles(16, 16) <= 256 && cb <= 64 && !SWIGLU)
+    const int64_t big = rounds(tiles(256, 128)), small = rounds(tiles(128, 128)), wide = tiles(128, 256);
+    if (tiles(16, 16) <= 256 && chunks <= kQ4SmallChunks && !SWIGLU)
       launch_q4_small<SWIGLU, 1, SWIGLU ? 2 : 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
-    else if (tiles(16, 32) <= 256 && cb <= 64)
+    else if (tiles(16, 32) <= 256 && chunks <= kQ4SmallChunks)
       launch_q4_small<SWIGLU, 1, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if ((int64_t)((M + 31) / 32) * ((n_out + 31) / 32) <= kQ4DirectBlocks)
       launch_q4_direct<SWIGLU>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
-    else if (tiles(64, 128) <= 256)
-      launch_q4_mid<SWIGLU, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
+    else if (chunks == 2 && tiles(64, 128) <= 256)
+      Q4_MID(2);
+    else if (chunks == 3 && tiles(64, 128) <= 256)
+      Q4_MID(3);
+    else if (chunks == 3 && small == 1)
+      Q4_TILE(4, 2, 3);
+    else if (chunks > 3 && tiles(64, 128) <= 512)
+      Q4_MID(1, true);
+    else if (chunks > 2 && wide > 256 && 256 * rounds(wide) * 100 > 115 * wide)
+      Q4_TILE(4, 2, 1, true);
+    else if (chunks > 2)
+      Q4_TILE(4, 4, 1, true);
     else if (small > 1 && 5 * big <= 3 * small)
       Q4_TILE(8, 2, 2);
     else
       Q4_TILE(4, 2, 2);
   }
+#undef Q4_MID
 #undef Q4_TILE
   return hipGetLastError();
 }

@@ -249,3 +249,26 @@ def test_q4_weights_need_only_4_byte_alignment(ctx, m, k, n):
     for b in (bx, bw, by):
         b.free()
     assert np.array_equal(y, run_q4(ctx, x, packed, k, n).view(np.uint16))
+
+
+@pytest.mark.parametrize("k", [3072, 3104, 4096, 5120, 8192])
+@pytest.mark.parametrize("m", [5, 100, 300, 500, 1419, 3000, 4200])
+def test_q4_sums_restart_every_1024_columns(ctx, m, k):
+    """fp32 sums over K are chains of 1,024 columns, added in order, so a chain's rounding bound does not
+    grow with K.  Column 0 contributes 2^30 and column 0 of the last chunk takes it away again; the
+    chunks between hold ones.  A chain that carried 2^30 (spacing 128) into a block of ones would lose
+    its 32; chains of their own keep every one: the result is the count of ones, exactly."""
+    n, kb, last = 1024, k // 32, (k - 1) // 1024 * 32
+    rec = np.zeros((n // 32, kb, 32, 20), np.uint8)
+    rec[..., 4:20] = 0x88  # q - 8 = 0
+    rec[:, [0, last], 0::2, 0:2] = np.array([8192], np.float16).view(np.uint8)
+    rec[:, [0, last], 0::2, 4] = 0x8C  # column 0: (12 - 8) * 8192 = 2^15
+    rec[:, 32:last, 0::2, 0:2] = np.array([1], np.float16).view(np.uint8)
+    rec[:, 32:last, 0::2, 4:20] = 0x99
+    x = np.ones((m, k), np.float16)
+    x[:, 0], x[:, 32 * last] = 2.0 ** 15, -(2.0 ** 15)
+    x[1::2] *= -1
+    y = run_q4(ctx, x, rec.reshape(-1), k, n).astype(np.float64)
+    expected = np.zeros((m, n))
+    expected[:, 0::2] = np.where(np.arange(m) % 2, -1.0, 1.0)[:, None] * (32 * last - 1024)
+    assert np.array_equal(y, expected)
