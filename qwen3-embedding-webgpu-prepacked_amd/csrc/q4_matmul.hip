@@ -691,7 +691,7 @@ void launch_q4_mid(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* 
 // ---- the smallest launches: one workgroup per 16 MB x 16 NB block of output (SWIGLU: 16 features),
 // its wavefronts sharing K.  Wavefront p of a chain loads and dequantises K blocks NKB p .. + NKB - 1,
 // all at once; then the chain runs through the wavefronts in turn, the accumulators passing from one
-// to the next through LDS, so the sums are the same as in one wavefront.  C > 1 (K above 1024): up to C
+// to the next through LDS, so the sums are the same as in one wavefront.  C > 1 (K above 1024): the C
 // chunks of K run side by side and are added in order at the end.
 // What bounds it: a launch's fixed 3 us or so, one memory round trip, and P hand-overs of about 0.2 us;
 // one wavefront running the whole chain dequantised 32 blocks in sequence instead.  Weight records
@@ -702,8 +702,9 @@ void launch_q4_mid(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* 
 template <bool SWIGLU, int MB, int NB, int NKB, int C>
 __global__ __launch_bounds__(64 * C * kQ4Chunk / NKB) void q4_small_kernel(
     const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N, _Float16* y, int64_t ldy,
-    int P, int blocks_m) {
+    int turns, int blocks_m) {
   __shared__ f4 hand[C][NB * MB][64];
+  const int P = C > 1 ? kQ4Chunk / NKB : turns;  // wavefronts of a chain
   const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = C > 1 ? wv / P : 0, p = wv - h * P;  // chunk, turn
@@ -781,7 +782,8 @@ __global__ __launch_bounds__(64 * C * kQ4Chunk / NKB) void q4_small_kernel(
   }
   if (h != 0 || p != P - 1) return;
   if constexpr (C > 1)
-    for (int c = 1; kQ4Chunk * c < kblocks; ++c)
+#pragma unroll
+    for (int c = 1; c < C; ++c)
 #pragma unroll
       for (int i = 0; i < NB * MB; ++i) acc[i / NB][i % NB] = acc[i / NB][i % NB] + hand[c][i][lane];
 
@@ -818,13 +820,15 @@ void launch_q4_small(const _Float16* x, int64_t ldx, int M, int K, const uint8_t
   // K blocks per wavefront: few, so that its loads and dequantising are short, but each turn of the chain
   // costs a barrier: at K = 2048 four turns of eight blocks beat eight of four (50 rows: 5.1 against 5.4 us).
 #define Q4_SMALL(NKB, C, P) \
-  hipLaunchKernelGGL((q4_small_kernel<SWIGLU, MB, NB, NKB, C>), dim3((unsigned)blocks), dim3(64 * (P) * chunks), 0, \
-                     stream, x, ldx, M, K, w, w_bytes, N, y, ldy, P, blocks_m)
+  hipLaunchKernelGGL((q4_small_kernel<SWIGLU, MB, NB, NKB, C>), dim3((unsigned)blocks), dim3(64 * (P) * C), 0, stream, \
+                     x, ldx, M, K, w, w_bytes, N, y, ldy, P, blocks_m)
   if constexpr (NB == 2) {
     if (chunks == 1) Q4_SMALL(4, 1, (K / 32 + 3) / 4);
   }
   if constexpr (MB == 1) {
-    if (chunks > 1) Q4_SMALL(8, kQ4SmallChunks, 4);
+    if (chunks == 2) Q4_SMALL(8, 2, 4);
+    if (chunks == 3) Q4_SMALL(8, 3, 4);
+    if (chunks == 4) Q4_SMALL(8, 4, 4);
   }
 #undef Q4_SMALL
 }
