@@ -39,12 +39,17 @@ __device__ inline void rmsnorm_row(const half_t* xr, const half_t* rr, half_t* x
       half8 a = *reinterpret_cast<const half8*>(xr + c);
       if (rr) {
         const half8 b = *reinterpret_cast<const half8*>(rr + c);
+        float s[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const float s = (float)a[e] + (float)b[e];
-          ss = fmaf(s, s, ss);
-          a[e] = (half_t)s;
+          s[e] = (float)a[e] + (float)b[e];
+          a[e] = (half_t)s[e];
         }
+        // The row's first pair adds its squares the other way round: the order (and so the rounding) that
+        // embeddings stored by earlier builds were made with.
+        if (j == 0) ss = fmaf(s[0], s[0], s[1] * s[1]);
+#pragma unroll
+        for (int e = j == 0 ? 2 : 0; e < 8; ++e) ss = fmaf(s[e], s[e], ss);
         if (x_out) *reinterpret_cast<half8*>(x_out + c) = a;
       } else {
 #pragma unroll

@@ -1,0 +1,39 @@
+"""The roundings of the residual add + RMSNorm (qattn_rmsnorm), bit for bit against a host restatement of
+its arithmetic: embeddings stored by earlier builds stay equal."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+F32 = np.float32
+
+
+def fma(a, b, c):
+    """a b + c of f32 values in 64 bits: the product is exact there, and the sum is rounded far below the
+    f32 or fp16 rounding that the caller applies."""
+    return a.astype(np.float64) * b.astype(np.float64) + c.astype(np.float64)
+
+
+def test_rmsnorm_with_residual_bits(ctx):
+    rows, width, eps = 8000, 1024, 1e-6
+    rng = np.random.default_rng(3)
+    x, r = (rng.standard_normal((rows, width)).astype(np.float16) for _ in range(2))
+    w = (1 + 0.1 * rng.standard_normal(width)).astype(F32)
+    bx, br, bw = ctx.upload(x.view(np.uint16)), ctx.upload(r.view(np.uint16)), ctx.upload(w)
+    bo = ctx.alloc(rows * width * 2)
+    ctx.rmsnorm(bx.ptr, bw.ptr, bo.ptr, rows, width, residual_ptr=br.ptr, eps=eps)
+    ctx.synchronize()
+    got_x, got = bx.read(np.uint16, (rows, width)), bo.read(np.uint16, (rows, width))
+    for b in (bx, br, bw, bo):
+        b.free()
+    s = x.astype(F32) + r.astype(F32)
+    # lane l sums columns 8 l .. + 7 and 512 + 8 l .. + 7, the first pair's squares as fma(s0, s0, s1 s1)
+    lanes = np.concatenate([s[:, :512].reshape(rows, 64, 8), s[:, 512:].reshape(rows, 64, 8)], axis=-1)
+    ss = fma(lanes[..., 0], lanes[..., 0], lanes[..., 1] * lanes[..., 1]).astype(F32)
+    for e in range(2, 16):
+        ss = fma(lanes[..., e], lanes[..., e], ss).astype(F32)
+    for d in (32, 16, 8, 4, 2, 1):
+        ss = ss + ss[:, np.arange(64) ^ d]
+    inv = F32(1) / np.sqrt(ss[:, :1] / F32(width) + F32(eps))
+    x16 = s.astype(np.float16)
+    assert np.array_equal(got_x, x16.view(np.uint16))
+    assert np.array_equal(got, (x16.astype(F32) * inv * w).astype(np.float16).view(np.uint16))
