@@ -976,7 +976,7 @@ __global__ __launch_bounds__(QKV ? 1024 : 512) void q4_fused_kernel(FusedNorm n,
     const float4 g0 = reinterpret_cast<const float4*>(gains)[2 * l16], g1 = reinterpret_cast<const float4*>(gains)[2 * l16 + 1];
     const float4* const cs = reinterpret_cast<const float4*>(out.rope + (int64_t)pos * 64 + 8 * (l16 & 7));
     const float4 c4[4] = {cs[0], cs[1], cs[2], cs[3]};
-    const rope_h8 r = rope_vector(x, g0, g1, c4, l16, out.eps);
+    const rope_h8 r = rope_vector(x, g0, g1, c4, l16, out.eps, nblk >> 2);
     half_t* const dst = nblk < 16 ? out.q + (size_t)t * 2048 + nblk * 128 : out.k + (size_t)t * 1024 + (nblk - 16) * 128;
     if (t < n.tokens) *reinterpret_cast<rope_h8*>(dst + 8 * l16) = r;
   }

@@ -38,7 +38,34 @@ __device__ inline float wave_sum(float v) {
 // reduced over the 16 lanes in a fixed order; the rotate-half partner of element d
 // (d +- 64) sits in lane j ^ 8 at the same slot.  The one formula of qk_norm_rope_kernel and of the
 // fused small projection, so the two agree bit for bit.
-__device__ inline rope_h8 rope_vector(rope_h8 x, float4 g0, float4 g1, const float4 (&c4)[4], int j, float eps) {
+// quad: the vector's place among a token's head vectors, in fours.
+// A rotated element is fma(n, cos, partner * sin) rounded once to fp16, except elements 1-6 of the first
+// four vectors and 2-7 of the second four: they round to fp32 and then to fp16, and every other one
+// of them is fma(partner, sin, n * cos).  That is how the compiler once laid out the separate launch;
+// it is spelled out so that embeddings stored by earlier builds stay equal bit for bit and no
+// longer depend on the compiler.
+template <int QUAD>
+__device__ inline rope_h8 rope_rotate(const float (&n)[8], const float (&partner)[8], const float4 (&c4)[4]) {
+  rope_h8 r;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float4 c = c4[e >> 1];  // (cos, sin) of slots e & ~1 and e | 1
+    const float cos = e & 1 ? c.z : c.x, sin = e & 1 ? c.w : c.y;
+    half_t h;
+    if (QUAD == 0 ? e >= 1 && e <= 6 : QUAD == 1 && e >= 2) {
+      float o = (e & 1) == (QUAD == 0) ? fmaf(partner[e], sin, n[e] * cos) : fmaf(n[e], cos, partner[e] * sin);
+      asm volatile("" : "+v"(o));  // rounded to fp32 first
+      h = (half_t)o;
+    } else {
+      h = (half_t)fmaf(n[e], cos, partner[e] * sin);
+      // Kept apart from its neighbour, so that the compiler fuses the rounding (v_fma_mix{lo,hi}_f16).
+      if (!(e & 1)) asm volatile("" : "+v"(h));
+    }
+    r[e] = h;
+  }
+  return r;
+}
+__device__ inline rope_h8 rope_vector(rope_h8 x, float4 g0, float4 g1, const float4 (&c4)[4], int j, float eps, int quad) {
   float v[8], ss = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -48,19 +75,14 @@ __device__ inline rope_h8 rope_vector(rope_h8 x, float4 g0, float4 g1, const flo
   ss = row_sum(ss);
   const float inv = __frsqrt_rn(fmaf(ss, 1.0f / 128.0f, eps));
   const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-  float n[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) n[e] = v[e] * inv * g[e];
-  rope_h8 r;
+  float n[8], partner[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const float4 c = c4[e >> 1];  // (cos, sin) of slots e & ~1 and e | 1
-    const float partner = row_rotate<8>(n[e]);
-    float o = fmaf(j < 8 ? -partner : partner, e & 1 ? c.w : c.y, n[e] * (e & 1 ? c.z : c.x));
-    asm volatile("" : "+v"(o));  // rounded to fp32, then to fp16, in every caller
-    r[e] = (half_t)o;
+    n[e] = v[e] * inv * g[e];
+    const float rotated = row_rotate<8>(n[e]);
+    partner[e] = j < 8 ? -rotated : rotated;
   }
-  return r;
+  return quad == 0 ? rope_rotate<0>(n, partner, c4) : quad == 1 ? rope_rotate<1>(n, partner, c4) : rope_rotate<2>(n, partner, c4);
 }
 
 constexpr int kRopeSeqs = 64;

@@ -52,8 +52,8 @@ __global__ void fill_normal_kernel(half_t* dst, int64_t rows, int64_t row_elems,
 // one token: its head vectors go four at a time to the four 16-lane groups (lane j of a group
 // holds elements 8j..8j+7 of its vector: 16-byte loads and stores), every vector's load issued
 // before the first is used.  The token's cos/sin row and the gains are read once per lane for
-// all its vectors.  The sum of squares is reduced over the 16 lanes by xor-shuffles in a fixed
-// order; the rotate-half partner of element d (d +- 64) sits in lane j ^ 8 at the same slot.
+// all its vectors.  The arithmetic is rope_vector's (qk_rope.h): sums and rotate-half partners move by DPP
+// within the 16 lanes.
 // Positions restart at every sequence boundary; the launch covers up to kRopeSeqs sequences whose
 // offsets come by value, the token's sequence found by one ballot over them.
 template <int ITERS>
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(RopeArgs a) {
   for (int it = 0; it < ITERS; ++it) {
     const int h = 4 * it + grp;
     const bool isq = h < a.split;
-    const h8v r = rope_vector(x[it], isq ? wq[0] : wk[0], isq ? wq[1] : wk[1], c4, j, a.eps);
+    const h8v r = rope_vector(x[it], isq ? wq[0] : wk[0], isq ? wq[1] : wk[1], c4, j, a.eps, it);
     half_t* dst = isq ? a.out_q + (int64_t)t * a.out_stride_q + h * 128
                       : a.out_k + (int64_t)t * a.out_stride_k + (h - a.split) * 128;
     *reinterpret_cast<h8v*>(dst + 8 * j) = r;

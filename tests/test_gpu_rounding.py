@@ -1,5 +1,6 @@
-"""The roundings of the residual add + RMSNorm (qattn_rmsnorm), bit for bit against a host restatement of
-its arithmetic: embeddings stored by earlier builds stay equal."""
+"""The roundings of the residual add + RMSNorm (qattn_rmsnorm) and of the QK norm + RoPE
+(qattn_qk_norm_rope*), bit for bit against a host restatement of their arithmetic: embeddings stored by
+earlier builds stay equal, and a row does not depend on the kernel that computed it."""
 import numpy as np
 import pytest
 
@@ -37,3 +38,34 @@ def test_rmsnorm_with_residual_bits(ctx):
     x16 = s.astype(np.float16)
     assert np.array_equal(got_x, x16.view(np.uint16))
     assert np.array_equal(got, (x16.astype(F32) * inv * w).astype(np.float16).view(np.uint16))
+
+
+@pytest.mark.parametrize("heads", [4, 8, 12, 24, 32])
+def test_rope_bits(ctx, heads):
+    """Rows of +-1 with eps = 0 have unit RMS, so the normalised element is the gain, exactly."""
+    tokens, theta = 1500, 1e6
+    rng = np.random.default_rng(heads)
+    sign = rng.choice(np.array([-1, 1], np.float16), (tokens, heads * 128))
+    gain = (1 + 0.1 * rng.standard_normal(128)).astype(F32)
+    bx, bw = ctx.upload(sign.view(np.uint16)), ctx.upload(gain)
+    ctx.qk_norm_rope(bx.ptr, heads * 128, 0, heads, np.array([0, tokens], np.int32), weight_ptr=bw.ptr, eps=0.0,
+                     theta=theta)
+    ctx.synchronize()
+    got = bx.read(np.uint16, (tokens, heads, 2, 8, 8))  # half, lane, element
+    bx.free()
+    bw.free()
+    angle = np.arange(tokens, dtype=np.float64)[:, None] * theta ** (-np.arange(64, dtype=np.float64) / 64)
+    cos, sin = (f(angle).astype(F32).reshape(tokens, 1, 1, 8, 8) for f in (np.cos, np.sin))
+    n = sign.astype(F32).reshape(tokens, heads, 2, 8, 8) * gain.reshape(1, 1, 2, 8, 8)
+    partner = np.stack([-n[:, :, 1], n[:, :, 0]], axis=2)
+    cos_last = fma(n, np.broadcast_to(cos, n.shape), partner * sin)  # one rounding, then two, then the other order
+    sin_last = fma(partner, np.broadcast_to(sin, n.shape), n * cos)
+    once, twice = cos_last.astype(np.float16), cos_last.astype(F32).astype(np.float16)
+    other = sin_last.astype(F32).astype(np.float16)
+    expected = once.copy()
+    expected[:, 0:4, ..., 1:7] = twice[:, 0:4, ..., 1:7]
+    expected[:, 0:4, ..., 1:7:2] = other[:, 0:4, ..., 1:7:2]
+    expected[:, 4:8, ..., 2:8] = twice[:, 4:8, ..., 2:8]
+    expected[:, 4:8, ..., 2:8:2] = other[:, 4:8, ..., 2:8:2]
+    differ = np.argwhere(got != expected.view(np.uint16))
+    assert len(differ) == 0, (len(differ), differ[:4])
