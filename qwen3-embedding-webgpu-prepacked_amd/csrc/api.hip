@@ -32,6 +32,7 @@ hipError_t launch_fill_normal(half_t* dst, int64_t rows, int64_t row_elems, int6
                               uint64_t seed, hipStream_t stream);
 hipError_t launch_fill_token_rows(half_t* dst, const int32_t* ids, int64_t rows, int64_t row_elems,
                                   int64_t row_stride, uint64_t seed, hipStream_t stream);
+// w_bytes: exactly the tensor's bytes (qattn_q4_compact_bytes), however many the caller's buffer holds.
 hipError_t launch_q4_matmul(const half_t* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
                             half_t* y, int64_t ldy, hipStream_t stream);
 hipError_t launch_q4_matmul_swiglu(const half_t* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes,
@@ -879,7 +880,8 @@ int qattn_q4_matmul(qattn_ctx* ctx, const void* x, int64_t ldx, int32_t M, int32
   if (rc != QATTN_OK) return rc;
   DeviceGuard g(ctx->device);
   HIP_TRY(ctx, launch_q4_matmul(static_cast<const half_t*>(x), ldx, M, K, static_cast<const uint8_t*>(w),
-                                (uint32_t)w_bytes, N, static_cast<half_t*>(y), ldy, pick_stream(ctx, stream)));
+                                (uint32_t)qattn_q4_compact_bytes(K, N), N, static_cast<half_t*>(y), ldy,
+                                pick_stream(ctx, stream)));
   return QATTN_OK;
 }
 
@@ -891,8 +893,8 @@ int qattn_q4_matmul_swiglu(qattn_ctx* ctx, const void* x, int64_t ldx, int32_t M
   if (rc != QATTN_OK) return rc;
   DeviceGuard g(ctx->device);
   HIP_TRY(ctx, launch_q4_matmul_swiglu(static_cast<const half_t*>(x), ldx, M, K, static_cast<const uint8_t*>(w),
-                                       (uint32_t)w_bytes, n_inter, static_cast<half_t*>(y), ldy,
-                                       pick_stream(ctx, stream)));
+                                       (uint32_t)qattn_q4_compact_bytes(K, 2 * n_inter), n_inter,
+                                       static_cast<half_t*>(y), ldy, pick_stream(ctx, stream)));
   return QATTN_OK;
 }
 

@@ -238,7 +238,7 @@ int enqueue_fused(qattn_model_plan* p, const int32_t* cu, int32_t nseq, float* o
     heads.weight_q = w.attn_q_norm;
     heads.weight_k = w.attn_k_norm;
     HIP_TRY(ctx, launch_q4_norm_qkv({x, l ? delta : nullptr, x_next, w.attn_norm, (float)d.eps, T},
-                                    static_cast<const uint8_t*>(w.attn_qkv), (uint32_t)w.attn_qkv_bytes, heads, stream));
+                                    static_cast<const uint8_t*>(w.attn_qkv), (uint32_t)qattn_q4_compact_bytes(kHidden, kQkvWidth), heads, stream));
     if (l) std::swap(x, x_next);
     done();
     stage(QATTN_STAGE_ROPE_ATTENTION);
@@ -253,7 +253,8 @@ int enqueue_fused(qattn_model_plan* p, const int32_t* cu, int32_t nseq, float* o
     done();
     stage(QATTN_STAGE_FFN_UP_GATE);
     HIP_TRY(ctx, launch_q4_norm_swiglu({x, delta, x_next, w.ffn_norm, (float)d.eps, T},
-                                       static_cast<const uint8_t*>(w.ffn_gate_up), (uint32_t)w.ffn_gate_up_bytes, kInter,
+                                       static_cast<const uint8_t*>(w.ffn_gate_up),
+                                       (uint32_t)qattn_q4_compact_bytes(kHidden, 2 * kInter), kInter,
                                        static_cast<half_t*>(p->ffn), kInter, stream));
     std::swap(x, x_next);
     done();

@@ -78,6 +78,12 @@ __device__ inline h8 dequant8(u2 q, h2 scale) {
   return __builtin_bit_cast(h8, u4{a[0], a[1], b[0], b[1]});
 }
 
+// Buffer ranges.  The range check covers the per-lane offset (and the instruction's), not the scalar one
+// that carries the K block, so a range ends exactly where its last row or weight tile does: w_bytes is the
+// tensor's own size, and a row past M or a weight row past the last tile of 32 lies outside whatever its K
+// block.  A row's K blocks lie within the row (K <= ldx).  Tiles overhang M by at most 255 rows:
+// (M + 255) * ldx * 2 < 2^32 for every x that the entry points accept ((M + 128) * ldx * 2 < 2^31), so
+// their offsets do not wrap.
 typedef __attribute__((address_space(3))) void lds_void_t;
 
 // LDS tiles: rows of 32 columns of fp16 (64 B per row) for X (A) and for the dequantised weights (B,
