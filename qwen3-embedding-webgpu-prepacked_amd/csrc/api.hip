@@ -730,10 +730,10 @@ namespace qattn {
 // The context's RoPE table covering `positions` positions for `theta` (model.ts:76-81: angle =
 // pos * theta^(-i/64) in f64, cos / sin rounded to f32), rebuilt only when it must grow or theta
 // changes.  A rebuild uploads synchronously; every other call only reads it.
-int rope_table(qattn_ctx* ctx, int32_t positions, double theta, const float2** out) {
-  std::lock_guard<std::mutex> lock(ctx->mu);
+int rope_table(qattn_ctx* ctx, int32_t positions, double theta, RopeTable* out) {
+  std::unique_lock<std::mutex> lock(ctx->rope_mu);
   if (ctx->rope && ctx->rope_positions >= positions && ctx->rope_theta == theta) {
-    *out = ctx->rope;
+    *out = {ctx->rope, std::move(lock)};
     return QATTN_OK;
   }
   const int32_t n = std::max(positions, std::max(ctx->rope_positions, 1024));
@@ -747,22 +747,22 @@ int rope_table(qattn_ctx* ctx, int32_t positions, double theta, const float2** o
   float2* dev = nullptr;
   hipError_t e = hipMalloc(&dev, table.size() * sizeof(float2));
   if (e != hipSuccess) {
-    ctx->last_error = std::string("RoPE table: ") + hipGetErrorString(e);
-    g_last_error = ctx->last_error;
+    set_last_error(ctx, std::string("RoPE table: ") + hipGetErrorString(e));
     return QATTN_ENOMEM;
   }
   e = hipMemcpy(dev, table.data(), table.size() * sizeof(float2), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     (void)hipFree(dev);
-    ctx->last_error = std::string("RoPE table upload: ") + hipGetErrorString(e);
-    g_last_error = ctx->last_error;
+    set_last_error(ctx, std::string("RoPE table upload: ") + hipGetErrorString(e));
     return QATTN_EHIP;
   }
-  if (ctx->rope) (void)hipFree(ctx->rope);  // waits for the device to be idle first
+  // hipFree waits for the device to be idle first, and no launch that reads the old table is yet to be
+  // enqueued: its caller would hold rope_mu.
+  if (ctx->rope) (void)hipFree(ctx->rope);
   ctx->rope = dev;
   ctx->rope_positions = n;
   ctx->rope_theta = theta;
-  *out = dev;
+  *out = {dev, std::move(lock)};
   return QATTN_OK;
 }
 
@@ -789,14 +789,14 @@ int qattn_qk_norm_rope(qattn_ctx* ctx, void* x, int64_t row_stride, int64_t col0
   int rc = validate_cu(ctx, cu_seqlens, nseq);
   if (rc) return rc;
   if (cu_seqlens[nseq] == 0) return QATTN_OK;
-  const float2* table = nullptr;
+  RopeTable table;
   rc = rope_table(ctx, longest(cu_seqlens, nseq), theta, &table);
   if (rc) return rc;
   RopeArgs a{};
   a.in = static_cast<const half_t*>(x);
   a.out_q = a.out_k = static_cast<half_t*>(x) + col0;
   a.weight_q = a.weight_k = weight;
-  a.rope = table;
+  a.rope = table.data;
   a.in_stride = a.out_stride_q = a.out_stride_k = row_stride;
   a.in_col_q = a.in_col_k = col0;
   a.heads = a.split = heads;
@@ -822,7 +822,7 @@ int qattn_qk_norm_rope_qkv(qattn_ctx* ctx, const void* qkv, int64_t qkv_row_stri
   int rc = validate_cu(ctx, cu_seqlens, nseq);
   if (rc) return rc;
   if (cu_seqlens[nseq] == 0) return QATTN_OK;
-  const float2* table = nullptr;
+  RopeTable table;
   rc = rope_table(ctx, longest(cu_seqlens, nseq), theta, &table);
   if (rc) return rc;
   RopeArgs a{};
@@ -831,7 +831,7 @@ int qattn_qk_norm_rope_qkv(qattn_ctx* ctx, const void* qkv, int64_t qkv_row_stri
   a.out_k = static_cast<half_t*>(k);
   a.weight_q = q_weight;
   a.weight_k = k_weight;
-  a.rope = table;
+  a.rope = table.data;
   a.in_stride = qkv_row_stride;
   a.out_stride_q = q_row_stride;
   a.out_stride_k = k_row_stride;

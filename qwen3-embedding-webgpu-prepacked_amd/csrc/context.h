@@ -16,11 +16,12 @@ struct qattn_ctx {
   hipStream_t read_stream = nullptr;  // qattn_buffer_read_after's copies (waits on events only)
   void* scratch = nullptr;  // this device's copy of the static work-list array (qattn_prefill_static)
   // RoPE table of the producer, [positions][64] (cos, sin), built for `rope_theta`; grown when a
-  // longer sequence arrives (the reference builds one per plan, model.ts:76-83).
+  // longer sequence arrives (the reference builds one per plan, model.ts:76-83).  Under rope_mu.
   float2* rope = nullptr;
   int32_t rope_positions = 0;
   double rope_theta = 0.0;
-  std::string last_error;
+  std::mutex rope_mu;
+  std::string last_error;  // under mu
   std::mutex mu;
 };
 
@@ -60,8 +61,14 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // Host cu_seqlens: nseq in [1, QATTN_MAX_SEQS], cu[0] = 0, non-decreasing.
 int validate_cu(qattn_ctx* ctx, const int32_t* cu, int32_t nseq);
 
-// The context's RoPE table of at least `positions` positions, and the longest sequence of cu (api.hip).
-int rope_table(qattn_ctx* ctx, int32_t positions, double theta, const float2** out);
+// The context's RoPE table, held: another thread's call can free it (for a longer one) only after
+// `lock` is released.  Release it when the launch that reads the table is enqueued.
+struct RopeTable {
+  const float2* data = nullptr;
+  std::unique_lock<std::mutex> lock;
+};
+// A table of at least `positions` positions, and the longest sequence of cu (api.hip).
+int rope_table(qattn_ctx* ctx, int32_t positions, double theta, RopeTable* out);
 int32_t longest(const int32_t* cu, int32_t nseq);
 
 }  // namespace qattn

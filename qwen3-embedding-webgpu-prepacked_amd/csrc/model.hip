@@ -224,21 +224,27 @@ int enqueue_fused(qattn_model_plan* p, const int32_t* cu, int32_t nseq, float* o
   const auto done = [&]() {
     if (rec) rec->end();
   };
-  const float2* table = nullptr;
-  int rc = rope_table(ctx, longest(cu, nseq), d.rope_theta, &table);
-  if (rc) return rc;
+  const int32_t positions = longest(cu, nseq);
+  int rc = QATTN_OK;
   half_t *x = static_cast<half_t*>(p->x), *x_next = static_cast<half_t*>(p->x2);
   half_t* const delta = static_cast<half_t*>(p->delta);
   FusedQkv heads{static_cast<half_t*>(p->q), static_cast<half_t*>(p->k), static_cast<half_t*>(p->qkv), nullptr, nullptr,
-                 table, (float)d.eps, nseq, {}};
+                 nullptr, (float)d.eps, nseq, {}};
   std::copy(cu, cu + nseq + 1, heads.cu);
   for (int32_t l = 0; l < d.n_layers; ++l) {
     const qattn_layer_weights& w = m->layers[l];
     stage(QATTN_STAGE_QKV);
     heads.weight_q = w.attn_q_norm;
     heads.weight_k = w.attn_k_norm;
-    HIP_TRY(ctx, launch_q4_norm_qkv({x, l ? delta : nullptr, x_next, w.attn_norm, (float)d.eps, T},
-                                    static_cast<const uint8_t*>(w.attn_qkv), (uint32_t)qattn_q4_compact_bytes(kHidden, kQkvWidth), heads, stream));
+    {
+      RopeTable table;  // for this launch: between layers another thread may replace it
+      rc = rope_table(ctx, positions, d.rope_theta, &table);
+      if (rc) return rc;
+      heads.rope = table.data;
+      HIP_TRY(ctx, launch_q4_norm_qkv({x, l ? delta : nullptr, x_next, w.attn_norm, (float)d.eps, T},
+                                      static_cast<const uint8_t*>(w.attn_qkv),
+                                      (uint32_t)qattn_q4_compact_bytes(kHidden, kQkvWidth), heads, stream));
+    }
     if (l) std::swap(x, x_next);
     done();
     stage(QATTN_STAGE_ROPE_ATTENTION);

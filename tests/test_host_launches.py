@@ -6,6 +6,7 @@ import os
 import shutil
 import subprocess
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -53,7 +54,56 @@ def weight_ranges():
     return out
 
 
-CASES = {f.__name__: f for f in (weight_ranges,)}
+def _model(h, layers):
+    compact = lambda k, n: (1 << 30, h.qattn.lib().qattn_q4_compact_bytes(k, n))  # noqa: E731
+    layer = {"attn_qkv": compact(1024, 4096), "attn_output": compact(2048, 1024), "ffn_gate_up": compact(1024, 6144),
+             "ffn_down": compact(3072, 1024)}
+    layer.update({n: 1 << 20 for n in ("attn_norm", "attn_q_norm", "attn_k_norm", "ffn_norm")})
+    return h.ctx.model((1 << 24, 840 * 1000), 1 << 20, [layer] * layers)
+
+
+def rope_table_lifetime():
+    """{call: [the table that a launch was passed was freed before the launch returned]} while another
+    thread grows the context's table in the middle of each launch that reads it."""
+    out = {}
+    for call in ("fused forward", "forward", "qkv", "in place"):
+        h = Launches()
+        freed, threads, longest = [], [], [1100]
+        main = threading.get_ident()
+
+        def grow():
+            longest[0] += 100
+            h.ctx.qk_norm_rope(1 << 20, 512, 0, 4, np.array([0, longest[0]], np.int32))
+
+        def on(name, grid, block, args):
+            # FusedQkv (q, k, qkv, weight_q, weight_k, rope) or RopeArgs (in, out_q, out_k, weight_q, weight_k, rope)
+            index = 7 if "q4_fused_kernelILb1" in name else 0 if "qk_norm_rope" in name else None
+            if index is None or threading.get_ident() != main:
+                return
+            table = h.word(args, index, ctypes.c_uint64, 40)
+            threads.append(threading.Thread(target=grow))
+            threads[-1].start()
+            threads[-1].join(0.2)  # the other thread may have to wait for this launch
+            freed.append(bool(h.fake.fake_hip_freed(table)))
+
+        h.ctx.qk_norm_rope(1 << 20, 512, 0, 4, np.array([0, 1050], np.int32))
+        tokens = 20 if call == "fused forward" else 40
+        cu = np.array([0, tokens], np.int32)
+        plan = _model(h, 3).plan(64, 4) if "forward" in call else None
+        h.on = on
+        if plan:
+            plan.run(np.zeros(tokens, np.int32), cu, 1 << 22)
+        elif call == "qkv":
+            h.ctx.qk_norm_rope_qkv(1 << 20, 1 << 21, 1 << 22, cu)
+        else:
+            h.ctx.qk_norm_rope(1 << 20, 512, 0, 4, cu)
+        for t in threads:
+            t.join()
+        out[call] = freed
+    return out
+
+
+CASES = {f.__name__: f for f in (weight_ranges, rope_table_lifetime)}
 
 
 # ---- the tests --------------------------------------------------------------------------------
@@ -87,6 +137,15 @@ def test_weight_ranges_end_with_the_tensor(child):
     for m, k, n, name, used in launches:
         rows = 2 * 1088 if "ILb1E" in name else n
         assert used == -(-rows // 32) * 32 * (k // 32) * 20, (m, k, n, name)
+
+
+def test_rope_table_outlives_the_launches_that_read_it(child):
+    """One context serves several threads.  A call that needs a longer RoPE table frees the old one, which
+    waits for the launches already enqueued only: no launch may be passed a table that is freed before
+    the launch is enqueued, in a forward of several layers neither."""
+    freed = child("rope_table_lifetime")
+    assert [len(freed[c]) for c in ("fused forward", "forward", "qkv", "in place")] == [3, 3, 1, 1]
+    assert not any(sum(freed.values(), [])), freed
 
 
 if __name__ == "__main__":
