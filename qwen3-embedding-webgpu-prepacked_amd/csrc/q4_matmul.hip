@@ -1180,6 +1180,11 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
 //     at most two (N = 4096: M = 50 5.2, mid 8.5; M = 100 7.3 against 8.6);
 //   * up to 512 tiles of 64 x 128: q4_mid_kernel (N = 4096: M = 1,000 14.7, 256 x 128 tiles 17.0;
 //     M = 1,500, 768 tiles, 19.6 against 18.1);
+//   * beyond, the rows a tile pads count: up to 64 rows stay with q4_mid_kernel (N = 70,016: M = 64 18.8,
+//     256 x 128 tiles 37.6), and 128 x 128 tiles serve where they pad at least a quarter fewer rows, up to
+//     128 and 257 to 384 (M = 100 26.8 against 39.0, M = 300 65 against 76; M = 500, 640 against 768 rows,
+//     86 against 77), unless 256 x 128 tiles fit in one round, of one per CU or of two where 128 x 128 ones do
+//     not (M = 300: N = 16,000 18.8 against 19.5, N = 24,000 26.9 against 27.7);
 //   * then 256 x 128 tiles while they are at most one per CU (N = 6144: M = 1,000 18.2, 256 x 256
 //     tiles 26.5);
 //   * then 256 x 256 tiles where their last round of 256 is mostly full (N = 4096: M = 2,400 27.5
@@ -1192,6 +1197,8 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
 //   * q4_direct_kernel up to kQ4DirectBlocks (K = 3072, M = 500 16.5, mid 17.5);
 //   * up to 256 tiles of 64 x 128: q4_mid_kernel, a group per chunk (K = 2048, M = 1,419 13.2, 128 x 128
 //     tiles 19.8; K = 3072 18.4);
+//   * up to 128 rows and beyond 256 tiles of 128 x 128, folding q4_mid_kernel (N = 40,000, M = 100: K = 2048 33.2, 128 x 128
+//     tiles 38.9; K = 3072 47.6 against 50.6);
 //   * K up to 2048: 128 x 128 tiles while at most one per CU (M = 2,400 20.3, mid 25.4, 256 x 128 27.6),
 //     then 256 x 128 or 128 x 128 tiles by the rounds each needs (M = 8,000: one round of 38.8 against two
 //     of 22.7);
@@ -1207,6 +1214,7 @@ hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t
                      _Float16* y, int64_t ldy, hipStream_t stream) {
   const int n_out = SWIGLU ? N / 2 : N, chunks = q4_chunks(K);
   const auto tiles = [&](int tm, int tn) { return (int64_t)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
+  const auto padded = [&](int tm) { return (int64_t)((M + tm - 1) / tm) * tm; };
   const auto rounds = [](int64_t t) { return (t + 255) / 256; };
 #define Q4_TILE(...) launch_q4_tile<SWIGLU, __VA_ARGS__>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream)
 #define Q4_MID(...) launch_q4_mid<SWIGLU, __VA_ARGS__>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream)
@@ -1216,8 +1224,11 @@ hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t
       launch_q4_small<SWIGLU, 1, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if (tiles(32, 32) <= 512)
       launch_q4_small<SWIGLU, 2, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
-    else if (tiles(64, 128) <= 512)
+    else if (tiles(64, 128) <= 512 || M <= 64)
       Q4_MID(1);
+    else if (4 * padded(128) <= 3 * padded(256) && tiles(256, 128) > 256 &&
+             (tiles(128, 128) <= 512 || tiles(256, 128) > 512))
+      Q4_TILE(4, 2, 1);
     else if (tiles(256, 128) <= 256 || (t > 256 && 256 * rounds(t) * 100 > 115 * t))
       Q4_TILE(8, 2, 1);
     else
@@ -1234,6 +1245,8 @@ hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t
       Q4_MID(2);
     else if (chunks == 3 && tiles(64, 128) <= 256)
       Q4_MID(3);
+    else if (M <= 128 && small > 1)
+      Q4_MID(1, true);
     else if (chunks == 3 && small == 1)
       Q4_TILE(4, 2, 3);
     else if (chunks > 3 && tiles(64, 128) <= 512)

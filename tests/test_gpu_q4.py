@@ -272,3 +272,29 @@ def test_q4_sums_restart_every_1024_columns(ctx, m, k):
     expected = np.zeros((m, n))
     expected[:, 0::2] = np.where(np.arange(m) % 2, -1.0, 1.0)[:, None] * (32 * last - 1024)
     assert np.array_equal(y, expected)
+
+
+# (m, k, n, swiglu): wide outputs, whose launches go by the rows that a tile would pad
+WIDE_CASES = [(64, 96, 65600, False), (40, 32, 65664, True), (65, 160, 40000, False), (128, 64, 65600, True),
+              (257, 1024, 20000, False), (384, 32, 33000, False), (300, 64, 33024, True),
+              (50, 1056, 33100, False), (128, 1120, 33000, False), (100, 2080, 33024, True)]
+
+
+@pytest.mark.parametrize("m,k,n,swiglu", WIDE_CASES)
+def test_q4_wide_launches_equal_their_columns_alone(ctx, m, k, n, swiglu):
+    """A projection to many columns against launches over 128 weight rows of it (64 gate and 64 up rows),
+    which take the kernels for small outputs: equal bit for bit."""
+    rng = np.random.default_rng(m + k + n)
+    packed = random_compact(rng, n, k)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    tiles = packed.reshape(-(-n // 32), -1)
+    cols = n // 2 if swiglu else n
+    whole = (run_q4_swiglu(ctx, x, packed, k, cols) if swiglu else run_q4(ctx, x, packed, k, n))[:, :cols]
+    for c in (0, cols // 64 // 2 * 64, (cols - 1) // 64 * 64):
+        if swiglu:
+            part = np.concatenate([tiles[c // 32:c // 32 + 2], tiles[(cols + c) // 32:(cols + c) // 32 + 2]])
+            alone, width = run_q4_swiglu(ctx, x, part.reshape(-1), k, 64), 64
+        else:
+            width = min(128, n - c)
+            alone = run_q4(ctx, x, tiles[c // 32:c // 32 + 4].reshape(-1), k, width)
+        assert np.array_equal(whole[:, c:c + width].view(np.uint16), alone[:, :width].view(np.uint16)), c

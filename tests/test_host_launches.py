@@ -3,6 +3,7 @@
 import ctypes
 import json
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -51,6 +52,26 @@ def weight_ranges():
         need = h.qattn.lib().qattn_q4_compact_bytes(k, n)
         h.ctx.q4_matmul(1 << 20, m, k, 1 << 30, need + 5 * 640, n, 1 << 40)
         h.ctx.q4_matmul_swiglu(1 << 20, m, k, 1 << 30, h.qattn.lib().qattn_q4_compact_bytes(k, 2 * 1088) + 4, 1088, 1 << 40)
+    return out
+
+
+def tile_heights():
+    """[(m, k, n, swiglu, rows of the kernel's output tile)] of projections to wide outputs."""
+    h, out = Launches(), []
+    for m in (1, 33, 64, 65, 100, 128, 129, 256, 257, 300, 384, 385, 500):
+        for k in (1024, 2048, 3072, 4096):
+            for n in (33024, 70016, 151680):
+                for swiglu in (False, True):
+                    def on(name, grid, block, args):
+                        kind, first = re.match(r"_ZN5qattn\d+q4_(\w+?)_kernelILb[01]EL[ib](\d+)E", name).groups()
+                        rows = {"tile": 32 * int(first), "mid": 64, "small": 16 * int(first), "direct": 32}[kind]
+                        out.append((m, k, n, swiglu, rows))
+                    h.on = on
+                    need = h.qattn.lib().qattn_q4_compact_bytes(k, n)
+                    if swiglu:
+                        h.ctx.q4_matmul_swiglu(1 << 20, m, k, 1 << 30, need, n // 2, 1 << 40)
+                    else:
+                        h.ctx.q4_matmul(1 << 20, m, k, 1 << 30, need, n, 1 << 40)
     return out
 
 
@@ -103,7 +124,7 @@ def rope_table_lifetime():
     return out
 
 
-CASES = {f.__name__: f for f in (weight_ranges, rope_table_lifetime)}
+CASES = {f.__name__: f for f in (weight_ranges, tile_heights, rope_table_lifetime)}
 
 
 # ---- the tests --------------------------------------------------------------------------------
@@ -137,6 +158,15 @@ def test_weight_ranges_end_with_the_tensor(child):
     for m, k, n, name, used in launches:
         rows = 2 * 1088 if "ILb1E" in name else n
         assert used == -(-rows // 32) * 32 * (k // 32) * 20, (m, k, n, name)
+
+
+def test_wide_projections_of_few_rows_take_short_tiles(child):
+    """However many tiles a wide weight makes, a launch of a few rows does not pay for tiles much taller
+    than them."""
+    launches = child("tile_heights")
+    assert len(launches) == 13 * 4 * 3 * 2
+    for m, k, n, swiglu, rows in launches:
+        assert rows <= (64 if m <= 64 else 128 if m <= 128 or (256 < m <= 384 and k <= 1024) else 256), (m, k, n, rows)
 
 
 def test_rope_table_outlives_the_launches_that_read_it(child):
