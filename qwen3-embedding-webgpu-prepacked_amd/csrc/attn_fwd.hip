@@ -778,15 +778,17 @@ __global__ void debug_mask_kernel(int S, MaskSpec mask, uint32_t* bits, int word
 hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t stream) {
   if (p.n_slots <= 0) return hipSuccess;
   // Plans without split items run the variant without the partial-result path (fewer live
-  // registers in the tile loop).
+  // registers in the tile loop).  The timeline and the mask check take the same one (but for LAST).
   const dim3 grid(p.n_slots), block(kThreads);
   if (p.timeline) {
     if (p.n_splits > 0) hipLaunchKernelGGL((attn_fwd_kernel<true, false, false, true>), grid, block, 0, stream, p);
+    else if (p.one_entry) hipLaunchKernelGGL((attn_fwd_kernel<false, false, false, true, true>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((attn_fwd_kernel<false, false, false, true>), grid, block, 0, stream, p);
     return hipGetLastError();
   }
   if (p.maskbits) {
     if (p.n_splits > 0) hipLaunchKernelGGL((attn_fwd_kernel<true, false, true>), grid, block, 0, stream, p);
+    else if (p.one_entry) hipLaunchKernelGGL((attn_fwd_kernel<false, false, true, false, true>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((attn_fwd_kernel<false, false, true>), grid, block, 0, stream, p);
     return hipGetLastError();
   }

@@ -23,6 +23,7 @@ def _ticks(row, t0):
     ([500] * 16, 0, 0),                   # the 16x500 headline packing, unsplit
     ([5000], 1, 0),                       # 1x5000 sparse: split items + merge kernel
     ([700, 1, 33, 1500, 64, 65], 1, 1),   # ragged, batch-invariant
+    ([150, 1, 65], 1, 1),                 # one entry per slot
 ])
 def test_timeline_variant_matches_encode_and_orders_its_stamps(ctx, qattn, lengths, mask, flags):
     cu = cu_of(lengths)

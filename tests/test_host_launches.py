@@ -75,6 +75,24 @@ def tile_heights():
     return out
 
 
+def attention_variants():
+    """{lengths: {launch: [split, one entry]}}, from the kernel's template arguments."""
+    h, out = Launches(), {}
+    for lengths, flags in (([50], 1), ([10, 150, 64], 1), ([500] * 16, 0), ([5000], 0)):
+        names = []
+        h.on = lambda name, *rest: names.append(re.match(r"_ZN5qattn15attn_fwd_kernelI((?:Lb[01]E)+)E", name))
+        run = h.ctx.run(h.qattn.make_desc(1 << 20, 1 << 30, 1 << 31, 1 << 32, np.cumsum([0] + lengths), flags=flags))
+        seen = {}
+        for launch in (run.encode, run.mask_bits, run.timeline):
+            names.clear()
+            launch()
+            bools = [m for m in names if m][0].group(1)
+            seen[launch.__name__] = [bools[2] == "1", bools[18] == "1"]
+        run.destroy()
+        out[",".join(map(str, lengths))] = seen
+    return out
+
+
 def _model(h, layers):
     compact = lambda k, n: (1 << 30, h.qattn.lib().qattn_q4_compact_bytes(k, n))  # noqa: E731
     layer = {"attn_qkv": compact(1024, 4096), "attn_output": compact(2048, 1024), "ffn_gate_up": compact(1024, 6144),
@@ -124,7 +142,7 @@ def rope_table_lifetime():
     return out
 
 
-CASES = {f.__name__: f for f in (weight_ranges, tile_heights, rope_table_lifetime)}
+CASES = {f.__name__: f for f in (weight_ranges, tile_heights, attention_variants, rope_table_lifetime)}
 
 
 # ---- the tests --------------------------------------------------------------------------------
@@ -167,6 +185,14 @@ def test_wide_projections_of_few_rows_take_short_tiles(child):
     assert len(launches) == 13 * 4 * 3 * 2
     for m, k, n, swiglu, rows in launches:
         assert rows <= (64 if m <= 64 else 128 if m <= 128 or (256 < m <= 384 and k <= 1024) else 256), (m, k, n, rows)
+
+
+def test_mask_check_and_timeline_run_the_variant_that_a_launch_runs(child):
+    """The executed mask and the phase stamps are those of the kernel that the run's launches take."""
+    seen = child("attention_variants")
+    assert {tuple(v["encode"]) for v in seen.values()} == {(False, True), (False, False), (True, False)}
+    for lengths, v in seen.items():
+        assert v["mask_bits"] == v["encode"] and v["timeline"] == v["encode"], (lengths, v)
 
 
 def test_rope_table_outlives_the_launches_that_read_it(child):
