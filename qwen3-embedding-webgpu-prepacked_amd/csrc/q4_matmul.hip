@@ -1179,7 +1179,9 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
 //   * q4_small_kernel while its 16-row blocks are at most one per CU, with 32-row blocks while those are
 //     at most two (N = 4096: M = 50 5.2, mid 8.5; M = 100 7.3 against 8.6);
 //   * up to 512 tiles of 64 x 128: q4_mid_kernel (N = 4096: M = 1,000 14.7, 256 x 128 tiles 17.0;
-//     M = 1,500, 768 tiles, 19.6 against 18.1);
+//     M = 1,500, 768 tiles, 19.6 against 18.1).  It works in passes of eight K blocks, so for K up to 256 only
+//     up to 256 tiles, and 128 x 128 tiles beyond (N = 1024, K = 64, M = 3,000 5.2 against 6.8), also in
+//     place of 256 x 128 ones that fill a gap (M = 20,000 14.2 against 15.6);
 //   * beyond, the rows a tile pads count: up to 64 rows stay with q4_mid_kernel (N = 70,016: M = 64 18.8,
 //     256 x 128 tiles 37.6), and 128 x 128 tiles serve where they pad at least a quarter fewer rows, up to
 //     128 and 257 to 384 (M = 100 26.8 against 39.0, M = 300 65 against 76; M = 500, 640 against 768 rows,
@@ -1204,11 +1206,14 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
 //     of 22.7);
 //   * K up to 3072: 128 x 128 tiles with three groups while at most one per CU (M = 4,000 31.9; mid 37.1,
 //     128 x 256 folding 49.5); beyond, three groups of larger tiles do not fit in LDS;
-//   * K above 3072: folding q4_mid_kernel up to 512 tiles, two workgroups per CU (K = 4096, M = 4,000 47.2,
+//   * groups run as long as a whole chunk, so where the last chunk is at most half full the chunks are folded
+//     instead (K = 1536: M = 1,419 12.5 against 13.6, M = 8,000 33.7 against 36.9; K = 1792, M = 5,000 30.2
+//     against 29.5), and so is K above 3072: folding q4_mid_kernel up to 512 tiles, two workgroups per CU (K = 4096, M = 4,000 47.2,
 //     128 x 256 tiles 64.4; M = 5,000, 632 tiles, 66.1 against 64.8);
 //   * the rest folds the chunks in 128 x 256 tiles where their last round of 256 is mostly full (K = 3072,
 //     M = 8,000 55 against 61 with 128 x 128 tiles, M = 16,000 114 against 120), else in 128 x 128 tiles, whose
-//     second workgroup per CU fills the gap (M = 12,000, 1.5 rounds, 92 against 106).
+//     second workgroup per CU fills the gap (M = 12,000, 1.5 rounds, 92 against 106; K = 1792 57 against 68
+//     with two groups, which at K = 2048, both chunks full, take the same 66).
 template <bool SWIGLU>
 hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t* w, uint32_t w_bytes, int N,
                      _Float16* y, int64_t ldy, hipStream_t stream) {
@@ -1220,20 +1225,24 @@ hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t
 #define Q4_MID(...) launch_q4_mid<SWIGLU, __VA_ARGS__>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream)
   if (chunks == 1) {
     const int64_t t = tiles(256, 256);
+    const bool partial = t > 256 && 256 * rounds(t) * 100 > 115 * t, shallow = K <= 256;
     if (tiles(16, 32) <= 256)
       launch_q4_small<SWIGLU, 1, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if (tiles(32, 32) <= 512)
       launch_q4_small<SWIGLU, 2, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
-    else if (tiles(64, 128) <= 512 || M <= 64)
+    else if (tiles(64, 128) <= (shallow ? 256 : 512) || M <= 64)
       Q4_MID(1);
+    else if (shallow && (tiles(64, 128) <= 512 || partial))
+      Q4_TILE(4, 2, 1);
     else if (4 * padded(128) <= 3 * padded(256) && tiles(256, 128) > 256 &&
              (tiles(128, 128) <= 512 || tiles(256, 128) > 512))
       Q4_TILE(4, 2, 1);
-    else if (tiles(256, 128) <= 256 || (t > 256 && 256 * rounds(t) * 100 > 115 * t))
+    else if (tiles(256, 128) <= 256 || partial)
       Q4_TILE(8, 2, 1);
     else
       Q4_TILE(8, 4, 1);
   } else {
+    const bool fold = chunks > 3 || K - 32 * kQ4Chunk * (chunks - 1) <= 512;
     const int64_t big = rounds(tiles(256, 128)), small = rounds(tiles(128, 128)), wide = tiles(128, 256);
     if (tiles(16, 16) <= 256 && chunks <= kQ4SmallChunks && !SWIGLU)
       launch_q4_small<SWIGLU, 1, SWIGLU ? 2 : 1>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
@@ -1241,19 +1250,19 @@ hipError_t launch_q4(const _Float16* x, int64_t ldx, int M, int K, const uint8_t
       launch_q4_small<SWIGLU, 1, 2>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
     else if ((int64_t)((M + 31) / 32) * ((n_out + 31) / 32) <= kQ4DirectBlocks)
       launch_q4_direct<SWIGLU>(x, ldx, M, K, w, w_bytes, N, y, ldy, stream);
-    else if (chunks == 2 && tiles(64, 128) <= 256)
+    else if (!fold && chunks == 2 && tiles(64, 128) <= 256)
       Q4_MID(2);
-    else if (chunks == 3 && tiles(64, 128) <= 256)
+    else if (!fold && tiles(64, 128) <= 256)
       Q4_MID(3);
     else if (M <= 128 && small > 1)
       Q4_MID(1, true);
-    else if (chunks == 3 && small == 1)
+    else if (!fold && chunks == 3 && small == 1)
       Q4_TILE(4, 2, 3);
-    else if (chunks > 3 && tiles(64, 128) <= 512)
+    else if (fold && tiles(64, 128) <= 512)
       Q4_MID(1, true);
-    else if (chunks > 2 && wide > 256 && 256 * rounds(wide) * 100 > 115 * wide)
+    else if (K != 64 * kQ4Chunk && wide > 256 && 256 * rounds(wide) * 100 > 115 * wide)
       Q4_TILE(4, 2, 1, true);
-    else if (chunks > 2)
+    else if (fold || chunks == 3)
       Q4_TILE(4, 4, 1, true);
     else if (small > 1 && 5 * big <= 3 * small)
       Q4_TILE(8, 2, 2);

@@ -75,6 +75,20 @@ def tile_heights():
     return out
 
 
+def k_blocks():
+    """[(m, k, K blocks that the kernel computes)] of projections whose K is no multiple of 1,024."""
+    h, out = Launches(), []
+    for m in (1419, 3000, 8000, 20000):
+        for k in (32, 64, 128, 256, 1056, 1280, 1536, 2080, 2560):
+            def on(name, grid, block, args):
+                kind, ints, fold = re.match(r"_ZN5qattn\d+q4_(\w+?)_kernelILb0E((?:Li\d+E)+)Lb([01])E", name).groups()
+                groups, step = int(re.findall(r"\d+", ints)[-1]), 8 if kind == "mid" else 4
+                out.append((m, k, grid, groups * 32 if groups > 1 else -(-(k // 32) // step) * step))
+            h.on = on
+            h.ctx.q4_matmul(1 << 20, m, k, 1 << 30, h.qattn.lib().qattn_q4_compact_bytes(k, 1024), 1024, 1 << 40)
+    return out
+
+
 def attention_variants():
     """{lengths: {launch: [split, one entry]}}, from the kernel's template arguments."""
     h, out = Launches(), {}
@@ -142,7 +156,7 @@ def rope_table_lifetime():
     return out
 
 
-CASES = {f.__name__: f for f in (weight_ranges, tile_heights, attention_variants, rope_table_lifetime)}
+CASES = {f.__name__: f for f in (weight_ranges, tile_heights, k_blocks, attention_variants, rope_table_lifetime)}
 
 
 # ---- the tests --------------------------------------------------------------------------------
@@ -185,6 +199,16 @@ def test_wide_projections_of_few_rows_take_short_tiles(child):
     assert len(launches) == 13 * 4 * 3 * 2
     for m, k, n, swiglu, rows in launches:
         assert rows <= (64 if m <= 64 else 128 if m <= 128 or (256 < m <= 384 and k <= 1024) else 256), (m, k, n, rows)
+
+
+def test_launches_that_fill_the_chip_do_not_pad_k(child):
+    """Groups that each run a chunk of K, and kernels that step by eight K blocks, compute blocks past K: no
+    launch of more than one workgroup per CU computes a third more than it has (or four blocks)."""
+    launches = child("k_blocks")
+    assert len(launches) == 4 * 9
+    for m, k, grid, blocks in launches:
+        assert grid <= 256 or blocks <= max(4, 4 * (k // 32) // 3), (m, k, grid, blocks)
+        assert k < 1024 or blocks <= 4 * (k // 32) / 3, (m, k, grid, blocks)
 
 
 def test_mask_check_and_timeline_run_the_variant_that_a_launch_runs(child):
