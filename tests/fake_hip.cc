@@ -40,6 +40,10 @@ bool inside(const std::map<uintptr_t, size_t>& m, uintptr_t p) {
 
 extern "C" {
 void fake_hip_hook(hook_t h) { hook = h; }
+// Calls `each` with the name of every kernel of the libraries loaded.
+void fake_hip_kernels(void (*each)(const char*)) {
+  for (const auto& k : names()) each(k.second.c_str());
+}
 int fake_hip_freed(uint64_t p) {
   std::lock_guard<std::mutex> lock(mu);
   return inside(freed, (uintptr_t)p) && !inside(live, (uintptr_t)p);

@@ -216,6 +216,31 @@ def test_fused_small_forward_equals_the_packed_forward(ctx, weights, lengths):
         m.free()
 
 
+@pytest.mark.parametrize("nseq", [63, 64, 65])
+def test_fused_small_forward_at_its_sequence_limit(ctx, weights, nseq):
+    """Up to 64 sequences (a ballot over the wavefront's lanes finds a token's) take the fused projections,
+    65 the separate launches: 31 tokens in runs of 1 to 3 among empty sequences, the last one full,
+    against the same requests packed with one more."""
+    m = DeviceModel(ctx, weights, flags=1)
+    rng = np.random.default_rng(nseq)
+    lengths = np.zeros(nseq, np.int64)
+    filled = np.sort(rng.choice(nseq - 1, 14, replace=False))
+    lengths[filled] = [1, 3, 2, 1, 2, 3, 1, 1, 2, 3, 2, 1, 3, 3]
+    lengths[-1] = 3
+    ids = rng.integers(0, weights["vocab"], int(lengths.sum())).astype(np.int32)
+    more = rng.integers(0, weights["vocab"], 40).astype(np.int32)
+    cu = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    try:
+        small = _run(ctx, m, ids, cu, max_tokens=100, max_seqs=66)
+        packed = _run(ctx, m, np.concatenate([ids, more]), np.append(cu, cu[-1] + 40).astype(np.int32), max_tokens=100,
+                      max_seqs=66)
+        keep = np.flatnonzero(lengths)
+        assert np.array_equal(small[keep].view(np.uint32), packed[:-1][keep].view(np.uint32))
+        _check_embeddings(small[keep], mr.forward(weights, ids, cu)[keep])
+    finally:
+        m.free()
+
+
 def test_model_plan_reuse_and_rejects(ctx, qattn, weights, dmodel):
     rng = np.random.default_rng(9)
     plan = dmodel.model.plan(400, 4)

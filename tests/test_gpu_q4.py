@@ -219,10 +219,20 @@ TILE_CASES = [
 ]
 
 
-@pytest.mark.parametrize("m,k,n,swiglu", TILE_CASES)
+# K above 1024 in every way to run its chunks: a group per chunk, or folded in one.
+TALL_CASES = [
+    (64, 2048, 10240, True), (65, 3072, 1000, False),
+    (1500, 2048, 1000, False), (320, 2048, 6144, True), (600, 2048, 6144, True), (4200, 2048, 1000, False),  # two chunks
+    (1500, 3072, 1000, False), (320, 3072, 6144, True), (2200, 3072, 1024, False), (600, 3072, 6144, True),  # three
+    (8300, 1088, 1000, False), (1400, 2080, 6144, True), (1200, 3072, 6144, True),  # folded
+]
+
+
+@pytest.mark.parametrize("m,k,n,swiglu", TILE_CASES + TALL_CASES)
 def test_q4_tiled_launches_equal_small_launches_bit_for_bit(ctx, m, k, n, swiglu):
-    """All rows of a launch against the same rows in launches of at most 32, which take the kernel
-    for the smallest launches (itself checked against the oracle above): equal bit for bit."""
+    """All rows of a launch against the same rows in launches of at most 32, which take the kernels
+    for small launches (themselves checked against the oracle): equal bit for bit.  Where both are the
+    same kernel (at most 33 to 64 rows) this holds only that a row does not depend on its place."""
     rng = np.random.default_rng(m + k + n)
     packed = random_compact(rng, n, k)
     x = rng.standard_normal((m, k)).astype(np.float16)
@@ -298,3 +308,47 @@ def test_q4_wide_launches_equal_their_columns_alone(ctx, m, k, n, swiglu):
             width = min(128, n - c)
             alone = run_q4(ctx, x, tiles[c // 32:c // 32 + 4].reshape(-1), k, width)
         assert np.array_equal(whole[:, c:c + width].view(np.uint16), alone[:, :width].view(np.uint16)), c
+
+
+@pytest.mark.parametrize("m,k,n", [(40, 4096, 9), (33, 4096, 1400), (33, 4160, 96), (9, 8192, 200), (40, 8224, 64)])
+def test_q4_long_k_matches_oracle(ctx, oracle, m, k, n):
+    """The kernels of small launches with more than three chunks of K, which other launches are compared with."""
+    rng = np.random.default_rng(m + k + n)
+    packed = random_compact(rng, n, k)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    check(oracle, run_q4(ctx, x, packed, k, n), x, packed, k, n, f"q4 {m}x{k}x{n}")
+
+
+@pytest.mark.parametrize("m,k,n_inter", [(40, 2048, 192), (17, 3072, 192), (40, 4096, 192), (5, 4160, 128)])
+def test_q4_long_k_swiglu_equals_the_two_launches(ctx, oracle, m, k, n_inter):
+    test_q4_matmul_swiglu_equals_the_two_launches(ctx, oracle, m, k, n_inter)
+
+
+# One case for every kernel and way to run the chunks of K, ragged in M and N.
+STRIDED_CASES = [(50, 1024, 1500), (70, 992, 4090), (150, 96, 6001), (1025, 1024, 4091), (500, 160, 12301), (2100, 64, 1021),
+                 (2100, 1024, 4090), (50, 2048, 1001), (65, 3072, 1003), (300, 2048, 1021), (1500, 2048, 1001),
+                 (2100, 2048, 1021), (4200, 2048, 1000), (1500, 3072, 1019), (2200, 3072, 1020), (1900, 1056, 517),
+                 (4200, 3072, 1005), (8300, 1088, 1001), (50, 3072, 1001), (40, 4096, 100), (65, 2048, 1001),
+                 (33, 4096, 1401), (150, 3072, 1021)]
+
+
+@pytest.mark.parametrize("m,k,n", STRIDED_CASES)
+def test_q4_strided_rows_equal_compact_ones(ctx, m, k, n):
+    """x rows inside a wider matrix (NaN between them, nothing after the last one's K columns but NaN) and y
+    rows inside a wider one: the same bits, and no column past N written."""
+    rng = np.random.default_rng(m + k + n)
+    packed = random_compact(rng, n, k)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    compact = run_q4(ctx, x, packed, k, n)
+    ldx, ldy = k + 40, -(-n // 8) * 8 + 24
+    wide = np.full((m + 1, ldx), np.nan, np.float16)
+    wide[:m, :k] = x
+    bx, bw, by = ctx.upload(wide.view(np.uint16)), ctx.upload(packed), ctx.alloc((m + 1) * ldy * 2)
+    by.fill_u16(0x7E01)
+    ctx.q4_matmul(bx.ptr, m, k, bw.ptr, packed.size, n, by.ptr, ldx=ldx, ldy=ldy)
+    ctx.synchronize()
+    y = by.read(np.uint16, (m + 1, ldy))
+    for b in (bx, bw, by):
+        b.free()
+    assert np.array_equal(y[:m, :n], compact[:, :n].view(np.uint16))
+    assert (y[:, n:] == 0x7E01).all() and (y[m] == 0x7E01).all()

@@ -89,6 +89,34 @@ def k_blocks():
     return out
 
 
+def kernel_coverage():
+    """The Q4_0 GEMM kernels of the library, and those that the bit-equality cases of test_gpu_q4.py launch
+    (the whole launch and the small one it is compared with) and its strided cases:
+    [[all], [[case, kernel, reference]], [strided]]."""
+    import test_gpu_q4 as cases
+    h, kernels, out, seen = Launches(), [], [], []
+    each = ctypes.CFUNCTYPE(None, ctypes.c_char_p)(lambda name: kernels.append(name.decode()))
+    h.fake.fake_hip_kernels(each)
+    h.on = lambda name, *rest: seen.append(name)
+
+    def launch(m, k, n, swiglu):
+        need = h.qattn.lib().qattn_q4_compact_bytes(k, n)
+        if swiglu:
+            h.ctx.q4_matmul_swiglu(1 << 20, m, k, 1 << 30, need, n // 2, 1 << 40)
+        else:
+            h.ctx.q4_matmul(1 << 20, m, k, 1 << 30, need, n, 1 << 40, ldy=-(-n // 8) * 8)
+        return seen[-1]
+
+    for m, k, n, swiglu in cases.TILE_CASES + cases.TALL_CASES:
+        out.append(((m, k, n, swiglu), launch(m, k, n, swiglu), launch(min(m, 32), k, n, swiglu)))
+    for m, k, n_inter in ((40, 4096, 192),):  # test_q4_long_k_swiglu_equals_the_two_launches
+        out.append(((m, k, 2 * n_inter, True), "", launch(m, k, 2 * n_inter, True)))
+    strided = [launch(m, k, n, False) for m, k, n in cases.STRIDED_CASES]
+    for m, k, n, swiglu in cases.WIDE_CASES:
+        out.append(((m, k, n, swiglu), launch(m, k, n, swiglu), launch(m, k, 128, swiglu)))
+    return [[k for k in kernels if re.search(r"q4_(tile|mid|direct|small)_kernel", k)], out, strided]
+
+
 def attention_variants():
     """{lengths: {launch: [split, one entry]}}, from the kernel's template arguments."""
     h, out = Launches(), {}
@@ -113,6 +141,20 @@ def _model(h, layers):
              "ffn_down": compact(3072, 1024)}
     layer.update({n: 1 << 20 for n in ("attn_norm", "attn_q_norm", "attn_k_norm", "ffn_norm")})
     return h.ctx.model((1 << 24, 840 * 1000), 1 << 20, [layer] * layers)
+
+
+def fused_routes():
+    """[(tokens, sequences, whether the forward takes the fused projections)]."""
+    h, out, names = Launches(), [], []
+    plan = _model(h, 1).plan(64, 70)
+    h.on = lambda name, *rest: names.append(name)
+    for tokens, nseq in ((1, 1), (32, 1), (33, 1), (32, 64), (32, 65), (31, 70)):
+        cu = np.minimum(np.arange(nseq + 1), tokens).astype(np.int32)
+        cu[-1] = tokens
+        names.clear()
+        plan.run(np.zeros(tokens, np.int32), cu, 1 << 22)
+        out.append((tokens, nseq, any("q4_fused" in n for n in names)))
+    return out
 
 
 def rope_table_lifetime():
@@ -156,7 +198,8 @@ def rope_table_lifetime():
     return out
 
 
-CASES = {f.__name__: f for f in (weight_ranges, tile_heights, k_blocks, attention_variants, rope_table_lifetime)}
+CASES = {f.__name__: f for f in (weight_ranges, tile_heights, k_blocks, kernel_coverage, attention_variants, fused_routes,
+                                rope_table_lifetime)}
 
 
 # ---- the tests --------------------------------------------------------------------------------
@@ -211,12 +254,26 @@ def test_launches_that_fill_the_chip_do_not_pad_k(child):
         assert k < 1024 or blocks <= 4 * (k // 32) / 3, (m, k, grid, blocks)
 
 
+def test_every_projection_kernel_is_compared_with_another(child):
+    """The library holds no GEMM kernel that nothing launches, and the GPU tests compare each with another
+    kernel's rows, bit for bit (or are that other kernel, which the oracle checks)."""
+    kernels, cases, strided = child("kernel_coverage")
+    reached = {whole for _, whole, other in cases if whole != other} | {other for *_, other in cases}
+    assert len(kernels) > 20 and sorted(set(kernels) - reached) == []
+    assert sorted({k for k in kernels if "ILb0E" in k} - set(strided)) == []
+
+
 def test_mask_check_and_timeline_run_the_variant_that_a_launch_runs(child):
     """The executed mask and the phase stamps are those of the kernel that the run's launches take."""
     seen = child("attention_variants")
     assert {tuple(v["encode"]) for v in seen.values()} == {(False, True), (False, False), (True, False)}
     for lengths, v in seen.items():
         assert v["mask_bits"] == v["encode"] and v["timeline"] == v["encode"], (lengths, v)
+
+
+def test_fused_forward_limits(child):
+    for tokens, nseq, fused in child("fused_routes"):
+        assert fused == (tokens <= 32 and nseq <= 64), (tokens, nseq)
 
 
 def test_rope_table_outlives_the_launches_that_read_it(child):
