@@ -866,6 +866,7 @@ int check_q4_args(qattn_ctx* ctx, const void* x, int64_t ldx, int32_t M, int32_t
   if (w_bytes < need || w_bytes > 0x7FFFFFFFll)
     return fail(ctx, QATTN_EINVAL, "w_bytes %lld: a %dx%d tile32-compact tensor holds %lld bytes (< 2 GiB)",
                 (long long)w_bytes, N, K, (long long)need);
+  // 128 spare rows of x: the kernels' tiles overhang M by up to 255 rows, whose offsets then stay below 2^32.
   if (((int64_t)M + 128) * ldx * 2 > 0x7FFFFFFFll || (int64_t)M * ldy * 2 > 0x7FFFFFFFll)
     return fail(ctx, QATTN_EINVAL, "x or y rows beyond 2 GiB (32-bit buffer offsets)");
   if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(y) % 16 || reinterpret_cast<uintptr_t>(w) % 4)
