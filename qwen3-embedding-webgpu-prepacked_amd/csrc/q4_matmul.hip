@@ -142,8 +142,10 @@ __device__ inline void q4_barrier() {
 // after the barrier they filled the texture unit's queue and stalled the MFMAs behind them (70.5 ->
 // 68.1 us).  Not kept: weights dequantised into registers at this size (VALU power: 73 us), four
 // wavefronts of 128 x 128 (one per SIMD cannot issue the dequantisation beside its MFMAs: 65 us).
+// The folding 128 x 256 tile spreads its loads and dequantising the same way (8000 x 3072 -> 1024 57.9 ->
+// 54.1 us); its 64 x 64 wavefronts leave registers for the second set of accumulators.
 // Measured (us, before -> after): 8000 x 1024 -> 4096 80.4 -> 65.5; 20000 x 1024 -> 6144 with SwiGLU
-// 292 -> 254; 8000 x 2048 -> 1024 44.8 -> 38.8; 8000 x 3072 -> 1024, folding in 128 x 256, 66.7 -> 55.5.
+// 292 -> 254; 8000 x 2048 -> 1024 44.8 -> 38.8; 8000 x 3072 -> 1024 66.7 -> 54.1.
 //
 // Step kb (X tile and weight tile kb in LDS; the first half's fragments in registers): half 1 reads
 // the other row fragments, dequantises weight tile kb + 1 into the free B buffer and runs the first
@@ -265,6 +267,18 @@ __global__ __launch_bounds__(128 * NWN * G, 2) void q4_tile_kernel(
     load_a(a_new, kb + 3, 0, A1);
     store_b(b_nxt, w_use);
     mma(b_cur, a_lo, 0);
+    if constexpr (FOLD && NWN == 4) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+#pragma unroll
+      for (int j = 0; j < 6; ++j) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    }
     if constexpr (MF == 8) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
@@ -287,6 +301,17 @@ __global__ __launch_bounds__(128 * NWN * G, 2) void q4_tile_kernel(
     load_a(a_new, kb + 3, A1, A2);
     load_wq(w_new, kb + 3);
     mma(b_cur, a_hi, H);
+    if constexpr (FOLD && NWN == 4) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+#pragma unroll
+      for (int j = 0; j < 6; ++j) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (j == 2) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    }
     if constexpr (MF == 8) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
 #pragma unroll
@@ -1211,7 +1236,7 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
 //     against 29.5), and so is K above 3072: folding q4_mid_kernel up to 512 tiles, two workgroups per CU (K = 4096, M = 4,000 47.2,
 //     128 x 256 tiles 64.4; M = 5,000, 632 tiles, 66.1 against 64.8);
 //   * the rest folds the chunks in 128 x 256 tiles where their last round of 256 is mostly full (K = 3072,
-//     M = 8,000 55 against 61 with 128 x 128 tiles, M = 16,000 114 against 120), else in 128 x 128 tiles, whose
+//     M = 8,000 54 against 61 with 128 x 128 tiles, M = 16,000 109 against 120), else in 128 x 128 tiles, whose
 //     second workgroup per CU fills the gap (M = 12,000, 1.5 rounds, 92 against 106; K = 1792 57 against 68
 //     with two groups, which at K = 2048, both chunks full, take the same 66).
 template <bool SWIGLU>
