@@ -45,8 +45,8 @@ __device__ inline void rmsnorm_row(const half_t* xr, const half_t* rr, half_t* x
           s[e] = (float)a[e] + (float)b[e];
           a[e] = (half_t)s[e];
         }
-        // The row's first pair adds its squares the other way round: the order (and so the rounding) that
-        // embeddings stored by earlier builds were made with.
+        // The row's first pair adds its squares the other way round: the order (and so the rounding) of
+        // embeddings stored before there was a fused projection.
         if (j == 0) ss = fmaf(s[0], s[0], s[1] * s[1]);
 #pragma unroll
         for (int e = j == 0 ? 2 : 0; e < 8; ++e) ss = fmaf(s[e], s[e], ss);

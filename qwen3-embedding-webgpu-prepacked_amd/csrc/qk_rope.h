@@ -42,8 +42,8 @@ __device__ inline float wave_sum(float v) {
 // A rotated element is fma(n, cos, partner * sin) rounded once to fp16, except elements 1-6 of the first
 // four vectors and 2-7 of the second four: they round to fp32 and then to fp16, and every other one
 // of them is fma(partner, sin, n * cos).  That is how the compiler once laid out the separate launch;
-// it is spelled out so that embeddings stored by earlier builds stay equal bit for bit and no
-// longer depend on the compiler.
+// it is spelled out so that embeddings stored before there was a fused projection stay equal bit for
+// bit and no longer depend on the compiler.
 template <int QUAD>
 __device__ inline rope_h8 rope_rotate(const float (&n)[8], const float (&partner)[8], const float4 (&c4)[4]) {
   rope_h8 r;

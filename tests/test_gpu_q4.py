@@ -135,9 +135,8 @@ def test_q4_matmul_swiglu_equals_the_two_launches(ctx, oracle, m, k, n_inter):
 
 
 def test_q4_rows_do_not_depend_on_the_launch_shape(ctx, oracle):
-    """Three kernels serve one projection, chosen by the launch's size: up to 512 output blocks of
-    32 x 32 the one-wavefront-per-block kernel, then the tiled kernel with 64-row tiles (fewer
-    than 160 tiles of 128 x 128), then 128-row tiles.  Every output element is computed the same
+    """Three kernels serve one projection, chosen by the launch's size: 32-row blocks whose wavefronts
+    share K, then tiles of 64 x 128, then of 256 x 128.  Every output element is computed the same
     way in all three (the same K blocks and MFMA order), so rows 0..63 of a 64-row, a 300-row and
     an 1100-row launch are equal bit for bit -- the model's batch invariance rests on this -- for
     the plain and the fused gate/up projections."""
@@ -145,27 +144,26 @@ def test_q4_rows_do_not_depend_on_the_launch_shape(ctx, oracle):
     k, n = 256, 4096
     packed = random_compact(rng, n, k)
     x = rng.standard_normal((1100, k)).astype(np.float16)
-    big = run_q4(ctx, x, packed, k, n)          # 9 x 32 = 288 tiles: 128-row tiles
-    mid = run_q4(ctx, x[:300], packed, k, n)    # 3 x 32 = 96 tiles: 64-row tiles
-    small = run_q4(ctx, x[:64], packed, k, n)   # 2 x 128 = 256 blocks: one wavefront per block
+    big = run_q4(ctx, x, packed, k, n)          # 576 tiles of 64 x 128: 256 x 128 tiles
+    mid = run_q4(ctx, x[:300], packed, k, n)    # 160 tiles of 64 x 128
+    small = run_q4(ctx, x[:64], packed, k, n)   # 256 blocks of 32 x 32
     check(oracle, big, x, packed, k, n, "q4 1100 rows")
     check(oracle, small, x[:64], packed, k, n, "q4 64 rows")
     assert np.array_equal(big[:64].view(np.uint16), small.view(np.uint16))
     assert np.array_equal(mid[:64].view(np.uint16), small.view(np.uint16))
     big_f = run_q4_swiglu(ctx, x, packed, k, n // 2)
     mid_f = run_q4_swiglu(ctx, x[:300], packed, k, n // 2)
-    small_f = run_q4_swiglu(ctx, x[:64], packed, k, n // 2)  # 2 x 64 = 128 blocks
+    small_f = run_q4_swiglu(ctx, x[:64], packed, k, n // 2)
     assert np.array_equal(big_f[:64].view(np.uint16), small_f.view(np.uint16))
     assert np.array_equal(mid_f[:64].view(np.uint16), small_f.view(np.uint16))
 
 
 def test_q4_chunked_k_rows_do_not_depend_on_the_launch_shape(ctx, oracle):
     """K = 3072 spans three chunks of 1024 columns, summed in chunk order by every kernel: the
-    direct kernel with one wavefront per chunk meeting in LDS (64 rows: 64 output blocks x 3
-    chunks), the direct kernel with one wavefront folding the chunks in turn (300 rows: 320
-    blocks, too many chunk wavefronts), the 64-row tiled kernel (1100 rows) and the 128-row tiled
-    kernel (2600 rows: 168 tiles of 128 x 128), both with a second accumulator set.  Rows 0..63
-    agree bit for bit."""
+    small kernel with the chunks side by side (64 rows: 256 blocks of 16 x 16), the direct kernel
+    with one wavefront folding the chunks in turn (300 rows: 320 blocks of 32 x 32, too many chunk
+    wavefronts), 64 x 128 tiles (1100 rows) and 128 x 128 tiles (2600 rows: 168) with a group of
+    wavefronts per chunk.  Rows 0..63 agree bit for bit."""
     rng = np.random.default_rng(6)
     k, n = 3072, 1024
     packed = random_compact(rng, n, k)
@@ -202,18 +200,18 @@ def test_q4_matmul_invalid_arguments(ctx, qattn):
 TILE_CASES = [
     (50, 1024, 4096, False), (50, 992, 1501, False), (33, 1024, 6144, True),  # 32-row blocks
     (300, 2048, 1024, False), (500, 3072, 1023, False), (150, 1056, 384, True),  # one wavefront per block
-    (150, 3072, 2048, True), (33, 4160, 96, False),  # halves of 72 K blocks
+    (150, 3072, 2048, True), (33, 4160, 96, False),  # five chunks
     (50, 2048, 1000, False), (64, 3072, 1023, False), (40, 4096, 9, False),  # 16 x 16 blocks
     (65, 2048, 1000, False), (33, 4096, 1400, False),  # 16 x 32 blocks
     (65, 96, 6001, False),      # 64 x 128 tiles, one row past a tile, N odd
     (1025, 1024, 4096, False),  # 256 x 128
     (500, 160, 12300, False),   # 256 x 128, K padded to 8 blocks, N = 8 k + 4
-    (4100, 64, 4352, False),    # 256 x 128 for its fuller last round
+    (4100, 64, 4352, False),    # shallow K: 128 x 128 where 256 x 256 leaves its last round empty
     (2100, 1024, 4096, False),  # 256 x 256
     (2570, 32, 4100, False),    # 256 x 256, one K block
-    (1900, 1056, 520, False),   # halves of 24 and 9 K blocks, 64 x 128
-    (2100, 2048, 1024, False),  # halves, 128 x 128
-    (4200, 3072, 1000, False),  # halves, 256 x 128
+    (1900, 1056, 520, False),    # a chunk of 32 K blocks and one of a single block, folded, 64 x 128
+    (2100, 2048, 1024, False),  # two chunks, 128 x 128
+    (4200, 3072, 1000, False),  # three chunks, folded, 128 x 256
     (200, 1024, 6144, True), (1030, 1024, 6144, True), (1300, 1024, 6144, True),  # n: gate + up rows
     (2100, 96, 6144, True), (23000, 32, 384, True), (5000, 1120, 384, True), (700, 2048, 6144, True),
 ]

@@ -1,6 +1,6 @@
 """The roundings of the residual add + RMSNorm (qattn_rmsnorm) and of the QK norm + RoPE
-(qattn_qk_norm_rope*), bit for bit against a host restatement of their arithmetic: embeddings stored by
-earlier builds stay equal, and a row does not depend on the kernel that computed it."""
+(qattn_qk_norm_rope*), bit for bit against a host restatement of their arithmetic: embeddings stored
+before there were fused projections stay equal, and a row does not depend on the kernel that computed it."""
 import numpy as np
 import pytest
 
