@@ -398,8 +398,9 @@ __global__ __launch_bounds__(128 * NWN * G, 2) void q4_tile_kernel(
   // 16 nb + 4 kq .. +3.
   constexpr int kMine = G > 1 ? H : MF;               // row fragments this wavefront finishes
   constexpr int kWriters = kWaves * (G > 1 ? 2 : 1);
-  // rows per pass: at most 64, and as many as the X buffers hold for every writer
-  constexpr int kRows = 16 * kMine < 64 ? 16 * kMine : G * kBytesA / 32 / kWriters < 64 ? G * kBytesA / 32 / kWriters : 64;
+  constexpr int kHold = 4 * G * kBytesA / 128 / kWriters;  // rows the X buffers hold for every writer
+  constexpr int kMost = kHold < 64 ? kHold : 64;
+  constexpr int kRows = 16 * kMine < kMost ? 16 * kMine : kMost;  // rows per pass
   constexpr int kPer = G * kBytesA / (128 * kRows);    // wavefronts per X buffer
   static_assert(4 * kPer >= kWriters && 16 * kMine % kRows == 0 && kRows % 16 == 0, "a stage per writer, whole fragments");
   const int slot = gwave / kPer;
@@ -1224,8 +1225,8 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
 //   * q4_direct_kernel up to kQ4DirectBlocks (K = 3072, M = 500 16.5, mid 17.5);
 //   * up to 256 tiles of 64 x 128: q4_mid_kernel, a group per chunk (K = 2048, M = 1,419 13.2, 128 x 128
 //     tiles 19.8; K = 3072 18.4);
-//   * up to 128 rows and beyond 256 tiles of 128 x 128, folding q4_mid_kernel (N = 40,000, M = 100: K = 2048 33.2, 128 x 128
-//     tiles 38.9; K = 3072 47.6 against 50.6);
+//   * up to 128 rows and beyond 256 tiles of 128 x 128, folding q4_mid_kernel (N = 40,000, M = 100:
+//     K = 2048 33.2, 128 x 128 tiles 38.9; K = 3072 47.6 against 50.6);
 //   * K up to 2048: 128 x 128 tiles while at most one per CU (M = 2,400 20.3, mid 25.4, 256 x 128 27.6),
 //     then 256 x 128 or 128 x 128 tiles by the rounds each needs (M = 8,000: one round of 38.8 against two
 //     of 22.7);
@@ -1233,8 +1234,8 @@ void launch_q4_direct(const _Float16* x, int64_t ldx, int M, int K, const uint8_
 //     128 x 256 folding 49.5); beyond, three groups of larger tiles do not fit in LDS;
 //   * groups run as long as a whole chunk, so where the last chunk is at most half full the chunks are folded
 //     instead (K = 1536: M = 1,419 12.5 against 13.6, M = 8,000 33.7 against 36.9; K = 1792, M = 5,000 30.2
-//     against 29.5), and so is K above 3072: folding q4_mid_kernel up to 512 tiles, two workgroups per CU (K = 4096, M = 4,000 47.2,
-//     128 x 256 tiles 64.4; M = 5,000, 632 tiles, 66.1 against 64.8);
+//     against 29.5), and so is K above 3072: folding q4_mid_kernel up to 512 tiles, two workgroups per CU
+//     (K = 4096, M = 4,000 47.2, 128 x 256 tiles 64.4; M = 5,000, 632 tiles, 66.1 against 64.8);
 //   * the rest folds the chunks in 128 x 256 tiles where their last round of 256 is mostly full (K = 3072,
 //     M = 8,000 54 against 61 with 128 x 128 tiles, M = 16,000 109 against 120), else in 128 x 128 tiles, whose
 //     second workgroup per CU fills the gap (M = 12,000, 1.5 rounds, 92 against 106; K = 1792 57 against 68
